@@ -77,7 +77,8 @@ struct m1lya_ctx {
     bool grid_set = false;
 
     // reductions and scratch
-    int col_blocks = 0, act_blocks = 0, pstride = 0, prows = 0;
+    ColumnShape col{};
+    int act_blocks = 0, pstride = 0, prows = 0;
     double *part = nullptr, *red = nullptr, *scalars = nullptr;
     int *krange = nullptr, *err_flag = nullptr;
     StepCtl* ctl = nullptr;                // halt flag and executed-step count (m1lya_run_until_steady)
@@ -383,10 +384,10 @@ void fused_step(m1lya_ctx* c, double c_tilde, double dt, double z_center, int bc
     a.c_tilde = c_tilde; a.dt = dt; a.dw = 1.0 / cdt; a.z_center = z_center; a.bc_z_bot = bc_z_bot;
     a.halt = halt;
     Prof p(c, "column", true);
-    launch_column(c->stream, a, c->col_blocks);
+    launch_column(c->stream, a, c->col);
     p.done();
     Prof p2(c, "reduce_cols");
-    launch_reduce_cols(c->stream, c->part, c->col_blocks, c->pstride, 2 * c->nn + kStepSums, c->red, halt);
+    launch_reduce_cols(c->stream, c->part, c->col.blocks, c->pstride, 2 * c->nn + kStepSums, c->red, halt);
     p2.done();
     Prof p3(c, "step_final");
     launch_step_final(c->stream, c->red, c->nn, c->kcore_min, c->kcore_max, bc_z_bot, c->krange, c->scalars,
@@ -439,7 +440,7 @@ void replay_step(m1lya_ctx* c, double c_tilde, double dt, double z_center, int b
     ColumnArgs a = column_args(c, COL_EMIT | COL_FREQ | COL_SOLVE | COL_HCORR | COL_FUSED);
     a.c_tilde = c_tilde; a.dt = dt; a.dw = 1.0 / cdt; a.z_center = z_center; a.bc_z_bot = bc_z_bot;
     Prof p(c, "column");
-    launch_column(c->stream, a, c->col_blocks);
+    launch_column(c->stream, a, c->col);
     p.done();
     c->old_stale = true;
     c->fij_stale = true;
@@ -513,12 +514,10 @@ int m1lya_create(int n_nu, int n_r, int n_z, int precision, m1lya_ctx** out)
         c->ivr = dalloc(c, (size_t)(n_r + 1) * 5); c->ivz = dalloc(c, (size_t)(n_z + 1) * 5);
         c->nu = dalloc(c, n_nu + 1); c->nuC = dalloc(c, n_nu); c->dnu = dalloc(c, n_nu);
         c->inv_dnu = dalloc(c, n_nu); c->inv_nuC = dalloc(c, n_nu);
-        const int W = column_width(n_nu) * column_waves(n_nu);   // columns per block
-        const int ngroups = (int)((nc + W - 1) / W);
-        c->col_blocks = column_blocks(n_nu, ngroups);
+        c->col = column_shape(n_nu, nc);
         c->act_blocks = (int)std::min<size_t>(nc, 1024);
         c->pstride = 2 * n_nu + 8;
-        c->prows = std::max(c->col_blocks, c->act_blocks);
+        c->prows = std::max(c->col.blocks, c->act_blocks);
         c->part = dalloc(c, (size_t)c->prows * c->pstride);
         c->red = dalloc(c, c->pstride);
         c->scalars = dalloc(c, 8);
@@ -743,7 +742,7 @@ int m1lya_emission_absorption_update(m1lya_ctx* c, double c_tilde, double dt)
         ColumnArgs a = column_args(c, COL_EMIT);
         a.c_tilde = c_tilde; a.dt = dt;
         Prof p(c, "column_emit");
-        launch_column(c->stream, a, c->col_blocks);
+        launch_column(c->stream, a, c->col);
         p.done();
         c->krange_valid = false;
         hipchk(c, hipStreamSynchronize(c->stream), "sync");
@@ -759,7 +758,7 @@ int m1lya_update_freq_factors(m1lya_ctx* c, const double* T, const double* dur_d
         upload_velocity(c, dur_dr, dur_dz, duz_dr, duz_dz, ur_over_r);
         ColumnArgs a = column_args(c, COL_FREQ | COL_STORE_F);
         Prof p(c, "column_freq_factors");
-        launch_column(c->stream, a, c->col_blocks);
+        launch_column(c->stream, a, c->col);
         p.done();
         c->fij_stale = false;
         hipchk(c, hipStreamSynchronize(c->stream), "sync");
@@ -781,7 +780,7 @@ int m1lya_frequency_update_all_cells(m1lya_ctx* c, double c_dt, const double* T,
         ColumnArgs a = column_args(c, flags);
         a.dw = 1.0 / c_dt;
         Prof p(c, "column_freq_update");
-        launch_column(c->stream, a, c->col_blocks);
+        launch_column(c->stream, a, c->col);
         p.done();
         if (update_freq_factors) c->fij_stale = false;
         c->krange_valid = false;

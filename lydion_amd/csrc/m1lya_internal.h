@@ -7,7 +7,7 @@
 
 namespace m1 {
 
-// Cell columns per wavefront in the column kernel (lane-per-column dgtsv).
+// Most cell columns per wavefront in the column kernel (lane-per-column dgtsv).
 constexpr int kColumnW = 4;
 // Largest N_ν of the FP64 context (nine bins per lane, one column per wavefront).
 constexpr int kMaxBinsFP64 = 576;
@@ -237,17 +237,23 @@ void launch_reduce_cols(hipStream_t s, const double* part, int nrows, int stride
                         const int* halt = nullptr);
 void launch_active_final(hipStream_t s, const double* red, int nn, int kcmin, int kcmax, int* krange);
 void launch_advect(hipStream_t s, const AdvectArgs& a);
-// Cell columns per wavefront of the column kernel for an N_ν-bin grid.
-int column_width(int nn);
-// Wavefronts per block of the column kernel for an N_ν-bin grid (the block shares its dgtsv phase).
-int column_waves(int nn);
-// Blocks of the column kernel for ngroups column groups: a fixed count (at most ngroups),
-// so that the partition of the fused reductions, and with it their bits, does not depend
-// on the device.  kColumnBlocks / column_waves(N_ν) blocks are one launch wave on MI355X
-// (8 wavefronts per CU, 256 CUs).
+// Shape of the column kernel's launch: w cell columns per wavefront, nw wavefronts per block
+// (the block shares its dgtsv phase), blocks of the grid.  It depends on the grid's dimensions
+// alone, so that the partition of the fused reductions, and with it their bits, does not depend
+// on the device.
+//
+// Four wavefronts per block fill 64 KB of LDS with the rows of w·nw columns (16 up to 128 bins, 8
+// up to 256); wider grids keep one wavefront and one column of up to 18 KB.  The grid is exactly
+// one wave of resident blocks (kColumnBlocks / nw on MI355X: 8 wavefronts per CU, 256 CUs), so
+// that every block loops over the same number of column groups and they all start together: a
+// larger one left a partial second wave starting late.  While fewer cells than one such wave
+// holds are there, w is halved, so that the columns spread over more blocks.
 constexpr int kColumnBlocks = 2048;
-int column_blocks(int nn, int ngroups);
-void launch_column(hipStream_t s, const ColumnArgs& a, int nblocks);
+struct ColumnShape {
+    int w, nw, blocks;
+};
+ColumnShape column_shape(int nn, size_t ncells);
+void launch_column(hipStream_t s, const ColumnArgs& a, const ColumnShape& c);
 // Step scalars {M_F, net, out, L, f_esc, kmin, kmax, ΔJ/J}; ΔJ/J is 0 unless the column
 // kernel ran with COL_CONV.  ctl may be null (no halt, no count); tol > 0 sets ctl->halt
 // once ΔJ/J < tol.  A non-finite count sets ERR_NONFINITE in err_flag.

@@ -348,35 +348,48 @@ __global__ __launch_bounds__(64 * WPB) void k_advect(AdvectArgs a, int seg_len)
     }
 }
 
+// Sum over the 64 lanes, in every lane, by register moves: scans within rows of 16 lanes (DPP
+// row_shr), then the four row totals.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double prev_lane(double v) { return dpp_f64<0x138>(v); }   // 0 in lane 0
+__device__ __forceinline__ double next_lane(double v) { return dpp_f64<0x130>(v); }   // 0 in lane 63
+__device__ __forceinline__ double lane_value(double v, int l)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+__device__ __forceinline__ double wave_sum_dpp(double v)
+{
+    v += dpp_f64<0x111>(v);
+    v += dpp_f64<0x112>(v);
+    v += dpp_f64<0x114>(v);
+    v += dpp_f64<0x118>(v);
+    return (lane_value(v, 15) + lane_value(v, 31)) + (lane_value(v, 47) + lane_value(v, 63));
+}
+
 // ------------------------------------------------------------------------
 // LAPACK dgtsv (NRHS = 1, published reference algorithm: elimination with
 // partial pivoting by row interchange) on one LDS-resident column, as called by
 // TridiagonalSolve (src/TridiagonalSolver.jl:54).  Row i of each array is at
-// [i]; the solution overwrites b.  The current and next rows are carried in
-// registers, so the dependent chain is arithmetic only; every value stored
-// is the one LAPACK would store, computed by the same operations.
+// [i]; the solution overwrites b.  Every value stored is the one LAPACK would
+// store, computed by the same operations.
+//
+// gtsv_general: entries of any magnitude.
 // ------------------------------------------------------------------------
-__device__ int gtsv_col(int n, double* __restrict__ dl, double* __restrict__ d, double* __restrict__ du,
-                        double* __restrict__ b)
+__device__ __forceinline__ int gtsv_general(int n, double* dl, double* d, double* du, double* b)
 {
-    double d_i = d[0], b_i = b[0];
-    double du_i = (n > 1) ? du[0] : 0.0;
-    // The inputs of row i+1 are read one row ahead of their use, so the LDS latency
-    // overlaps the previous row's division instead of lengthening the chain.  No row
-    // step writes what a later read takes (it writes dl, d, du, b at row i only).
-    double dl_c = 0.0, d_c = 0.0, b_c = 0.0, du_c = 0.0;
-    if (n > 1) { dl_c = dl[0]; d_c = d[1]; b_c = b[1]; du_c = du[min(1, n - 2)]; }
+    double d_i = d[0], b_i = b[0], du_i = (n > 1) ? du[0] : 0.0;
     int info = 0;
+#pragma unroll 1
     for (int i = 0; i < n - 1; ++i) {
         const bool last = (i == n - 2);
-        const double dl_i = dl_c, d_n = d_c, b_n = b_c, du_n = last ? 0.0 : du_c;
-        {
-            // unconditional reads, clamped to the column (what a clamped read returns is
-            // never used), so that nothing waits for them before the next row step
-            const int r1 = min(i + 1, n - 2), r2 = min(i + 2, n - 1), r3 = max(min(i + 2, n - 2), 0);
-            dl_c = dl[r1]; d_c = d[r2]; b_c = b[r2]; du_c = du[r3];
-        }
-        __builtin_amdgcn_sched_barrier(0);   // keep the reads ahead of the row step
+        const double dl_i = dl[i], d_n = d[i + 1], b_n = b[i + 1], du_n = last ? 0.0 : du[i + 1];
         // Both branches of the row step as selects around one division: without an
         // interchange fact = dl_i/d_i, row i stays and row i+1 loses fact·row i; with
         // one (|d_i| < |dl_i|) fact = d_i/dl_i, rows i and i+1 swap places, row i+1
@@ -405,6 +418,7 @@ __device__ int gtsv_col(int n, double* __restrict__ dl, double* __restrict__ d, 
     if (n == 1) return 0;
     double x0 = (b[n - 2] - du[n - 2] * x1) / d[n - 2];
     b[n - 2] = x0;
+#pragma unroll 1
     for (int i = n - 3; i >= 0; --i) {
         double x = (b[i] - du[i] * x0 - dl[i] * x1) / d[i];
         b[i] = x;
@@ -412,6 +426,180 @@ __device__ int gtsv_col(int n, double* __restrict__ dl, double* __restrict__ d, 
         x0 = x;
     }
     return 0;
+}
+
+// The solve is one serial chain per column, and one wavefront's worth of instructions whatever the
+// number of columns it solves: dependent FP64 operations issue back to back on CDNA4 (5 cycles,
+// 16 for the reciprocal estimate), so its time is the count of a row's instructions, forward and
+// back.  For tame systems (every sub-diagonal entry at least kTameMin and no entry above kTameMax
+// in magnitude, which row formation tests) a pivot, interchanged or not, is no smaller than the
+// entry below it, so that every division is one of quot's: reciprocal refinement and residual
+// correction, the same quotient.  The pivots' reciprocals stay in rp for the back substitution,
+// where a row is then four operations for its numerator and three for the quotient instead of a
+// whole division.  About 20 % of the physical rows interchange, so both branches are selects.
+// Rows go in chunks of kRows, loaded a chunk ahead into the other of two register sets.  The loads
+// ahead run up to 2 kRows rows past either end of the column (their values are not used): kColPad
+// doubles of the block's LDS lie before the first array and after the last.
+constexpr int kColPad = 8;
+constexpr double kTameMax = 0x1p500, kTameMin = 0x1p-500;
+
+__device__ __forceinline__ int gtsv_tame(int n, double* __restrict__ dl, double* __restrict__ d,
+                                         double* __restrict__ du, double* __restrict__ b, double* __restrict__ rp)
+{
+    constexpr int kRows = 2;
+    struct Rows {
+        double l[kRows], d[kRows], u[kRows], b[kRows], r[kRows];
+    };
+    double d_i = d[0], b_i = b[0], du_i = du[0];
+    // row step i from the carried row (d_i, du_i, b_i); reads of rows past the column feed nothing
+    auto row = [&](int i, double l, double dn, double un, double bn) {
+        const bool swap = !(fabs(d_i) >= fabs(l));
+        const double piv = swap ? l : d_i, r = rcp_nr(piv);
+        const double fact = quot(swap ? d_i : l, piv, r);
+        const double u = swap ? dn : du_i, v = swap ? bn : b_i;
+        d[i] = piv; du[i] = u; b[i] = v; rp[i] = r;
+        dl[i] = swap ? un : 0.0;
+        d_i = (swap ? du_i : dn) - fact * u;
+        b_i = (swap ? b_i : bn) - fact * v;
+        du_i = swap ? -fact * un : un;
+    };
+    auto fetch = [&](Rows& x, int at) {
+#pragma unroll
+        for (int t = 0; t < kRows; ++t) {
+            x.l[t] = dl[at + t]; x.d[t] = d[at + t + 1]; x.u[t] = du[at + t + 1]; x.b[t] = b[at + t + 1];
+        }
+    };
+    auto chunk = [&](const Rows& x, int at) {
+#pragma unroll
+        for (int t = 0; t < kRows; ++t) row(at + t, x.l[t], x.d[t], x.u[t], x.b[t]);
+    };
+    Rows x0, x1;
+    int i = 0;
+    fetch(x0, 0);
+#pragma unroll 1
+    for (; i + 2 * kRows <= n - 1; i += 2 * kRows) {
+        fetch(x1, i + kRows);
+        __builtin_amdgcn_sched_barrier(0);   // keep the reads ahead of the row steps
+        chunk(x0, i);
+        fetch(x0, i + 2 * kRows);
+        __builtin_amdgcn_sched_barrier(0);
+        chunk(x1, i + kRows);
+    }
+#pragma unroll 1
+    for (; i < n - 1; ++i) row(i, dl[i], d[i + 1], du[i + 1], b[i + 1]);
+    if (d_i == 0.0) return n;
+    // back substitution: rows n-1 and n-2, then the rows with a second super-diagonal
+    double p1 = b_i / d_i;
+    b[n - 1] = p1;
+    if (n == 1) return 0;
+    double p0 = quot(b[n - 2] - du[n - 2] * p1, d[n - 2], rp[n - 2]);
+    b[n - 2] = p0;
+    auto back = [&](int at, double bb, double u, double l, double dd, double r) {
+        const double x = quot(bb - u * p0 - l * p1, dd, r);
+        b[at] = x;
+        p1 = p0;
+        p0 = x;
+    };
+    auto fetch_back = [&](Rows& x, int top) {
+#pragma unroll
+        for (int t = 0; t < kRows; ++t) {
+            x.b[t] = b[top - t]; x.u[t] = du[top - t]; x.l[t] = dl[top - t]; x.d[t] = d[top - t];
+            x.r[t] = rp[top - t];
+        }
+    };
+    auto chunk_back = [&](const Rows& x, int top) {
+#pragma unroll
+        for (int t = 0; t < kRows; ++t) back(top - t, x.b[t], x.u[t], x.l[t], x.d[t], x.r[t]);
+    };
+    int top = n - 3;
+    if (top >= 2 * kRows - 1) fetch_back(x0, top);
+#pragma unroll 1
+    for (; top >= 2 * kRows - 1; top -= 2 * kRows) {
+        fetch_back(x1, top - kRows);
+        __builtin_amdgcn_sched_barrier(0);
+        chunk_back(x0, top);
+        fetch_back(x0, top - 2 * kRows);
+        __builtin_amdgcn_sched_barrier(0);
+        chunk_back(x1, top - kRows);
+    }
+#pragma unroll 1
+    for (; top >= 0; --top) back(top, b[top], du[top], dl[top], d[top], rp[top]);
+    return 0;
+}
+
+// One row of UpdateFreqFactors! (src/FreqFactors.jl:142-278) with divisions of any range: the
+// general form, for rows whose factors come out infinite or NaN in the kernel's own form (a
+// vanishing diffusion coefficient).
+__device__ __forceinline__ void freq_row_general(const ColumnArgs& a, size_t idx, int k, double VEL, double PREFACT, double RECOIL_0,
+                                 double& Fkp, double& Fk, double& Fkm)
+{
+    const double nuCk = a.nuC[k], nuCkp = a.nuC[k + 1], nuCkm = a.nuC[k - 1];
+    const double dkp = nuCkp - a.nu[k + 1], dk = a.nu[k + 1] - nuCk, dkm = a.nu[k] - nuCkm;
+    const double inv_dnu_k = a.inv_dnu[k];
+    const double Kkp = PREFACT * a.Hv[idx + 1], Kk = PREFACT * a.Hv[idx], Kkm = PREFACT * a.Hv[idx - 1];
+    double Ckp = VEL * nuCkp, Ck = VEL * nuCk, Ckm = VEL * nuCkm;
+    if (a.recoil) {
+        Ckp += Kkp * (RECOIL_0 - 2.0 * a.inv_nuC[k + 1]);
+        Ck += Kk * (RECOIL_0 - 2.0 * a.inv_nuC[k]);
+        Ckm += Kkm * (RECOIL_0 - 2.0 * a.inv_nuC[k - 1]);
+    }
+    const double qkp = dkp * (1.0 / Kkp), qk = dk * (1.0 / Kk), qkm = dkm * (1.0 / Kkm);
+    const double Pkp = dclamp(Ckp * qkp, -kPmax, kPmax);
+    const double Pk = dclamp(Ck * qk, -kPmax, kPmax);
+    const double Pkm = dclamp(Ckm * qkm, -kPmax, kPmax);
+    double oRkp, xRkp, oLk, xLk, oRk, xRk, oLkm, xLkm;
+    one_minus_phi_R(Pkp, oRkp, xRkp);
+    one_minus_phi_L(Pk, oLk, xLk);
+    one_minus_phi_R(Pk, oRk, xRk);
+    one_minus_phi_L(Pkm, oLkm, xLkm);
+    const double den_kp = inv_dnu_k * (1.0 / (xLk * qk - xRkp * qkp));
+    Fkp = oRkp * den_kp;
+    const double den_km = inv_dnu_k * (1.0 / (xLkm * qkm - xRk * qk));
+    Fkm = oLkm * den_km;
+    Fk = oLk * den_kp + oRk * den_km;
+}
+
+// OneMinusϕ_L_and_χ_L (sgn = -1) / OneMinusϕ_R_and_χ_R (sgn = +1) of src/FreqFactors.jl:54-133
+// for a clamped P and its reciprocal's estimate r = rcp_nr(P): at |P| = kPmax the clamped
+// branches of the reference are the general one, and |P| < kPmin is a select.
+template <int sgn>
+__device__ __forceinline__ void one_minus_phi(double P, double r, double& o, double& chi)
+{
+    const double e = exp_core(sgn < 0 ? -P : P);
+    const bool small = fabs(P) < kPmin;
+    o = small ? (sgn < 0 ? 1.0 - P : 1.0 + P) + 0.5 * (P * P) : e;
+    chi = small ? (sgn < 0 ? 1.0 : -1.0) - 0.5 * P : quot(1.0 - e, P, r);
+}
+
+// The KPL consecutive bins of a lane, from k0; bins past N_ν are left as they are.
+template <int KPL>
+__device__ __forceinline__ void load_bins(const double* __restrict__ p, int k0, int nn, double (&v)[KPL])
+{
+    using V2 = double __attribute__((ext_vector_type(2), aligned(8)));
+    if (KPL % 2 == 0 && k0 + KPL <= nn) {
+#pragma unroll
+        for (int q = 0; q + 1 < KPL; q += 2) {
+            const V2 x = *reinterpret_cast<const V2*>(p + k0 + q);
+            v[q] = x.x; v[q + 1] = x.y;
+        }
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < KPL; ++q)
+        if (k0 + q < nn) v[q] = p[k0 + q];
+}
+template <int KPL>
+__device__ __forceinline__ void store_bins(double* __restrict__ p, int k0, int nn, const double (&v)[KPL])
+{
+    using V2 = double __attribute__((ext_vector_type(2), aligned(8)));
+    if (KPL % 2 == 0 && k0 + KPL <= nn) {
+#pragma unroll
+        for (int q = 0; q + 1 < KPL; q += 2) *reinterpret_cast<V2*>(p + k0 + q) = V2{v[q], v[q + 1]};
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < KPL; ++q)
+        if (k0 + q < nn) p[k0 + q] = v[q];
 }
 
 // ------------------------------------------------------------------------
@@ -424,8 +612,16 @@ __device__ int gtsv_col(int n, double* __restrict__ dl, double* __restrict__ d, 
 //       one wavefront instruction per row step for as many columns as lanes take part;
 //   P3 (lanes over k): J floor, H rescale and causality, old copies
 //       (src/UpdateLyaJandH.jl:335-379), plus the fused step's reductions.
-// LDS per block: 4 arrays x (N_ν-2) rows x W·NW columns (column index fastest, odd row
-// stride, so the lane-per-column sweep is bank-conflict free).
+// A lane holds KPL consecutive bins, so that a row's neighbours k-1 and k+1 are mostly the
+// lane's own: what a bin contributes to three rows (its diffusion coefficient's reciprocal, its
+// drift, and in cells at rest its exponentials too) is formed once and passed on.
+// What bounds it: instruction issue in P1 and P3 (two wavefronts per SIMD, whose loads are not
+// all covered), and P2's one wavefront per block.  256x256x128 cone cloud: 592 -> 397 us (P1 and
+// P3 alone 410 -> 240 us: shared factors, divisions without range handling, one pass of per-cell
+// terms per column group); 77x90x194: 251 -> 179 us; 32x32x64: 33 -> 18 us (columns spread over
+// four times the blocks).  Loads three or four rows ahead in P2 measured no better than two.
+// LDS per block: 5 arrays x (N_ν-2) rows x W·NW columns (odd row stride, so the
+// lane-per-column sweep is bank-conflict free).
 // ------------------------------------------------------------------------
 // kFused: the instantiation for the fused step's phases (emission, frequency factors, solve,
 // H correction and reductions, kFusedFlags), with the phase tests resolved at compile time;
@@ -433,26 +629,36 @@ __device__ int gtsv_col(int n, double* __restrict__ dl, double* __restrict__ d, 
 constexpr int kFusedFlags = COL_EMIT | COL_FREQ | COL_SOLVE | COL_HCORR | COL_FUSED;
 
 template <int W, int KPL, int NW, bool kFused>
-__global__ __launch_bounds__(64 * NW) void k_column(ColumnArgs a)
+__global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a)
 {
     extern __shared__ double lds[];
     const int nn = a.nn, nr = a.nr, nz = a.nz;
     const int n = nn - 2;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int k0 = lane * KPL;   // the lane's bins are k0 .. k0 + KPL - 1
     constexpr int WB = W * NW;   // columns of the block
     const int flags = kFused ? (kFusedFlags | (a.flags & COL_CONV)) : a.flags;
     const bool EMIT = flags & COL_EMIT, FREQ = flags & COL_FREQ, STOREF = flags & COL_STORE_F;
     const bool SOLVE = flags & COL_SOLVE, HCORR = flags & COL_HCORR, FUSED = flags & COL_FUSED;
     const bool CONV = flags & COL_CONV;
     if (a.halt && *a.halt) return;
-    // [column][row] with an odd row stride: conflict-free for both the lanes-over-k
-    // writes (consecutive rows) and the lane-per-column sweep (stride S, S odd).
     const int S = col_stride(nn);
-    double* sDL = lds;
-    double* sD = lds + (size_t)S * WB;
-    double* sDU = lds + (size_t)2 * S * WB;
-    double* sB = lds + (size_t)3 * S * WB;
+    double* sDL = lds + kColPad;
+    double* sD = sDL + (size_t)S * WB;
+    double* sDU = sD + (size_t)S * WB;
+    double* sB = sDU + (size_t)S * WB;
+    __shared__ int s_wild[WB];     // the column's rows are not tame (gtsv_tame)
+    __shared__ int s_slot;
+    // The two blocks of a CU start together, and in step both would run P1 and P3 at half rate and
+    // then leave the SIMDs idle through both their P2.  The block in the odd wavefront slots
+    // (HW_ID, bits 0-3) gets priority in P1 and P3, so that it draws ahead and each block's P2 lies
+    // over the other's P1 and P3 (cone cloud: 415 us without, 397 us with).
+    if (threadIdx.x == 0) s_slot = __builtin_amdgcn_s_getreg(4 | (0 << 6) | (3 << 11));
+    __syncthreads();
+    const bool ahead = __builtin_amdgcn_readfirstlane(s_slot) & 1;
+    if (ahead) __builtin_amdgcn_s_setprio(1);
+    const int solver = (NW > 1 && ahead) ? NW / 2 : 0;   // of the two blocks' P2, each on a SIMD of its own
     const int ncells = nr * nz;
     const int ngroups = (ncells + WB - 1) / WB;
     const double ct = a.c_tilde, dt = a.dt, dw = a.dw;
@@ -460,15 +666,34 @@ __global__ __launch_bounds__(64 * NW) void k_column(ColumnArgs a)
     const double fpc_ict = (kFourPi / kC) * inv_ct;
     const double inv_dt = 1.0 / dt;
 
+    // the grid's constants of the lane's bins: widths of the two halves, Δν, 1/Δν, 2/νC.  Up to two
+    // bins per lane they stay in registers; beyond, they are loaded again for every column.
+    double hR[KPL], hL[KPL], dnu[KPL], idn[KPL], two[KPL];
+    auto load_grid = [&](bool factors) {
+#pragma unroll
+        for (int q = 0; q < KPL; ++q) {
+            const int k = min(k0 + q, nn - 1);
+            dnu[q] = a.dnu[k];
+            if (!factors) continue;
+            const double nuC = a.nuC[k];
+            hR[q] = a.nu[k + 1] - nuC;
+            hL[q] = nuC - a.nu[k];
+            idn[q] = a.inv_dnu[k];
+            two[q] = 2.0 * a.inv_nuC[k];
+        }
+    };
+    if (KPL <= 2) load_grid(true);
     double e1[KPL], e10[KPL];
 #pragma unroll
     for (int kk = 0; kk < KPL; ++kk) { e1[kk] = 0.0; e10[kk] = 0.0; }
+    // per lane: the step sums of the columns whose terms the lane formed
     double acc_mf = 0.0, acc_L = 0.0, acc_net = 0.0, acc_out = 0.0, acc_esc = 0.0;
     double conv = 0.0;   // per lane: Σ Δν ΔV |J_new - J_start| (COL_CONV)
     int bad = 0;         // per lane: non-finite outputs of the fused step
 
     for (int grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
         double Jo[W][KPL], Hr[W][KPL], Hz[W][KPL];
+        double sum_r = 0.0, sum_z = 0.0;   // lane w: Σ Δν ΔH of column w of the wavefront
         // ================= P1 =================
 #pragma unroll
         for (int w = 0; w < W; ++w) {
@@ -476,155 +701,222 @@ __global__ __launch_bounds__(64 * NW) void k_column(ColumnArgs a)
             const int c = grp * WB + lc;
             if (c >= ncells) continue;
             const size_t base = (size_t)c * nn;
-            double sr = 0.0, sz = 0.0;
-            double al_pd = 0.0, js_ct = 0.0, ac = 0.0;
-            if (EMIT) {
-                ac = a.alpha_c[c];
-                al_pd = a.alpha[c] * a.pd[c];
-                js_ct = a.js[c] * ct;
-            }
-            double Jcur[KPL];
+            if (KPL > 2) load_grid(true);
+            double Jcur[KPL], hv[KPL];
 #pragma unroll
-            for (int kk = 0; kk < KPL; ++kk) {
-                const int k = lane + 64 * kk;
-                if (k >= nn) continue;
-                const size_t idx = base + k;
-                double jc = a.J[idx];
-                double jo = FUSED ? jc : a.J_old[idx];
-                double hr = a.Hr[idx], hz = a.Hz[idx];
-                if (EMIT) {
-                    // AbsorptionUpdateJorH (src/ConstantsAndFunctions.jl:451-462)
-                    double aJ = ac + al_pd * a.Hv[idx];
-                    double dJdt = js_ct * a.phi[idx];
-                    double jn = (jo + dJdt * dt) / (1.0 + aJ * ct * dt);
-                    double aH = a.aF[idx];
-                    double hrn = (hr + 0.0 * dt) / (1.0 + aH * ct * dt);
-                    double hzn = (hz + 0.0 * dt) / (1.0 + aH * ct * dt);
-                    const double dk = a.dnu[k];
-                    sr += dk * (hr - hrn);
-                    sz += dk * (hz - hzn);
-                    jo = jn; jc = jn; hr = hrn; hz = hzn;
-                }
-                Jo[w][kk] = jo; Hr[w][kk] = hr; Hz[w][kk] = hz; Jcur[kk] = jc;
-            }
+            for (int q = 0; q < KPL; ++q) { Jo[w][q] = 1.0; Hr[w][q] = 0.5; Hz[w][q] = 0.5; hv[q] = 1.0; }   // bins past N_ν
+            load_bins<KPL>((FUSED ? a.J : a.J_old) + base, k0, nn, Jo[w]);
+            load_bins<KPL>(a.Hr + base, k0, nn, Hr[w]);
+            load_bins<KPL>(a.Hz + base, k0, nn, Hz[w]);
+            if (EMIT || FREQ) load_bins<KPL>(a.Hv + base, k0, nn, hv);
             if (EMIT) {
-                sr = wave_sum(sr);
-                sz = wave_sum(sz);
+                const double ac = a.alpha_c[c], al_pd = a.alpha[c] * a.pd[c], js_ct = a.js[c] * ct;
+                double ph[KPL], aF[KPL], sr = 0.0, sz = 0.0;
+#pragma unroll
+                for (int q = 0; q < KPL; ++q) { ph[q] = 0.0; aF[q] = 0.0; }
+                load_bins<KPL>(a.phi + base, k0, nn, ph);
+                load_bins<KPL>(a.aF + base, k0, nn, aF);
+#pragma unroll
+                for (int q = 0; q < KPL; ++q) {
+                    // AbsorptionUpdateJorH (src/ConstantsAndFunctions.jl:451-462); the two
+                    // components of H share their divisor
+                    const double aJ = ac + al_pd * hv[q];
+                    const double dJdt = js_ct * ph[q];
+                    const double jn = quot(Jo[w][q] + dJdt * dt, 1.0 + aJ * ct * dt);
+                    const double den = 1.0 + aF[q] * ct * dt, rden = rcp_nr(den);
+                    const double hr = Hr[w][q], hz = Hz[w][q];
+                    double hrn = quot(hr + 0.0 * dt, den, rden);
+                    double hzn = quot(hz + 0.0 * dt, den, rden);
+                    // numerators whose residual could underflow, and divisors out of range
+                    if (__builtin_expect(!(fabs(hr) > 0x1p-900) || !(fabs(hz) > 0x1p-900) || !(fabs(den) < 0x1p500) ||
+                                             !(fabs(aJ) * ct * dt < 0x1p500), 0)) {
+                        hrn = (hr + 0.0 * dt) / den;
+                        hzn = (hz + 0.0 * dt) / den;
+                        Jcur[q] = (Jo[w][q] + dJdt * dt) / (1.0 + aJ * ct * dt);
+                    } else {
+                        Jcur[q] = jn;
+                    }
+                    if (k0 + q < nn) {
+                        sr += dnu[q] * (hr - hrn);
+                        sz += dnu[q] * (hz - hzn);
+                    }
+                    Jo[w][q] = Jcur[q]; Hr[w][q] = hrn; Hz[w][q] = hzn;
+                }
+                sr = wave_sum_dpp(sr);
+                sz = wave_sum_dpp(sz);
                 if (!FUSED) {
                     if (lane == 0) {
                         a.drhou_r[c] += fpc_ict * sr;
                         a.drhou_z[c] += fpc_ict * sz;
                     }
-                } else {
-                    // Update_f_Lyα_MF_L_Lyα! per-cell terms (src/ConstantsAndFunctions.jl:612-660)
-                    const int i = c % nr, j = c / nr;
-                    double dr_u = a.drhou_r[c] + fpc_ict * sr;
-                    double dz_u = a.drhou_z[c] + fpc_ict * sz;
-                    double fr = dr_u * inv_dt, fz = dz_u * inv_dt;
-                    if (lane == 0) {
-                        a.f_r[c] = fr; a.f_z[c] = fz;
-                        a.drhou_r[c] = 0.0; a.drhou_z[c] = 0.0;
-                    }
-                    const double dV = a.dV[c];
-                    acc_mf += dV * sqrt(fr * fr + fz * fz);
-                    acc_L += kFourPi * dV * a.js[c];
-                    double dr = a.rcom[i], dz = a.zcom[j] - a.z_center;
-                    double dist = sqrt(dr * dr + dz * dz);
-                    double frad = 0.0;
-                    if (dist > 0.0) {
-                        double inv_d = 1.0 / dist;
-                        frad = fr * (dr * inv_d) + fz * (dz * inv_d);
-                    }
-                    acc_net += dV * frad;
-                    acc_out += dV * dmax(frad, 0.0);
+                } else if (lane == w) {
+                    sum_r = sr;
+                    sum_z = sz;
                 }
+            } else if (FREQ) {
+#pragma unroll
+                for (int q = 0; q < KPL; ++q) Jcur[q] = 0.0;
+                load_bins<KPL>(a.J + base, k0, nn, Jcur);
             }
             if (FREQ || SOLVE) {
-                const double dnuD = a.dnuD ? a.dnuD[c] : 0.0;
-                const double PREFACT = FREQ ? 0.5 * dmax(a.alpha[c], a.alpha_floor) * (dnuD * dnuD) : 0.0;
-                const double RECOIL_0 = FREQ ? kHoverKB / a.T[c] : 0.0;
-                const double durdr = FREQ ? a.dur_dr[c] : 0.0, durdz = FREQ ? a.dur_dz[c] : 0.0;
-                const double duzdr = FREQ ? a.duz_dr[c] : 0.0, duzdz = FREQ ? a.duz_dz[c] : 0.0;
-                const double urr = FREQ ? a.ur_over_r[c] : 0.0;
-                // With no velocity gradient D:∇u is +0 whatever D is (D finite; its rr, zz and
-                // ϕϕ entries are >= 0), so the cell's bins skip the closure
-                const bool still = durdr == 0.0 && durdz == 0.0 && duzdr == 0.0 && duzdz == 0.0 && urr == 0.0;
+                double Fkp[KPL], Fk[KPL], Fkm[KPL];
+                if (FREQ) {
+                    const double dnuD = a.dnuD ? a.dnuD[c] : 0.0;
+                    const double PREFACT = 0.5 * dmax(a.alpha[c], a.alpha_floor) * (dnuD * dnuD);
+                    const double RECOIL_0 = kHoverKB / a.T[c];
+                    const double durdr = a.dur_dr[c], durdz = a.dur_dz[c];
+                    const double duzdr = a.duz_dr[c], duzdz = a.duz_dz[c], urr = a.ur_over_r[c];
+                    // With no velocity gradient D:∇u is +0 whatever D is (D finite; its rr, zz and
+                    // ϕϕ entries are >= 0): the cell's bins skip the closure, and a bin's exponents
+                    // are the same in the three rows it enters
+                    const bool still = durdr == 0.0 && durdz == 0.0 && duzdr == 0.0 && duzdz == 0.0 && urr == 0.0;
+                    double VEL[KPL];
+                    // per bin: the recoil drift, the half-widths over K
+                    double S0[KPL], qR[KPL], qL[KPL];
 #pragma unroll
-                for (int kk = 0; kk < KPL; ++kk) {
-                    const int k = lane + 64 * kk;
-                    if (k < 1 || k > nn - 2) continue;
-                    const size_t idx = base + k;
-                    double Fkp, Fk, Fkm;
-                    if (FREQ) {
-                        const double* nu = a.nu;
-                        const double* nuC = a.nuC;
-                        double nuCk = nuC[k], nuCkp = nuC[k + 1], nuCkm = nuC[k - 1];
-                        double dkp = nuCkp - nu[k + 1];
-                        double dk = nu[k + 1] - nuCk;
-                        double dkm = nu[k] - nuCkm;
-                        double inv_dnu_k = a.inv_dnu[k];
-                        double two_k = 2.0 * a.inv_nuC[k];
-                        double two_kp = 2.0 * a.inv_nuC[k + 1];
-                        double two_km = 2.0 * a.inv_nuC[k - 1];
-                        double VEL = 0.0;
-                        if (!still) {
-                            Edd D = D_edd(Hr[w][kk], Hz[w][kk], Jcur[kk]);
-                            double Ddu = D_colon_grad_u(D, durdr, durdz, duzdr, duzdz, urr);
-                            VEL = Ddu * kInvC;
+                    for (int q = 0; q < KPL; ++q) {
+                        const double K = PREFACT * hv[q];
+                        const double iK = recip(K);
+                        S0[q] = a.recoil ? K * (RECOIL_0 - two[q]) : -0.0;
+                        qR[q] = hR[q] * iK;
+                        qL[q] = hL[q] * iK;
+                        VEL[q] = 0.0;
+                    }
+                    if (still) {
+                        // rows share what their bins form: A = χL(P) q, exp(-P), χR(P) q, exp(P) over
+                        // the right half, χR(P') q' and exp(P') over the left half
+                        double A[KPL], oL[KPL], B[KPL], oR[KPL], Bl[KPL], oRl[KPL];
+#pragma unroll
+                        for (int q = 0; q < KPL; ++q) {
+                            const double C = 0.0 + S0[q];
+                            const double P = dclamp(C * qR[q], -kPmax, kPmax);
+                            const double Pl = dclamp(C * qL[q], -kPmax, kPmax);
+                            const double rP = rcp_nr(P);
+                            double x;
+                            one_minus_phi<-1>(P, rP, oL[q], x);
+                            A[q] = x * qR[q];
+                            one_minus_phi<1>(P, rP, oR[q], x);
+                            B[q] = x * qR[q];
+                            one_minus_phi<1>(Pl, rcp_nr(Pl), oRl[q], x);
+                            Bl[q] = x * qL[q];
                         }
-                        double Kkp = PREFACT * a.Hv[idx + 1], Kk = PREFACT * a.Hv[idx];
-                        double Kkm = PREFACT * a.Hv[idx - 1];
-                        double Ckp = VEL * nuCkp, Ck = VEL * nuCk, Ckm = VEL * nuCkm;
-                        if (a.recoil) {
-                            Ckp += Kkp * (RECOIL_0 - two_kp);
-                            Ck += Kk * (RECOIL_0 - two_k);
-                            Ckm += Kkm * (RECOIL_0 - two_km);
+                        const double A_p = prev_lane(A[KPL - 1]), oL_p = prev_lane(oL[KPL - 1]);
+                        const double Bl_n = next_lane(Bl[0]), oRl_n = next_lane(oRl[0]);
+#pragma unroll
+                        for (int q = 0; q < KPL; ++q) {
+                            const double Am = q > 0 ? A[q > 0 ? q - 1 : 0] : A_p, oLm = q > 0 ? oL[q > 0 ? q - 1 : 0] : oL_p;
+                            const double Bp = q + 1 < KPL ? Bl[q + 1 < KPL ? q + 1 : 0] : Bl_n;
+                            const double oRp = q + 1 < KPL ? oRl[q + 1 < KPL ? q + 1 : 0] : oRl_n;
+                            const double den_kp = idn[q] * recip(A[q] - Bp);
+                            const double den_km = idn[q] * recip(Am - B[q]);
+                            Fkp[q] = oRp * den_kp;
+                            Fkm[q] = oLm * den_km;
+                            Fk[q] = oL[q] * den_kp + oR[q] * den_km;
                         }
-                        double qkp = dkp * (1.0 / Kkp), qk = dk * (1.0 / Kk), qkm = dkm * (1.0 / Kkm);
-                        double Pkp = dclamp(Ckp * qkp, -kPmax, kPmax);
-                        double Pk = dclamp(Ck * qk, -kPmax, kPmax);
-                        double Pkm = dclamp(Ckm * qkm, -kPmax, kPmax);
-                        double oRkp, xRkp, oLk, xLk, oRk, xRk, oLkm, xLkm;
-                        one_minus_phi_R(Pkp, oRkp, xRkp);
-                        one_minus_phi_L(Pk, oLk, xLk);
-                        one_minus_phi_R(Pk, oRk, xRk);
-                        one_minus_phi_L(Pkm, oLkm, xLkm);
-                        double den_kp = inv_dnu_k * (1.0 / (xLk * qk - xRkp * qkp));
-                        Fkp = oRkp * den_kp;
-                        double den_km = inv_dnu_k * (1.0 / (xLkm * qkm - xRk * qk));
-                        Fkm = oLkm * den_km;
-                        Fk = oLk * den_kp + oRk * den_km;
-                        if (STOREF) { a.Fkp[idx] = Fkp; a.Fk[idx] = Fk; a.Fkm[idx] = Fkm; }
                     } else {
-                        Fkp = a.Fkp[idx]; Fk = a.Fk[idx]; Fkm = a.Fkm[idx];
+                        // every row with its own bin's VEL in the exponents of its three bins
+                        const double S_p = prev_lane(S0[KPL - 1]), qR_p = prev_lane(qR[KPL - 1]);
+                        const double S_n = next_lane(S0[0]), qL_n = next_lane(qL[0]);
+#pragma unroll
+                        for (int q = 0; q < KPL; ++q) {
+                            const int k = min(max(k0 + q, 1), nn - 2);
+                            const Edd D = D_edd(Hr[w][q], Hz[w][q], Jcur[q]);
+                            VEL[q] = D_colon_grad_u(D, durdr, durdz, duzdr, duzdz, urr) * kInvC;
+                            const double Sm = q > 0 ? S0[q > 0 ? q - 1 : 0] : S_p, qm = q > 0 ? qR[q > 0 ? q - 1 : 0] : qR_p;
+                            const double Sp = q + 1 < KPL ? S0[q + 1 < KPL ? q + 1 : 0] : S_n;
+                            const double qp = q + 1 < KPL ? qL[q + 1 < KPL ? q + 1 : 0] : qL_n;
+                            const double Pkp = dclamp((VEL[q] * a.nuC[k + 1] + Sp) * qp, -kPmax, kPmax);
+                            const double Pk = dclamp((VEL[q] * a.nuC[k] + S0[q]) * qR[q], -kPmax, kPmax);
+                            const double Pkm = dclamp((VEL[q] * a.nuC[k - 1] + Sm) * qm, -kPmax, kPmax);
+                            double oRkp, xRkp, oLk, xLk, oRk, xRk, oLkm, xLkm;
+                            const double rPk = rcp_nr(Pk);
+                            one_minus_phi<1>(Pkp, rcp_nr(Pkp), oRkp, xRkp);
+                            one_minus_phi<-1>(Pk, rPk, oLk, xLk);
+                            one_minus_phi<1>(Pk, rPk, oRk, xRk);
+                            one_minus_phi<-1>(Pkm, rcp_nr(Pkm), oLkm, xLkm);
+                            const double den_kp = idn[q] * recip(xLk * qR[q] - xRkp * qp);
+                            const double den_km = idn[q] * recip(xLkm * qm - xRk * qR[q]);
+                            Fkp[q] = oRkp * den_kp;
+                            Fkm[q] = oLkm * den_km;
+                            Fk[q] = oLk * den_kp + oRk * den_km;
+                        }
                     }
-                    if (SOLVE) {
-                        // rows of FrequencyUpdateJLyα! (src/UpdateLyaJandH.jl:200-215) in gtsv form:
-                        // dl <- A[2:end], du <- C[1:end-1] (src/TridiagonalSolver.jl:45-46)
-                        const int row = k - 1;
-                        sD[(size_t)lc * S + row] = -(Fk + dw);
-                        sB[(size_t)lc * S + row] = -dw * Jo[w][kk];
-                        if (row >= 1) sDL[(size_t)lc * S + row - 1] = Fkm;
-                        if (row <= n - 2) sDU[(size_t)lc * S + row] = Fkp;
+#pragma unroll
+                    for (int q = 0; q < KPL; ++q) {
+                        const int k = k0 + q;
+                        // infinite or NaN factors: the row again in the general form
+                        if (__builtin_expect(k >= 1 && k <= nn - 2 && !(fabs(Fkp[q]) + fabs(Fk[q]) + fabs(Fkm[q]) < 0x1p500), 0))
+                            freq_row_general(a, base + k, k, VEL[q], PREFACT, RECOIL_0, Fkp[q], Fk[q], Fkm[q]);
+                        if (STOREF && k >= 1 && k <= nn - 2) {
+                            a.Fkp[base + k] = Fkp[q]; a.Fk[base + k] = Fk[q]; a.Fkm[base + k] = Fkm[q];
+                        }
                     }
+                } else {
+                    load_bins<KPL>(a.Fkp + base, k0, nn, Fkp);
+                    load_bins<KPL>(a.Fk + base, k0, nn, Fk);
+                    load_bins<KPL>(a.Fkm + base, k0, nn, Fkm);
                 }
+                if (SOLVE) {
+                    // rows of FrequencyUpdateJLyα! (src/UpdateLyaJandH.jl:200-215) in gtsv form:
+                    // dl <- A[2:end], du <- C[1:end-1] (src/TridiagonalSolver.jl:45-46)
+                    bool wild = !(dw >= kTameMin);
+#pragma unroll
+                    for (int q = 0; q < KPL; ++q) {
+                        const int k = k0 + q, row = k - 1;
+                        if (k < 1 || k > nn - 2) continue;
+                        sD[(size_t)lc * S + row] = -(Fk[q] + dw);
+                        sB[(size_t)lc * S + row] = -dw * Jo[w][q];
+                        if (row >= 1) sDL[(size_t)lc * S + row - 1] = Fkm[q];
+                        if (row <= n - 2) sDU[(size_t)lc * S + row] = Fkp[q];
+                        wild |= (row >= 1 && !(fabs(Fkm[q]) >= kTameMin)) ||
+                                !(fabs(Fkp[q]) + fabs(Fk[q] + dw) + fabs(Fkm[q]) < kTameMax);
+                    }
+                    const bool any_wild = __any(wild);
+                    if (lane == 0) s_wild[lc] = any_wild;
+                }
+            }
+        }
+        if (FUSED && EMIT && lane < W) {
+            // Update_f_Lyα_MF_L_Lyα! per-cell terms (src/ConstantsAndFunctions.jl:612-660), a column per lane
+            const int c = grp * WB + wave * W + lane;
+            if (c < ncells) {
+                const int i = c % nr, j = c / nr;
+                const double dr_u = a.drhou_r[c] + fpc_ict * sum_r;
+                const double dz_u = a.drhou_z[c] + fpc_ict * sum_z;
+                const double fr = dr_u * inv_dt, fz = dz_u * inv_dt;
+                a.f_r[c] = fr; a.f_z[c] = fz;
+                a.drhou_r[c] = 0.0; a.drhou_z[c] = 0.0;
+                const double dV = a.dV[c];
+                acc_mf += dV * sqrt(fr * fr + fz * fz);
+                acc_L += kFourPi * dV * a.js[c];
+                const double dr = a.rcom[i], dz = a.zcom[j] - a.z_center;
+                const double dist = sqrt(dr * dr + dz * dz);
+                double frad = 0.0;
+                if (dist > 0.0) {
+                    const double inv_d = 1.0 / dist;
+                    frad = fr * (dr * inv_d) + fz * (dz * inv_d);
+                }
+                acc_net += dV * frad;
+                acc_out += dV * dmax(frad, 0.0);
             }
         }
         // ================= P2 =================
         if (SOLVE) {
             __syncthreads();
             const int c = grp * WB + lane;
-            if (wave == 0) {
-                // The solve is one dependent chain per column; the other block on the CU keeps
-                // its SIMD busy meanwhile.  At raised priority the chain's instructions issue as
-                // soon as they are ready, and the other wavefronts fill the cycles in between.
+            if (wave == solver) {
+                // At raised priority the chain's instructions issue as soon as they are ready, and the
+                // other wavefronts of the SIMD fill the cycles in between.
                 __builtin_amdgcn_s_setprio(3);
                 if (lane < WB && c < ncells && n > 0) {
-                    int info = gtsv_col(n, sDL + (size_t)lane * S, sD + (size_t)lane * S, sDU + (size_t)lane * S,
-                                        sB + (size_t)lane * S);
+                    double* p = sDL + (size_t)lane * S;
+                    const size_t st = (size_t)S * WB;
+                    const int info = __any(s_wild[lane]) ? gtsv_general(n, p, p + st, p + 2 * st, p + 3 * st)
+                                                         : gtsv_tame(n, p, p + st, p + 2 * st, p + 3 * st, p + 4 * st);
                     if (info != 0) atomicMax(a.err_flag, 1);
                 }
-                __builtin_amdgcn_s_setprio(0);
+                if (ahead) __builtin_amdgcn_s_setprio(1);
+                else __builtin_amdgcn_s_setprio(0);
             }
             __syncthreads();
         }
@@ -638,49 +930,57 @@ __global__ __launch_bounds__(64 * NW) void k_column(ColumnArgs a)
             const size_t base = (size_t)c * nn;
             const int i = c % nr, j = c / nr;
             const double dV = a.dV ? a.dV[c] : 0.0;
-            double esc = 0.0;
+            double jn[KPL], Js[KPL], esc = 0.0;
+            if (KPL > 2) load_grid(false);
+            const bool edge = FUSED && (i == nr - 1 || j == nz - 1 || (j == 0 && a.bc_z_bot == BC_OUTFLOW));
+            if (SOLVE && !FUSED) load_bins<KPL>(a.J + base, k0, nn, jn);
+            if (FUSED && CONV) load_bins<KPL>(a.J_old + base, k0, nn, Js);
 #pragma unroll
-            for (int kk = 0; kk < KPL; ++kk) {
-                const int k = lane + 64 * kk;
-                if (k >= nn) continue;
-                const size_t idx = base + k;
-                double jn = Jo[w][kk];
-                double hr = Hr[w][kk], hz = Hz[w][kk];
-                if (SOLVE) {
-                    if (k >= 1 && k <= nn - 2) jn = sB[(size_t)lc * S + (k - 1)];
-                    else if (!FUSED) jn = a.J[idx];
-                }
+            for (int q = 0; q < KPL; ++q) {
+                const int k = k0 + q;
+                if (!(SOLVE && !FUSED) || k >= nn) jn[q] = Jo[w][q];
+                if (SOLVE && k >= 1 && k <= nn - 2) jn[q] = sB[(size_t)lc * S + (k - 1)];
+                double hr = Hr[w][q], hz = Hz[w][q];
                 // the floor below would hide a NaN in J (max(NaN, Jeps) = Jeps): test first
-                if (FUSED) bad += !(__builtin_isfinite(jn) && __builtin_isfinite(hr) && __builtin_isfinite(hz));
+                if (FUSED && k < nn) bad += !(__builtin_isfinite(jn[q]) && __builtin_isfinite(hr) && __builtin_isfinite(hz));
                 if (HCORR) {
-                    double Jk = dmax(jn, kJeps);
-                    double inv_Jold = 1.0 / dmax(Jo[w][kk], kJeps);
-                    double ratio = Jk * inv_Jold;
+                    const double Jk = dmax(jn[q], kJeps);
+                    const double Jf = dmax(Jo[w][q], kJeps);
+                    double inv_Jold = recip(Jf);
+                    if (__builtin_expect(!(Jf < 0x1p500), 0)) inv_Jold = 1.0 / Jf;
+                    const double ratio = Jk * inv_Jold;
                     hr = hr * ratio;
                     hz = hz * ratio;
-                    double Hm2 = hr * hr + hz * hz;
+                    const double Hm2 = hr * hr + hz * hz;
                     if (Hm2 > Jk * Jk) {
-                        double s = Jk / sqrt(Hm2);
+                        const double s = Jk / sqrt(Hm2);
                         hr = hr * s;
                         hz = hz * s;
                     }
-                    jn = Jk;
+                    jn[q] = Jk;
                 }
-                a.J[idx] = jn; a.Hr[idx] = hr; a.Hz[idx] = hz;
-                if (!FUSED) { a.J_old[idx] = jn; a.Hr_old[idx] = hr; a.Hz_old[idx] = hz; }
-                if (FUSED) {
-                    const double dk = a.dnu[k];
-                    if (CONV) conv += dk * fabs(jn - a.J_old[idx]) * dV;
-                    e1[kk] += dk * dmax(jn - kJeps, 0.0) * dV;
-                    e10[kk] += dk * dmax(jn - 10 * kJeps, 0.0) * dV;
+                Hr[w][q] = hr; Hz[w][q] = hz;
+                if (FUSED && k < nn) {
+                    if (CONV) conv += dnu[q] * fabs(jn[q] - Js[q]) * dV;
+                    e1[q] += dnu[q] * dmax(jn[q] - kJeps, 0.0) * dV;
+                    e10[q] += dnu[q] * dmax(jn[q] - 10 * kJeps, 0.0) * dV;
                     // Compute_f_esc_Cylindrical terms (src/ConstantsAndFunctions.jl:937-953)
-                    if (i == nr - 1) esc += dk * (a.A_r[(size_t)j * (nr + 1) + nr] * kFourPi * dmax(hr, 0.0));
-                    if (j == nz - 1) esc += dk * (a.A_z[(size_t)nz * nr + i] * kFourPi * dmax(hz, 0.0));
-                    if (j == 0 && a.bc_z_bot == BC_OUTFLOW) esc += dk * (a.A_z[i] * kFourPi * dmax(-hz, 0.0));
+                    if (edge) {
+                        if (i == nr - 1) esc += dnu[q] * (a.A_r[(size_t)j * (nr + 1) + nr] * kFourPi * dmax(hr, 0.0));
+                        if (j == nz - 1) esc += dnu[q] * (a.A_z[(size_t)nz * nr + i] * kFourPi * dmax(hz, 0.0));
+                        if (j == 0 && a.bc_z_bot == BC_OUTFLOW) esc += dnu[q] * (a.A_z[i] * kFourPi * dmax(-hz, 0.0));
+                    }
                 }
             }
-            if (FUSED && (i == nr - 1 || j == nz - 1 || (j == 0 && a.bc_z_bot == BC_OUTFLOW)))
-                acc_esc += wave_sum(esc);
+            store_bins<KPL>(a.J + base, k0, nn, jn);
+            store_bins<KPL>(a.Hr + base, k0, nn, Hr[w]);
+            store_bins<KPL>(a.Hz + base, k0, nn, Hz[w]);
+            if (!FUSED) {
+                store_bins<KPL>(a.J_old + base, k0, nn, jn);
+                store_bins<KPL>(a.Hr_old + base, k0, nn, Hr[w]);
+                store_bins<KPL>(a.Hz_old + base, k0, nn, Hz[w]);
+            }
+            if (edge) acc_esc += esc;
         }
     }
     if (FUSED) {
@@ -689,20 +989,16 @@ __global__ __launch_bounds__(64 * NW) void k_column(ColumnArgs a)
         __syncthreads();
         double* wrow = lds + (size_t)wave * ncol;
 #pragma unroll
-        for (int kk = 0; kk < KPL; ++kk) {
-            const int k = lane + 64 * kk;
-            if (k < nn) { wrow[k] = e1[kk]; wrow[nn + k] = e10[kk]; }
+        for (int q = 0; q < KPL; ++q) {
+            const int k = k0 + q;
+            if (k < nn) { wrow[k] = e1[q]; wrow[nn + k] = e10[q]; }
         }
-        conv = wave_sum(conv);
-        const double nbad = wave_sum((double)bad);
+        const double sums[kStepSums] = {wave_sum_dpp(acc_mf), wave_sum_dpp(acc_L), wave_sum_dpp(acc_net),
+                                        wave_sum_dpp(acc_out), wave_sum_dpp(acc_esc), wave_sum_dpp(conv),
+                                        wave_sum_dpp((double)bad)};
         if (lane == 0) {
-            wrow[2 * nn + SUM_MF] = acc_mf;
-            wrow[2 * nn + SUM_L] = acc_L;
-            wrow[2 * nn + SUM_NET] = acc_net;
-            wrow[2 * nn + SUM_OUT] = acc_out;
-            wrow[2 * nn + SUM_ESC] = acc_esc;
-            wrow[2 * nn + SUM_CONV] = conv;
-            wrow[2 * nn + SUM_BAD] = nbad;
+#pragma unroll
+            for (int m = 0; m < kStepSums; ++m) wrow[2 * nn + m] = sums[m];
         }
         __syncthreads();
         double* prow = a.part + (size_t)blockIdx.x * a.pstride;
@@ -936,7 +1232,7 @@ void launch_advect(hipStream_t s, const AdvectArgs& a)
 template <int W, int KPL, int NW>
 static void launch_column_t(hipStream_t s, const ColumnArgs& a, int nblocks)
 {
-    const size_t rows = 4 * (size_t)col_stride(a.nn) * W * NW;
+    const size_t rows = 5 * (size_t)col_stride(a.nn) * W * NW + 2 * kColPad;
     const size_t sums = (size_t)NW * (2 * a.nn + kStepSums);
     const size_t lds = std::max(rows, sums) * sizeof(double);
     if ((a.flags & ~COL_CONV) == kFusedFlags)
@@ -945,39 +1241,39 @@ static void launch_column_t(hipStream_t s, const ColumnArgs& a, int nblocks)
         hipLaunchKernelGGL((k_column<W, KPL, NW, false>), dim3(nblocks), dim3(64 * NW), lds, s, a);
 }
 
-// Up to 256 bins (four per lane) four cell columns share a wavefront; beyond, up to 576 bins
-// (nine per lane, the reference's q = 1.03 grid of 542 bins), one column per wavefront keeps the
-// per-lane registers and the LDS rows within bounds.
-int column_width(int nn) { return nn <= 256 ? kColumnW : 1; }
-
-// Wavefronts per block of the column kernel: the block's W·NW columns fill 64 KB of LDS up to
-// 128 bins (16 columns), 64 KB up to 256 bins (8 columns); wider grids keep one wavefront
-// (one column of up to 18 KB).  Two blocks per CU then hold 8 wavefronts.
-int column_waves(int nn) { return nn <= 128 ? 4 : (nn <= 256 ? 2 : 1); }
-
-// A grid of exactly one wave of resident blocks: every block loops over the same number of
-// column groups and they all start together.  A larger grid left a partial second wave of
-// blocks starting late (2560 blocks against 2048 resident ones on the 256x256x128 cone
-// cloud: 1.15 ms against 0.81 ms for the kernel).  The count is fixed per block shape, so the
-// partition of the fused reductions does not depend on the device.
-int column_blocks(int nn, int ngroups)
+ColumnShape column_shape(int nn, size_t ncells)
 {
-    return std::max(1, std::min(ngroups, kColumnBlocks / column_waves(nn)));
+    ColumnShape c;
+    c.nw = nn <= 256 ? 4 : 1;
+    c.w = nn <= 128 ? kColumnW : (nn <= 256 ? 2 : 1);
+    while (c.w > 1 && ncells < (size_t)c.w * c.nw * 512) c.w /= 2;
+    const size_t groups = (ncells + (size_t)c.w * c.nw - 1) / ((size_t)c.w * c.nw);
+    c.blocks = (int)std::max<size_t>(1, std::min<size_t>(groups, (size_t)kColumnBlocks / c.nw));
+    return c;
 }
 
-void launch_column(hipStream_t s, const ColumnArgs& a, int nblocks)
+template <int KPL>
+static void launch_column_w(hipStream_t s, const ColumnArgs& a, const ColumnShape& c)
 {
-    const int kpl = (a.nn + 63) / 64;
-    switch (kpl) {
-    case 1: launch_column_t<kColumnW, 1, 4>(s, a, nblocks); break;
-    case 2: launch_column_t<kColumnW, 2, 4>(s, a, nblocks); break;
-    case 3: launch_column_t<kColumnW, 3, 2>(s, a, nblocks); break;
-    case 4: launch_column_t<kColumnW, 4, 2>(s, a, nblocks); break;
-    case 5: launch_column_t<1, 5, 1>(s, a, nblocks); break;
-    case 6: launch_column_t<1, 6, 1>(s, a, nblocks); break;
-    case 7: launch_column_t<1, 7, 1>(s, a, nblocks); break;
-    case 8: launch_column_t<1, 8, 1>(s, a, nblocks); break;
-    default: launch_column_t<1, 9, 1>(s, a, nblocks); break;
+    if constexpr (KPL <= 2) {
+        if (c.w == 4) return launch_column_t<4, KPL, 4>(s, a, c.blocks);
+    }
+    if (c.w >= 2) return launch_column_t<2, KPL, 4>(s, a, c.blocks);
+    launch_column_t<1, KPL, 4>(s, a, c.blocks);
+}
+
+void launch_column(hipStream_t s, const ColumnArgs& a, const ColumnShape& c)
+{
+    switch ((a.nn + 63) / 64) {
+    case 1: launch_column_w<1>(s, a, c); break;
+    case 2: launch_column_w<2>(s, a, c); break;
+    case 3: launch_column_w<3>(s, a, c); break;
+    case 4: launch_column_w<4>(s, a, c); break;
+    case 5: launch_column_t<1, 5, 1>(s, a, c.blocks); break;
+    case 6: launch_column_t<1, 6, 1>(s, a, c.blocks); break;
+    case 7: launch_column_t<1, 7, 1>(s, a, c.blocks); break;
+    case 8: launch_column_t<1, 8, 1>(s, a, c.blocks); break;
+    default: launch_column_t<1, 9, 1>(s, a, c.blocks); break;
     }
 }
 
