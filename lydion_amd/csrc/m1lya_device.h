@@ -31,6 +31,9 @@ enum { BC_REFLECT = 0, BC_OUTFLOW = 1 };
 
 __device__ __forceinline__ double dmax(double a, double b) { return (b > a) ? b : a; }
 __device__ __forceinline__ double dmin(double a, double b) { return (b < a) ? b : a; }
+// dmax for operands whose NaN, if any, reaches the result by another way: one instruction, and the
+// other operand where one is NaN
+__device__ __forceinline__ double dmax_num(double a, double b) { return __builtin_fmax(a, b); }
 __device__ __forceinline__ double dclamp(double x, double lo, double hi)
 {
     return (x > hi) ? hi : ((x < lo) ? lo : x);
@@ -121,11 +124,11 @@ __device__ __forceinline__ double minmod(double A, double B)
     return (fabs(A) < fabs(B)) ? A : B;
 }
 
-// Levermore (1984) closure factor: src/M1Closure.jl:28-33
+// Levermore (1984) closure factor, 0 <= f <= 1: src/M1Closure.jl:28-33
 __device__ __forceinline__ double chi_L84(double f)
 {
     double f2 = f * f;
-    return (3.0 + 4.0 * f2) / (5.0 + 2.0 * sqrt(4.0 - 3.0 * f2));
+    return quot(3.0 + 4.0 * f2, 5.0 + 2.0 * root(4.0 - 3.0 * f2));
 }
 
 struct Edd { double rr, zz, rz; };
@@ -141,10 +144,15 @@ __device__ inline Edd D_edd(double H_r, double H_z, double J)
         D.rr = kOneThird; D.zz = kOneThird; D.rz = 0.0;
         return D;
     }
-    double Hmag = sqrt(Hmag2);
-    double f = dclamp(Hmag / J, kFmin, kFmax);
+    double Hmag = root(Hmag2);   // Hmag2 > 1e-200 and J > 1e-60 here
+    double f = dclamp(quot(Hmag, J), kFmin, kFmax);
+    double inv_Hmag = recip(Hmag);
+    if (__builtin_expect(!(Hmag2 < 0x1p900) || !(J < 0x1p500), 0)) {
+        Hmag = sqrt(Hmag2);
+        f = dclamp(Hmag / J, kFmin, kFmax);
+        inv_Hmag = 1.0 / Hmag;
+    }
     double chi = chi_L84(f);
-    double inv_Hmag = 1.0 / Hmag;
     double a = (1.0 - chi) * 0.5;
     double b = (3.0 * chi - 1.0) * 0.5;
     double nr = H_r * inv_Hmag;
@@ -181,39 +189,47 @@ __device__ inline void hll_eigen(double f, double mu, double& l1, double& l3)
     f = dclamp(f, kFmin, kFmax);
     mu = dclamp(mu, -1.0, 1.0);
     double f2 = f * f, mu2 = mu * mu, muf = mu * f;
-    double SQ = sqrt(dmax(4.0 - 3.0 * f2, 0.0));
-    double inv_SQ = 1.0 / SQ;
+    double SQ = root(dmax(4.0 - 3.0 * f2, 0.0));   // f <= kFmax: the argument is above 1
+    double inv_SQ = recip(SQ);
     double FAC = sqrt(dmax(kTwoThirds * (4.0 - 3.0 * f2 - SQ) + 2.0 * mu2 * (2.0 - f2 - SQ), 0.0));
     l1 = dclamp((muf - FAC) * inv_SQ, -1.0, 1.0);
     l3 = dclamp((muf + FAC) * inv_SQ, -1.0, 1.0);
 }
 
-// State of the four cells of one interface stencil, in the reference's
+// H/J of one cell (J floored as in the reference's reconstruction): every interface whose stencil
+// holds the cell divides by the same J, so a cell's ratios are formed once.
+__device__ __forceinline__ void flux_ratios(double J, double Hr, double Hz, double& fr, double& fz)
+{
+    const double Jm = dmax(J, kJeps);
+    double inv_J = recip(Jm);
+    if (__builtin_expect(!(Jm < 0x1p500), 0)) inv_J = 1.0 / Jm;
+    fr = Hr * inv_J;
+    fz = Hz * inv_J;
+}
+
+// State of the four cells of one interface stencil (J and the flux ratios), in the reference's
 // argument order: (i, i+1, i+2, i-1) where i is the cell left of the face.
 struct Stencil {
-    double J[4], Hr[4], Hz[4];
+    double J[4], fr[4], fz[4];
 };
 
 struct Recon {
-    double J_L, J_R, Hr_L, Hr_R, Hz_L, Hz_R, tau_L, tau_R, f_L, f_R, nr_L, nr_R, nz_L, nz_R;
+    double J_L, J_R, Hr_L, Hr_R, Hz_L, Hz_R, tau, f_L, f_R, nr_L, nr_R, nz_L, nz_R;
+    bool plain;   // no lane needs the general divisions of this interface
 };
 
 // ReconstructInterface: src/AdvectJandH.jl:359-473.
 // iv = {ΔL, ΔR, 1/(x_i-x_{i-1}), 1/(x_{i+1}-x_i), 1/(x_{i+2}-x_{i+1})}
-__device__ inline Recon reconstruct(const Stencil& s, const double* iv, double aF_i, double aF_ip1)
+// With f > 1 the limited direction (f_r, f_Z)/f is the direction itself, so that one reciprocal
+// of |f| serves the limiter and the direction.  A vanishing flux or a depth beyond 2^400 in any
+// lane sends the wavefront to the divisions and roots of any range.
+__device__ __forceinline__ Recon reconstruct(const Stencil& s, const double* iv, double aF_i, double aF_ip1)
 {
     const double dL = iv[0], dR = iv[1], inv_i_im1 = iv[2], inv_ip1_i = iv[3], inv_ip2_ip1 = iv[4];
     Recon o;
-    o.tau_L = aF_i * dL;
-    o.tau_R = aF_ip1 * dR;
-    double inv_J_i = 1.0 / dmax(s.J[0], kJeps);
-    double inv_J_ip1 = 1.0 / dmax(s.J[1], kJeps);
-    double inv_J_ip2 = 1.0 / dmax(s.J[2], kJeps);
-    double inv_J_im1 = 1.0 / dmax(s.J[3], kJeps);
-    double fr_i = s.Hr[0] * inv_J_i, fr_ip1 = s.Hr[1] * inv_J_ip1;
-    double fr_ip2 = s.Hr[2] * inv_J_ip2, fr_im1 = s.Hr[3] * inv_J_im1;
-    double fz_i = s.Hz[0] * inv_J_i, fz_ip1 = s.Hz[1] * inv_J_ip1;
-    double fz_ip2 = s.Hz[2] * inv_J_ip2, fz_im1 = s.Hz[3] * inv_J_im1;
+    o.tau = aF_i * dL + aF_ip1 * dR;
+    const double fr_i = s.fr[0], fr_ip1 = s.fr[1], fr_ip2 = s.fr[2], fr_im1 = s.fr[3];
+    const double fz_i = s.fz[0], fz_ip1 = s.fz[1], fz_ip2 = s.fz[2], fz_im1 = s.fz[3];
 
     double dJc = (s.J[1] - s.J[0]) * inv_ip1_i;
     double dJL = minmod((s.J[0] - s.J[3]) * inv_i_im1, dJc);
@@ -225,26 +241,32 @@ __device__ inline Recon reconstruct(const Stencil& s, const double* iv, double a
     double dfzL = minmod((fz_i - fz_im1) * inv_i_im1, dfzc);
     double dfzR = minmod((fz_ip2 - fz_ip1) * inv_ip2_ip1, dfzc);
 
-    double J_L = dmax(s.J[0] + dJL * dL, kJeps);
-    double J_R = dmax(s.J[1] - dJR * dR, kJeps);
+    // a NaN J leaves the flux ratios NaN, and with them every flux
+    double J_L = dmax_num(s.J[0] + dJL * dL, kJeps);
+    double J_R = dmax_num(s.J[1] - dJR * dR, kJeps);
     double fr_L = fr_i + dfrL * dL;
     double fr_R = fr_ip1 - dfrR * dR;
     double fz_L = fz_i + dfzL * dL;
     double fz_R = fz_ip1 - dfzR * dR;
 
-    double f_L = sqrt(fr_L * fr_L + fz_L * fz_L);
-    if (f_L > 1.0) {
-        double inv_f = 1.0 / f_L;
-        fr_L *= inv_f; fz_L *= inv_f; f_L = 1.0;
+    const double f2_L = fr_L * fr_L + fz_L * fz_L, f2_R = fr_R * fr_R + fz_R * fz_R;
+    double f_L, f_R, inv_L, inv_R;
+    o.plain = !__any(!(f2_L >= 0x1p-700) || !(f2_R >= 0x1p-700) || !(o.tau <= 0x1p400));
+    if (__builtin_expect(o.plain, 1)) {
+        f_L = root(f2_L);
+        f_R = root(f2_R);
+        inv_L = recip(f_L);
+        inv_R = recip(f_R);
+    } else {
+        f_L = sqrt(f2_L);
+        f_R = sqrt(f2_R);
+        inv_L = f_L > 0.0 ? 1.0 / f_L : 0.0;
+        inv_R = f_R > 0.0 ? 1.0 / f_R : 0.0;
     }
-    double f_R = sqrt(fr_R * fr_R + fz_R * fz_R);
-    if (f_R > 1.0) {
-        double inv_f = 1.0 / f_R;
-        fr_R *= inv_f; fz_R *= inv_f; f_R = 1.0;
-    }
-    o.nr_L = 0.0; o.nz_L = 0.0; o.nr_R = 0.0; o.nz_R = 0.0;
-    if (f_L > 0.0) { double inv = 1.0 / f_L; o.nr_L = fr_L * inv; o.nz_L = fz_L * inv; }
-    if (f_R > 0.0) { double inv = 1.0 / f_R; o.nr_R = fr_R * inv; o.nz_R = fz_R * inv; }
+    o.nr_L = fr_L * inv_L; o.nz_L = fz_L * inv_L;
+    o.nr_R = fr_R * inv_R; o.nz_R = fz_R * inv_R;
+    if (f_L > 1.0) { fr_L = o.nr_L; fz_L = o.nz_L; f_L = 1.0; }
+    if (f_R > 1.0) { fr_R = o.nr_R; fz_R = o.nz_R; f_R = 1.0; }
     o.J_L = J_L; o.J_R = J_R;
     o.Hr_L = fr_L * J_L; o.Hr_R = fr_R * J_R;
     o.Hz_L = fz_L * J_L; o.Hz_R = fz_R * J_R;
@@ -254,16 +276,28 @@ __device__ inline Recon reconstruct(const Stencil& s, const double* iv, double a
 
 struct Flux3 { double J, Hr, Hz; };
 
+// ϵ of the thick / thin blend and the Fick flux -ΔJ/(3τ)
+__device__ __forceinline__ void thick_blend(const Recon& q, double J_i, double J_ip1, double& eps, double& F_J_diff)
+{
+    const double num = 0.2 + q.tau, den = num + q.tau * q.tau;
+    const double tau_eff = dmax(q.tau, 1e-300);
+    const double d = -kOneThird * (J_ip1 - J_i);
+    if (__builtin_expect(q.plain, 1)) {
+        eps = quot(num, den);
+        F_J_diff = quot(d, tau_eff);
+    } else {
+        eps = num / den;
+        F_J_diff = d / tau_eff;
+    }
+}
+
 // GetFluxGLF: src/AdvectJandH.jl:81-118 (F* are the physical fluxes at the two sides)
 __device__ inline Flux3 flux_glf(double FJ_L, double FJ_R, double FHr_L, double FHr_R,
                                  double FHz_L, double FHz_R, const Recon& q, double J_i, double J_ip1)
 {
-    double tau_cell = q.tau_L + q.tau_R;
-    double num = 0.2 + tau_cell;
-    double eps = num / (num + tau_cell * tau_cell);
+    double eps, F_J_diff;
+    thick_blend(q, J_i, J_ip1, eps, F_J_diff);
     double ome = 1.0 - eps;
-    double tau_eff = dmax(tau_cell, 1e-300);
-    double F_J_diff = -kOneThird * (J_ip1 - J_i) / tau_eff;
     double F_J_GLF = 0.5 * (FJ_L + FJ_R) - 0.5 * (q.J_R - q.J_L);
     Flux3 F;
     F.J = eps * F_J_GLF + ome * F_J_diff;
@@ -278,16 +312,13 @@ __device__ inline Flux3 flux_hll(double FJ_L, double FJ_R, double FHr_L, double 
                                  double FHz_L, double FHz_R, const Recon& q, double J_i, double J_ip1,
                                  double l1L, double l1R, double l3L, double l3R)
 {
-    double tau_cell = q.tau_L + q.tau_R;
-    double num = 0.2 + tau_cell;
-    double eps = num / (num + tau_cell * tau_cell);
+    double eps, F_J_diff;
+    thick_blend(q, J_i, J_ip1, eps, F_J_diff);
     double ome = 1.0 - eps;
     double half_ome = 0.5 * ome;
-    double tau_eff = dmax(tau_cell, 1e-300);
-    double F_J_diff = -kOneThird * (J_ip1 - J_i) / tau_eff;
     double S_R = dmax(dmax(l3L, l3R), 0.0);
     double S_L = dmin(dmin(l1L, l1R), 0.0);
-    double inv_dS = 1.0 / dmax(S_R - S_L, 1e-300);
+    double inv_dS = recip(dmax(S_R - S_L, 1e-300));
     double SRSL = S_R * S_L;
     double FJ = (S_R * FJ_L - S_L * FJ_R + SRSL * (q.J_R - q.J_L)) * inv_dS;
     double FHr = (S_R * FHr_L - S_L * FHr_R + SRSL * (q.Hr_R - q.Hr_L)) * inv_dS;
@@ -321,7 +352,7 @@ struct FaceResult {
     double kphi_L, kphi_R;   // clamp(1 - D_rr - D_ZZ, 0, 1) * J at the two sides (r only)
 };
 
-__device__ inline FaceResult interface_flux(int dir, int hll, const Stencil& s, const double* iv,
+__device__ __forceinline__ FaceResult interface_flux(int dir, int hll, const Stencil& s, const double* iv,
                                             double aF_L, double aF_R, double u_over_c)
 {
     Recon q = reconstruct(s, iv, aF_L, aF_R);
@@ -346,15 +377,18 @@ __device__ inline FaceResult interface_flux(int dir, int hll, const Stencil& s, 
     } else {
         F = flux_glf(FJ_L, FJ_R, FHr_L, FHr_R, FHz_L, FHz_R, q, s.J[0], s.J[1]);
     }
-    // GetAdvectionFlux: src/AdvectJandH.jl:276-282
-    bool up = (u_over_c < 0.0);
     FaceResult r;
-    r.F.J = F.J + u_over_c * (up ? q.J_R : q.J_L);
-    r.F.Hr = F.Hr + u_over_c * (up ? q.Hr_R : q.Hr_L);
-    r.F.Hz = F.Hz + u_over_c * (up ? q.Hz_R : q.Hz_L);
+    r.F = F;
+    if (u_over_c != 0.0) {   // the face velocity is one value for all bins: a uniform branch
+        // GetAdvectionFlux: src/AdvectJandH.jl:276-282
+        bool up = (u_over_c < 0.0);
+        r.F.J = F.J + u_over_c * (up ? q.J_R : q.J_L);
+        r.F.Hr = F.Hr + u_over_c * (up ? q.Hr_R : q.Hr_L);
+        r.F.Hz = F.Hz + u_over_c * (up ? q.Hz_R : q.Hz_L);
+    }
     r.J_L = q.J_L; r.J_R = q.J_R; r.Hz_R = q.Hz_R;
-    r.kphi_L = dclamp(1.0 - DL.rr - DL.zz, 0.0, 1.0) * q.J_L;
-    r.kphi_R = dclamp(1.0 - DR.rr - DR.zz, 0.0, 1.0) * q.J_R;
+    r.kphi_L = __builtin_fmin(dmax_num(1.0 - DL.rr - DL.zz, 0.0), 1.0) * q.J_L;
+    r.kphi_R = __builtin_fmin(dmax_num(1.0 - DR.rr - DR.zz, 0.0), 1.0) * q.J_R;
     return r;
 }
 

@@ -195,12 +195,14 @@ __device__ __forceinline__ void advect_cell_update(const AdvectArgs& a, int i, i
     const double cdt_over_c = cdt * kInvC;
     const double durdr = a.v.dur_dr[c], durdz = a.v.dur_dz[c], duzdr = a.v.duz_dr[c];
     const double duzdz = a.v.duz_dz[c], urr = a.v.ur_over_r[c];
-    Edd D = D_edd(Hrs, Hzs, Js);
+    // With no velocity gradient D:∇u is +0 whatever D is (its rr, zz and ϕϕ entries are >= 0)
+    const bool still = durdr == 0.0 && durdz == 0.0 && duzdr == 0.0 && duzdz == 0.0 && urr == 0.0;
+    double Ddu = 0.0;
+    if (!still) Ddu = D_colon_grad_u(D_edd(Hrs, Hzs, Js), durdr, durdz, duzdr, duzdz, urr);
     double Jn = Js - cdt_dV * ((Ar_R * FrR[0] - Ar_L * FrL[0]) + (Az_R * FzR[0] - Az_L * FzL[0]));
     Jn = dmax(Jn, kJeps);
     double Hzn = Hzs - cdt_dV * ((Ar_R * FrR[2] - Ar_L * FrL[2]) + (Az_R * FzR[2] - Az_L * FzL[2]));
     double Hrn = Hrs - cdt_dV * ((Ar_R * FrR[1] - Ar_L * FrL[1]) + (Az_R * FzR[1] - Az_L * FzL[1]));
-    double Ddu = D_colon_grad_u(D, durdr, durdz, duzdr, duzdz, urr);
     double Kav = 0.5 * (kphi_im + kphi_ip);
     Hrn += cdt * Kav * a.g.inv_r_cell[i];
     double dHr = -cdt_over_c * (Hrs * durdr + Hzs * durdz);
@@ -228,20 +230,26 @@ __device__ __forceinline__ void advect_cell_update(const AdvectArgs& a, int i, i
 // row) in registers and evaluates one r face per cell; the left face of a cell
 // is the right face of the one before it.  The Z faces of the block's rows go
 // through LDS: every wavefront publishes its cell's state, wavefront w evaluates
-// face j0 + w and wavefront 0 also the block's top face.  That is 1 + 1/seg_len
+// face j0 + w and one wavefront also the block's top face.  That is 1 + 1/seg_len
 // r faces and 1 + 1/WPB Z faces per cell.  All fluxes of a step are computed from
 // the same old state (read from the input buffers, written to separate ones), as
 // in the reference; bins outside [kmin, kmax] are copied.  A face's value does not
 // depend on which wavefront evaluates it, so the result is the one of a per-cell
 // evaluation.
+// What bounds it: FP64 instruction issue (67 % of its cycles) and the wait for the block's
+// slowest wavefront at each cell's barrier.  256x256x128 cone cloud: 405 -> 345 us and 1.58e8 ->
+// 1.05e8 wave instructions (H/J formed once per cell, divisions and roots without range
+// handling, no closure for cells at rest), -> 325 us with one barrier per cell instead of two
+// and the window loaded a cell ahead.  Blocks of 4 rows: 344 us.
 // ------------------------------------------------------------------------
 template <int WPB>
-__global__ __launch_bounds__(64 * WPB) void k_advect(AdvectArgs a, int seg_len)
+__global__ __launch_bounds__(64 * WPB, 4) void k_advect(AdvectArgs a, int seg_len)
 {
-    // Z stencil rows j0-2 .. j0+WPB+1 of the current column (J, H_r, H_Z, ghost-mapped) and the
-    // Z faces j0 .. j0+WPB (F_J, F_Hr, F_HZ)
-    __shared__ double zrow[WPB + 4][3][64];
-    __shared__ double zflx[WPB + 1][3][64];
+    // Z stencil rows j0-2 .. j0+WPB+1 of a column (J, H_r/J, H_Z/J, ghost-mapped) and the Z faces
+    // j0 .. j0+WPB (F_J, F_Hr, F_HZ), each for two columns in turn: the rows of column i+1 are
+    // published while the faces of column i are evaluated, so that one barrier per cell does
+    __shared__ double zrow[2][WPB + 4][3][64];
+    __shared__ double zflx[2][WPB + 1][3][64];
     if (a.halt && *a.halt) return;
     const int nn = a.nn, nr = a.g.nr, nz = a.g.nz;
     const int lane = threadIdx.x & 63;
@@ -254,65 +262,74 @@ __global__ __launch_bounds__(64 * WPB) void k_advect(AdvectArgs a, int seg_len)
     const int kmin = a.krange[0], kmax = a.krange[1];
     const bool act = kin && k >= kmin && k <= kmax;
     const SpecIn s{a.J, a.Hr, a.Hz};
+    auto put_zrow = [&](int buf, int slot, int i, int row) {
+        double vj, vr, vz, fr, fz;
+        load_z(s, nn, nr, nz, i, k, min(row, nz + 1), a.bc_z_bot, a.bc_z_top, vj, vr, vz);
+        flux_ratios(vj, vr, vz, fr, fz);
+        zrow[buf][slot][0][lane] = vj; zrow[buf][slot][1][lane] = fr; zrow[buf][slot][2][lane] = fz;
+    };
 
-    // r window of row j: cells (i-1, i, i+1, i+2) in slots 0..3; before the march, cells
-    // i0-2, i0-1, i0 in slots 1..3, so that the first shift and load make (i0-2 .. i0+1)
-    double wJ[4] = {0.0, 0.0, 0.0, 0.0}, wHr[4] = {0.0, 0.0, 0.0, 0.0}, wHz[4] = {0.0, 0.0, 0.0, 0.0};
-    if (act && row_ok) {
+    // r window of row j (J, H_r/J, H_Z/J): cells (i-1, i, i+1, i+2) in slots 0..3; before the
+    // march, cells i0-2, i0-1, i0 in slots 1..3, so that the first shift and load make (i0-2 .. i0+1)
+    double wJ[4] = {0.0, 0.0, 0.0, 0.0}, wR[4] = {0.0, 0.0, 0.0, 0.0}, wZ[4] = {0.0, 0.0, 0.0, 0.0};
+    double nJ = 0.0, nHr = 0.0, nHz = 0.0;   // the window's next cell, loaded a cell ahead
+    double aFL = 0.0;                        // α_F of cell i, the left side of its right face
+    const bool march = act && row_ok;
+    if (march) {
 #pragma unroll
-        for (int m = 1; m < 4; ++m) load_r(s, nn, nr, j, k, i0 - 3 + m, a.bc_r_right, wJ[m], wHr[m], wHz[m]);
+        for (int m = 1; m < 4; ++m) {
+            double vr, vz;
+            load_r(s, nn, nr, j, k, i0 - 3 + m, a.bc_r_right, wJ[m], vr, vz);
+            flux_ratios(wJ[m], vr, vz, wR[m], wZ[m]);
+        }
+        load_r(s, nn, nr, j, k, i0 + 1, a.bc_r_right, nJ, nHr, nHz);
+        aFL = a.aF[((size_t)j * nr + max(i0 - 1, 0)) * nn + k];
     }
     // left r face of cell i: its flux and the K_ϕϕ of its right side
     double FL[3] = {0.0, 0.0, 0.0}, KL = 0.0;
     for (int i = i0 - 1; i < i1; ++i) {
-        double FR[3] = {0.0, 0.0, 0.0}, KRl = 0.0, KRr = 0.0;
-        if (act && row_ok) {
+        double FR[3] = {0.0, 0.0, 0.0}, KRl = 0.0, KRr = 0.0, Hrs = 0.0, Hzs = 0.0;
+        if (march) {
 #pragma unroll
-            for (int m = 0; m < 3; ++m) { wJ[m] = wJ[m + 1]; wHr[m] = wHr[m + 1]; wHz[m] = wHz[m + 1]; }
-            load_r(s, nn, nr, j, k, i + 2, a.bc_r_right, wJ[3], wHr[3], wHz[3]);
+            for (int m = 0; m < 3; ++m) { wJ[m] = wJ[m + 1]; wR[m] = wR[m + 1]; wZ[m] = wZ[m + 1]; }
+            wJ[3] = nJ;
+            flux_ratios(nJ, nHr, nHz, wR[3], wZ[3]);
+            if (i + 1 < i1) load_r(s, nn, nr, j, k, i + 3, a.bc_r_right, nJ, nHr, nHz);
             // face f = i + 1 between cells i and i+1; stencil (i, i+1, i+2, i-1)
             const int f = i + 1;
             Stencil st;
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 const int slot = (m + 1) & 3;
-                st.J[m] = wJ[slot]; st.Hr[m] = wHr[slot]; st.Hz[m] = wHz[slot];
+                st.J[m] = wJ[slot]; st.fr[m] = wR[slot]; st.fz[m] = wZ[slot];
             }
-            const double aFL = a.aF[((size_t)j * nr + max(f - 1, 0)) * nn + k];
             const double aFR = a.aF[((size_t)j * nr + min(f, nr - 1)) * nn + k];
             const double u = a.v.ur_star[(size_t)j * (nr + 1) + f] * kInvC;
             const FaceResult r = interface_flux(0, a.hll, st, a.g.ivr + (size_t)f * 5, aFL, aFR, u);
             FR[0] = r.F.J; FR[1] = r.F.Hr; FR[2] = r.F.Hz;
             KRl = r.kphi_L;
             KRr = (f == 0) ? kphi_inner_axis(r.J_R, r.Hz_R) : r.kphi_R;
+            aFL = aFR;
         }
-        if (i < i0) {
-#pragma unroll
-            for (int m = 0; m < 3; ++m) FL[m] = FR[m];
-            KL = KRr;
-            continue;
-        }
-        // ---- Z faces of column i through LDS ----
-        if (act) {
+        // ---- Z faces through LDS: column i+1's rows out, column i's faces ----
+        if (act && i + 1 < i1) {
+            const int buf = (i + 1) & 1;
             if (row_ok) {
-                zrow[w + 2][0][lane] = wJ[1]; zrow[w + 2][1][lane] = wHr[1]; zrow[w + 2][2][lane] = wHz[1];
+                zrow[buf][w + 2][0][lane] = wJ[2]; zrow[buf][w + 2][1][lane] = wR[2]; zrow[buf][w + 2][2][lane] = wZ[2];
             } else {
-                double vj, vr, vz;   // a ghost row above the grid (rows past N_Z + 1 feed no needed face)
-                load_z(s, nn, nr, nz, i, k, min(j, nz + 1), a.bc_z_bot, a.bc_z_top, vj, vr, vz);
-                zrow[w + 2][0][lane] = vj; zrow[w + 2][1][lane] = vr; zrow[w + 2][2][lane] = vz;
+                put_zrow(buf, w + 2, i + 1, j);   // a ghost row above the grid (rows past N_Z + 1 feed no needed face)
             }
             for (int h = w; h < 4; h += WPB) {
                 const int slot = (h < 2) ? h : WPB + h;
-                double vj, vr, vz;
-                load_z(s, nn, nr, nz, i, k, min(j0 - 2 + slot, nz + 1), a.bc_z_bot, a.bc_z_top, vj, vr, vz);
-                zrow[slot][0][lane] = vj; zrow[slot][1][lane] = vr; zrow[slot][2][lane] = vz;
+                put_zrow(buf, slot, i + 1, j0 - 2 + slot);
             }
         }
-        __syncthreads();
-        if (act) {
+        if (act && i >= i0) {
+            const int buf = i & 1;
+            // wavefront w evaluates face j0 + w, and each in turn the block's top face too
 #pragma unroll 1
             for (int it = 0; it < 2; ++it) {
-                if (it && w != 0) break;
+                if (it && w != (i & (WPB - 1))) break;
                 const int fz = it ? WPB : w;    // the face's slot: face g = j0 + fz
                 const int g = j0 + fz;
                 if (g > nz) continue;
@@ -320,26 +337,32 @@ __global__ __launch_bounds__(64 * WPB) void k_advect(AdvectArgs a, int seg_len)
 #pragma unroll
                 for (int m = 0; m < 4; ++m) {
                     const int slot = fz + ((m + 1) & 3);   // rows (g-1, g, g+1, g-2)
-                    st.J[m] = zrow[slot][0][lane]; st.Hr[m] = zrow[slot][1][lane]; st.Hz[m] = zrow[slot][2][lane];
+                    st.J[m] = zrow[buf][slot][0][lane]; st.fr[m] = zrow[buf][slot][1][lane];
+                    st.fz[m] = zrow[buf][slot][2][lane];
                 }
-                const double aFL = a.aF[((size_t)max(g - 1, 0) * nr + i) * nn + k];
-                const double aFR = a.aF[((size_t)min(g, nz - 1) * nr + i) * nn + k];
+                const double aL = a.aF[((size_t)max(g - 1, 0) * nr + i) * nn + k];
+                const double aR = a.aF[((size_t)min(g, nz - 1) * nr + i) * nn + k];
                 const double u = a.v.uz_star[(size_t)g * nr + i] * kInvC;
-                const FaceResult r = interface_flux(1, a.hll, st, a.g.ivz + (size_t)g * 5, aFL, aFR, u);
-                zflx[fz][0][lane] = r.F.J; zflx[fz][1][lane] = r.F.Hr; zflx[fz][2][lane] = r.F.Hz;
+                const FaceResult r = interface_flux(1, a.hll, st, a.g.ivz + (size_t)g * 5, aL, aR, u);
+                zflx[buf][fz][0][lane] = r.F.J; zflx[buf][fz][1][lane] = r.F.Hr; zflx[buf][fz][2][lane] = r.F.Hz;
             }
         }
+        const size_t idx = ((size_t)j * nr + max(i, 0)) * nn + k;
+        if (march && i >= i0) {   // the cell's own H, for its update
+            Hrs = s.Hr[idx];
+            Hzs = s.Hz[idx];
+        }
         __syncthreads();
-        if (row_ok && kin) {
-            const size_t idx = ((size_t)j * nr + i) * nn + k;
+        if (row_ok && kin && i >= i0) {
             if (!act) {
                 a.J_out[idx] = s.J[idx];
                 a.Hr_out[idx] = s.Hr[idx];
                 a.Hz_out[idx] = s.Hz[idx];
             } else {
-                const double FzL[3] = {zflx[w][0][lane], zflx[w][1][lane], zflx[w][2][lane]};
-                const double FzR[3] = {zflx[w + 1][0][lane], zflx[w + 1][1][lane], zflx[w + 1][2][lane]};
-                advect_cell_update(a, i, j, idx, wJ[1], wHr[1], wHz[1], FL, FR, FzL, FzR, KL, KRl);
+                const int buf = i & 1;
+                const double FzL[3] = {zflx[buf][w][0][lane], zflx[buf][w][1][lane], zflx[buf][w][2][lane]};
+                const double FzR[3] = {zflx[buf][w + 1][0][lane], zflx[buf][w + 1][1][lane], zflx[buf][w + 1][2][lane]};
+                advect_cell_update(a, i, j, idx, wJ[1], Hrs, Hzs, FL, FR, FzL, FzR, KL, KRl);
             }
         }
 #pragma unroll
@@ -1216,15 +1239,22 @@ void launch_active_final(hipStream_t s, const double* red, int nn, int kcmin, in
 
 void launch_advect(hipStream_t s, const AdvectArgs& a)
 {
-    // Rows of 8 wavefronts marching over segments of 16 cells: 1.0625 r faces and 1.125 Z faces
-    // per cell, 32 KB of LDS per block.  Segments are halved while the grid holds fewer blocks
-    // than MI355X keeps resident (2 per CU at 123 VGPRs, 512 in all): on the 128x128x128
-    // expanding cloud 8-cell segments take 0.110 ms against 0.120 ms for 16 (256 blocks), on
-    // the 256x256x128 cone cloud 16 and 8 are within 1%.
-    constexpr int WPB = 8, kResident = 512;
+    // Rows of 8 wavefronts marching over segments of up to 16 cells: 1.0625 r faces and 1.125 Z
+    // faces per cell, 32 KB of LDS per block.  The segment is the one of the least estimated time: a
+    // block takes its cells plus the face before the first one (about 0.6 of a cell), two blocks on a
+    // CU (all that 121 VGPRs allow) take 1.65 times one block's time, and a CU gets its share of the
+    // blocks.  On the 32x32x64 cloud that is single cells, 13 us against 29 us for the four-cell
+    // segments that a fixed lower bound gave; on 77x90x194 eight cells, 133 against 135 us for four;
+    // on 128x192x64 four, 80 against 86 us for seven.
+    constexpr int WPB = 8, kCUs = 256, kSegMax = 16;
     const int chunks = (a.nn + 63) / 64, rows = (a.g.nz + WPB - 1) / WPB;
-    int seg = 16;
-    while (seg > 4 && chunks * ((a.g.nr + seg - 1) / seg) * rows < kResident) seg /= 2;
+    int seg = kSegMax;
+    double best = 0.0;
+    for (int t = kSegMax; t >= 1; --t) {
+        const long per_cu = ((long)chunks * ((a.g.nr + t - 1) / t) * rows + kCUs - 1) / kCUs;
+        const double cost = (1.65 * (double)(per_cu / 2) + (double)(per_cu % 2)) * (t + 0.6);
+        if (t == kSegMax || cost < best) { best = cost; seg = t; }
+    }
     dim3 grid(chunks, (a.g.nr + seg - 1) / seg, rows);
     hipLaunchKernelGGL((k_advect<WPB>), grid, dim3(64 * WPB), 0, s, a, seg);
 }
