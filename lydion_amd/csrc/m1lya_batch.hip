@@ -18,13 +18,13 @@
 //     reduction across the 64 lanes;
 //   * H rescale and causality, FP32 store into the other state buffer;
 //   * Neumaier-compensated FP64 accumulation of M_F, L, f_esc and the active-bin
-//     energies: per block (k_step), per slice of a cloud's blocks (k_reduce), then per
-//     cloud (k_final).
+//     energies: per block (k_step, or k_rows for short segments), per slice of a cloud's blocks
+//     (k_reduce), then per cloud (k_final).
 //
 // Work items (one per wavefront) and partial-sum rows (one per block) cover every
-// cloud of the batch, so uneven clouds share one launch.  The three launches of a
-// step can be captured into a hipGraph per buffer parity; the segment length and
-// the number of wavefronts per block are chosen by a timing autotuner.
+// cloud of the batch, so uneven clouds share one launch.  The launches of a step can be
+// captured into a hipGraph per buffer parity.  The segment length follows from the batch's
+// sizes; a caller may set the tile shape, or have the timing autotuner choose it.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -33,6 +33,8 @@
 #include <cstring>
 #include <map>
 #include <string>
+#include <tuple>
+#include <utility>
 #include <vector>
 
 #include "../../include/m1lya.h"
@@ -59,6 +61,8 @@ constexpr int kMaxBins = 256;                    // four bins per lane
 constexpr int kNScal = 7;                        // MF, L, net, out, esc, ΔJ sum, non-finite count
 constexpr int kPartStride = 2 * kMaxBins + 8;    // e1[N_ν], e10[N_ν], scalars
 constexpr int kMaxWaves = 8;
+constexpr int kSegLen = 16;                      // segment and block height of the default tiles, and of
+constexpr int kRowWaves = 8;                     // the blocks whose partial rows k_rows forms
 constexpr int kSlices = 16;                      // row slices of the first reduction stage
 
 // Per-cell inputs of the step, one 160-byte record per cell (read with scalar loads).
@@ -81,7 +85,7 @@ struct Cloud {
     int nn, nr, nz, R;
     int pair;                      // N_ν <= 32: two cells per wavefront (k_step<..., 1, true>)
     long long o3, oc, ofr, ofz, obin, oivr, oivz;
-    int blk0, blk1;                // this cloud's partial rows (= its blocks)
+    int row0, row1;                // this cloud's partial rows
     int kcore_min, kcore_max, recoil, hll;
     int bc_r_right, bc_z_bot, bc_z_top, has_vel;
     float cdt, cdtc;               // c̃Δt and c̃Δt/c for the FP32 flux sweep
@@ -126,6 +130,7 @@ struct Arrays {
     float *uc_r, *uc_z;
     float *ivr, *ivz;
     double *f_r, *f_z;
+    int* bad;            // [n_clouds]: a step of short segments wrote a non-finite J, H_r or H_Z
 };
 
 // ------------------------------------------------------------------------
@@ -410,6 +415,21 @@ __device__ __forceinline__ void aniso_row(const BinRec* __restrict__ bins, const
     rd = -dw * jo;
 }
 
+// Update_f_Lyα_MF_L_Lyα! terms of one cell (src/ConstantsAndFunctions.jl:612-660)
+__device__ __forceinline__ void cell_terms(const CellRec* cr, double fr, double fz, double z_center, double& mf,
+                                           double& ls, double& net, double& out)
+{
+    const double dV = cr->dV;
+    mf = dV * sqrt(fr * fr + fz * fz);
+    ls = kFourPi * dV * cr->js;
+    const double ddr = cr->rcom, ddz = cr->zcom - z_center;
+    const double d2 = ddr * ddr + ddz * ddz;
+    double frad = 0.0;
+    if (d2 > 0.0) frad = (fr * ddr + fz * ddz) * drcp1(sqrt(d2));
+    net = dV * frad;
+    out = dV * (frad > 0.0 ? frad : 0.0);
+}
+
 // LDS of a k_step block of wpb wavefronts (dynamic, so that 4-wavefront blocks keep four
 // blocks per CU while 8-wavefront blocks take two):
 //   sbin  BinRec[64 NQ]                 the cloud's frequency-bin constants, read every cell
@@ -428,11 +448,13 @@ constexpr size_t step_lds_bytes(int wpb, int nq)
 // kPair (with NQ = 1, clouds of N_ν <= 32): the two halves of a wavefront hold two neighbouring
 // cells of its row, i (lanes 0-31) and i+1 (lanes 32-63), one bin per lane, so that such clouds
 // fill every lane; the march advances two cells at a time.  The launch covers the blocks
-// [blk0, blk1) of the batch.
+// [blk0, blk1) of the batch.  rows: the block forms its partial row; without it (short segments)
+// k_rows does.
 template <bool kShear, int NQ, bool kPair>
 __global__ __launch_bounds__(64 * kMaxWaves, NQ <= 2 ? 4 : 2) void k_step(const Cloud* __restrict__ clouds, Arrays A,
                                                             const Seg* __restrict__ segs, int blk0, int blk1,
-                                                            int wpb, int parity, const int* __restrict__ krange,
+                                                            int wpb, int parity, int rows,
+                                                            const int* __restrict__ krange,
                                                             double* __restrict__ part, const Ctrl* __restrict__ ctrl)
 {
     static_assert(!kPair || NQ == 1, "pair mode holds one bin per lane");
@@ -1026,6 +1048,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, NQ <= 2 ? 4 : 2) void k_step(const 
             cw.sJ[parity ^ 1][idx] = Jf;
             cw.sHr[parity ^ 1][idx] = hrf;
             cw.sHz[parity ^ 1][idx] = hzf;
+            if (!rows) continue;
             const double Jd = Jf, dk = bins[k].dnu;
             conv += dk * (double)fabsf(Jf - wJ[q][1]) * cr.dV;
             const int e1k = kPair ? 32 * half + k : k, e10k = kPair ? 64 + 32 * half + k : nn + k;
@@ -1037,7 +1060,7 @@ __global__ __launch_bounds__(64 * kMaxWaves, NQ <= 2 ? 4 : 2) void k_step(const 
                         (cr.A_rout * fmax((double)hrf, 0.0) + cr.A_ztop * fmax((double)hzf, 0.0) +
                          Azb * fmax(-(double)hzf, 0.0));
         }
-        if (kPair ? (__ballot(edge) != 0) : edge) kadd(S_ESC, wave_sum64(escl) * cv.J0);
+        if (rows && (kPair ? (__ballot(edge) != 0) : edge)) kadd(S_ESC, wave_sum64(escl) * cv.J0);
     }
 
     // ---- Update_f_Lyα_MF_L_Lyα! per-cell terms (src/ConstantsAndFunctions.jl:612-660) of the
@@ -1052,20 +1075,18 @@ __global__ __launch_bounds__(64 * kMaxWaves, NQ <= 2 ? 4 : 2) void k_step(const 
             const double fr = seg_sr * cv.mf_scale, fz = seg_sz * cv.mf_scale;
             cv.sfr[cell] = fr;
             cv.sfz[cell] = fz;
-            const double dV = cr->dV;
-            mf = dV * sqrt(fr * fr + fz * fz);
-            ls = kFourPi * dV * cr->js;
-            const double ddr = cr->rcom, ddz = cr->zcom - cv.z_center;
-            const double d2 = ddr * ddr + ddz * ddz;
-            double frad = 0.0;
-            if (d2 > 0.0) frad = (fr * ddr + fz * ddz) * drcp1(sqrt(d2));
-            net = dV * frad;
-            out = dV * (frad > 0.0 ? frad : 0.0);
+            cell_terms(cr, fr, fz, cv.z_center, mf, ls, net, out);
         }
-        kadd(S_MF, wave_sum64(mf));
-        kadd(S_L, wave_sum64(ls));
-        kadd(S_NET, wave_sum64(net));
-        kadd(S_OUT, wave_sum64(out));
+        if (rows) {
+            kadd(S_MF, wave_sum64(mf));
+            kadd(S_L, wave_sum64(ls));
+            kadd(S_NET, wave_sum64(net));
+            kadd(S_OUT, wave_sum64(out));
+        }
+    }
+    if (!rows) {
+        if (__any(bad != 0) && lane == 0) A.bad[cidx] = 1;
+        return;
     }
 
     // ---- block partial row: per-wavefront values in LDS, summed in wavefront order ----
@@ -1103,52 +1124,204 @@ __global__ __launch_bounds__(64 * kMaxWaves, NQ <= 2 ? 4 : 2) void k_step(const 
     }
 }
 
-// Active-bin energies straight from the state (before the first step after an
-// upload): block rows in k_step's format, scalars zero.
-__global__ __launch_bounds__(64 * kMaxWaves) void k_active_rows(const Cloud* __restrict__ clouds, Arrays A,
-                                                     const Seg* __restrict__ segs, int nblk, int wpb, int parity,
-                                                     double* __restrict__ part)
+// Element off of a wave-uniform slice (a 32-bit byte offset: one register per load in flight)
+__device__ __forceinline__ float at(const float* base, unsigned off)
 {
-    __shared__ double sh[kMaxWaves][kPartStride];
-    const int lb = xcd_block(blockIdx.x, gridDim.x);
-    if (lb >= nblk) return;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const Seg sg = segs[(size_t)lb * wpb + wave];
-    const Cloud& cb = clouds[segs[(size_t)lb * wpb].cloud];
-    const int nnb = cb.nn, R = cb.R;
-    double e1[4] = {0.0, 0.0, 0.0, 0.0}, e10[4] = {0.0, 0.0, 0.0, 0.0};
-    if (sg.j < cb.nz) {
-        const float* J = A.J[parity] + cb.o3;
-        for (int i = sg.i0; i < sg.i1; ++i) {
-            const size_t cell = (size_t)sg.j * cb.nr + i;
-            const double dV = A.rec[cb.oc + cell].dV;
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + off * 4u);
+}
+
+// Change of J over a row segment's cells, a lane's bins kl .. kl + NQ - 1 each.  All of a group's
+// loads are issued before the first is used; the terms and their order are k_step's.
+template <int NQ>
+__device__ __forceinline__ double row_change(const Cloud& cb, const BinRec* __restrict__ bin, const Seg& sg, int half,
+                                             int kl, int step, int parity)
+{
+    constexpr int kGroup = NQ == 4 ? 4 : 8;
+    const int nnb = cb.nn;
+    double dk[NQ], conv = 0.0;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int k = lane * R + q;
-                if (q >= R || k >= nnb) continue;
-                const double Jd = J[cell * nnb + k];
-                const double dk = A.bin[cb.obin + k].dnu;
-                e1[q] += dk * ((Jd - kJeps) > 0.0 ? (Jd - kJeps) : 0.0) * dV;
-                e10[q] += dk * ((Jd - 10.0 * kJeps) > 0.0 ? (Jd - 10.0 * kJeps) : 0.0) * dV;
+    for (int q = 0; q < NQ; ++q) dk[q] = bin[min(kl + q, nnb - 1)].dnu;
+    for (int g = sg.i0; g < sg.i1; g += kGroup * step) {
+        const size_t cell = (size_t)sg.j * cb.nr + g;
+        const float *J = cb.sJ[parity] + cell * nnb, *Jp = cb.sJ[parity ^ 1] + cell * nnb;
+        const CellRec* cr = cb.srec + cell;
+        const int n = sg.i1 - g;
+        float Jf[kGroup][NQ], Jo[kGroup][NQ];
+#pragma unroll
+        for (int m = 0; m < kGroup; ++m) {
+            const int i = min(m * step + half, n - 1);
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const unsigned off = i * nnb + min(kl + q, nnb - 1);
+                Jf[m][q] = at(J, off);
+                Jo[m][q] = at(Jp, off);
             }
         }
-    }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int k = lane * R + q;
-        if (q < R && k < nnb) {
-            sh[wave][k] = e1[q] * cb.J0;
-            sh[wave][nnb + k] = e10[q] * cb.J0;
+        for (int m = 0; m < kGroup; ++m) {
+            const int i = m * step + half;
+            const double dV = cr[min(i, n - 1)].dV;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q)
+                if (i < n && kl + q < nnb) conv += dk[q] * (double)fabsf(Jf[m][q] - Jo[m][q]) * dV;
         }
     }
-    if (lane < kNScal) sh[wave][2 * nnb + lane] = 0.0;
+    return conv;
+}
+
+// Escaping flux of a row segment's edge cells, as row_change.
+template <int NQ>
+__device__ __forceinline__ double row_escape(const Cloud& cb, const BinRec* __restrict__ bin, const Seg& sg, int lane,
+                                             int half, int kl, int step, int parity)
+{
+    constexpr int kGroup = NQ == 4 ? 4 : 8;
+    const int nnb = cb.nn;
+    const bool open = cb.bc_z_bot == M1LYA_OUTFLOW;
+    double dk[NQ];
+    KSum esc{0.0, 0.0};
+    const CellRec* ce = cb.srec + (size_t)sg.j * cb.nr + min(sg.i0 + lane, sg.i1 - 1);
+    if (!__any(ce->A_rout != 0.0 || ce->A_ztop != 0.0 || (open && ce->A_zbot != 0.0))) return 0.0;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) dk[q] = bin[min(kl + q, nnb - 1)].dnu;
+    for (int g = sg.i0; g < sg.i1; g += kGroup * step) {
+        const size_t cell = (size_t)sg.j * cb.nr + g;
+        const float *Hr = cb.sHr[parity] + cell * nnb, *Hz = cb.sHz[parity] + cell * nnb;
+        const CellRec* cr = cb.srec + cell;
+        const int n = sg.i1 - g;
+        float hr[kGroup][NQ], hz[kGroup][NQ];
+        double Ar[kGroup], At[kGroup], Ab[kGroup];
+#pragma unroll
+        for (int m = 0; m < kGroup; ++m) {
+            const int i = min(m * step + half, n - 1);
+            Ar[m] = cr[i].A_rout;
+            At[m] = cr[i].A_ztop;
+            Ab[m] = open ? cr[i].A_zbot : 0.0;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const unsigned off = i * nnb + min(kl + q, nnb - 1);
+                hr[m][q] = at(Hr, off);
+                hz[m][q] = at(Hz, off);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < kGroup; ++m) {
+            const bool edge = m * step + half < n && (Ar[m] != 0.0 || At[m] != 0.0 || Ab[m] != 0.0);
+            double escl = 0.0;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                if (!edge || kl + q >= nnb) continue;
+                escl += dk[q] * kFourPi * (Ar[m] * fmax((double)hr[m][q], 0.0) + At[m] * fmax((double)hz[m][q], 0.0) +
+                                           Ab[m] * fmax(-(double)hz[m][q], 0.0));
+            }
+            if (__any(edge)) esc.add(wave_sum64(escl) * cb.J0);
+        }
+    }
+    return esc.value();
+}
+
+// Partial rows straight from the state: the active-bin energies alone before the first step after
+// an upload (sums = 0), and all of a row's sums after a step whose k_step ran on shorter segments,
+// for the blocks of the default tiles (kRowWaves rows of kSegLen cells).  Every lane takes the bins
+// and, in the same order, the cells that it takes in k_step, and the terms are formed by the same
+// operations, so a row has the bits that k_step gives it, and no result depends on the tiles.
+// Blocks (row, 0 .. R - 1): the energies of the lanes' bin q; (row, R): the escaping flux;
+// (row, R + 1): the other scalars.  Grids that need this leave the chip idle, so it is bound by
+// latency: a wavefront has the loads of many cells in flight, and a row is cut into R + 2 blocks.  32x32x64 7.0 us, 100x84x194 21 us;
+// 9.7 and 21 with a block per row, 16 and 36 with a cell at a time.
+__global__ __launch_bounds__(64 * kMaxWaves, 4) void k_rows(const Cloud* __restrict__ clouds, Arrays A,
+                                                         const Seg* __restrict__ segs, int nblk, int wpb, int parity,
+                                                         int sums, double* __restrict__ part,
+                                                         const Ctrl* __restrict__ ctrl)
+{
+    __shared__ double sh[kMaxWaves][128];
+    if (sums && ctrl->halt) return;
+    const int lb = xcd_block(blockIdx.x, gridDim.x);
+    if (lb >= nblk) return;
+    const int lane = threadIdx.x & 63, q = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const Seg sg = segs[(size_t)lb * wpb + wave];
+    const int cidx = segs[(size_t)lb * wpb].cloud;
+    const Cloud& cb = clouds[cidx];
+    const int nnb = cb.nn, R = cb.R, pair = cb.pair;
+    if (q > R + 1) return;
+    const int half = pair ? lane >> 5 : 0, kl = pair ? (lane & 31) : lane * R, step = pair ? 2 : 1;
+    const BinRec* bin = A.bin + cb.obin;
+    double* row = part + (size_t)lb * kPartStride;
+    if (q < R) {
+        // active-bin energies of the lane's bin kl + q
+        const int k = min(kl + q, nnb - 1);
+        double e1 = 0.0, e10 = 0.0;
+        if (sg.j < cb.nz) {
+            const double dk = bin[k].dnu;
+            for (int g = sg.i0; g < sg.i1; g += 8 * step) {
+                const size_t cell = (size_t)sg.j * cb.nr + g;
+                const float* J = cb.sJ[parity] + cell * nnb;
+                const CellRec* cr = cb.srec + cell;
+                const int n = sg.i1 - g;
+                float Jf[8];
+#pragma unroll
+                for (int m = 0; m < 8; ++m) Jf[m] = at(J, min(m * step + half, n - 1) * nnb + k);
+#pragma unroll
+                for (int m = 0; m < 8; ++m) {
+                    if (m * step + half >= n) continue;
+                    const double Jd = Jf[m], dV = cr[min(m * step + half, n - 1)].dV;
+                    e1 += dk * ((Jd - kJeps) > 0.0 ? (Jd - kJeps) : 0.0) * dV;
+                    e10 += dk * ((Jd - 10.0 * kJeps) > 0.0 ? (Jd - 10.0 * kJeps) : 0.0) * dV;
+                }
+            }
+        }
+        if (pair) {
+            // fold the two halves, as k_step does
+            e1 += __shfl_xor(e1, 32, 64);
+            e10 += __shfl_xor(e10, 32, 64);
+        }
+        sh[wave][lane] = e1 * cb.J0;
+        sh[wave][64 + lane] = e10 * cb.J0;
+        __syncthreads();
+        for (int t = threadIdx.x; t < 128; t += blockDim.x) {
+            const int l = t & 63, kt = pair ? l : l * R + q;
+            if (kt >= nnb) continue;
+            KSum s{0, 0};
+            for (int w = 0; w < wpb; ++w) s.add(sh[w][t]);
+            row[t < 64 ? kt : nnb + kt] = s.value();
+        }
+        return;
+    }
+    // M_F, L, net, out, change of J, non-finite count; or the escaping flux alone
+    const bool escape = q == R;
+    double v[kNScal] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (sums && sg.j < cb.nz) {
+        if (escape) {
+            if (R == 1) v[4] = row_escape<1>(cb, bin, sg, lane, half, kl, step, parity);
+            else if (R == 2) v[4] = row_escape<2>(cb, bin, sg, lane, half, kl, step, parity);
+            else v[4] = row_escape<4>(cb, bin, sg, lane, half, kl, step, parity);
+        } else {
+            const int i = sg.i0 + lane;
+            if (i < sg.i1) {
+                const size_t cell = (size_t)sg.j * cb.nr + i;
+                cell_terms(cb.srec + cell, cb.sfr[cell], cb.sfz[cell], cb.z_center, v[0], v[1], v[2], v[3]);
+            }
+            if (R == 1) v[5] = row_change<1>(cb, bin, sg, half, kl, step, parity);
+            else if (R == 2) v[5] = row_change<2>(cb, bin, sg, half, kl, step, parity);
+            else v[5] = row_change<4>(cb, bin, sg, half, kl, step, parity);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) v[m] = wave_sum64(v[m]);
+            v[5] = wave_sum64(v[5]) * cb.J0;
+        }
+    }
+    if (lane == 0) {
+        if (sums && !escape && wave == 0 && lb == cb.row0) {
+            v[6] = A.bad[cidx];
+            A.bad[cidx] = 0;
+        }
+#pragma unroll
+        for (int m = 0; m < kNScal; ++m) sh[wave][m] = v[m];
+    }
     __syncthreads();
-    const int ncol = 2 * nnb + kNScal;
-    for (int t = threadIdx.x; t < ncol; t += blockDim.x) {
+    if (threadIdx.x < kNScal && (threadIdx.x == 4) == escape) {
         KSum s{0, 0};
-        for (int w = 0; w < wpb; ++w) s.add(sh[w][t]);
-        part[(size_t)lb * kPartStride + t] = s.value();
+        for (int w = 0; w < wpb; ++w) s.add(sh[w][threadIdx.x]);
+        row[2 * nnb + threadIdx.x] = s.value();
     }
 }
 
@@ -1163,7 +1336,7 @@ __global__ __launch_bounds__(256) void k_reduce(const Cloud* __restrict__ clouds
     // the halt flag and the cloud's extents are loaded together (one memory latency)
     const int halt = ctrl->halt;
     const Cloud& cl = clouds[blockIdx.y];
-    const int nn = cl.nn, blk0 = cl.blk0, blk1 = cl.blk1;
+    const int nn = cl.nn, row0 = cl.row0, row1 = cl.row1;
     const bool halted = halt != 0;
     if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) {
         ctrl->live = !halted;
@@ -1174,9 +1347,9 @@ __global__ __launch_bounds__(256) void k_reduce(const Cloud* __restrict__ clouds
     const int col = blockIdx.x * 64 + lane;
     const int ncol = 2 * nn + kNScal;
     if ((int)blockIdx.x * 64 >= ncol) return;
-    const int nrow = blk1 - blk0;
+    const int nrow = row1 - row0;
     const int per = (nrow + kSlices - 1) / kSlices;
-    const int r0 = blk0 + (int)blockIdx.z * per, r1 = min(blk1, r0 + per);
+    const int r0 = row0 + (int)blockIdx.z * per, r1 = min(row1, r0 + per);
     KSum acc{0, 0};
     if (col < ncol) {
         // kRows rows of the wavefront's share are loaded before any is added, so their loads
@@ -1347,6 +1520,7 @@ struct m1lya_batch {
     double nu_lya = 0.0;
     bool shear = false;                    // a cell's velocity gradient is sheared or anisotropic
     bool wide = false;                     // a cloud has more than 128 bins (four per lane)
+    int max_R = 1;                         // most bins per lane of any cloud
     std::vector<BinRec> h_bin;
     CellRec* d_rec = nullptr;
     BinRec* d_bin = nullptr;
@@ -1355,11 +1529,15 @@ struct m1lya_batch {
     bool krange_valid = false;
 
     // tile shape and the work / partial-row tables it implies
-    int seg_len = 16, wpb = 8;   // the autotuner's choice on the 256x256x128 cone cloud
+    int seg_len = kSegLen, wpb = kRowWaves;
+    bool auto_tiles = true;      // the segments follow from the batch's sizes (until a caller sets the shape)
     std::vector<Seg> segs;
     Seg* d_segs = nullptr;
     size_t segs_cap = 0;
-    int nblk = 0, grid = 0;
+    Seg* d_row_segs = nullptr;             // the default tiles, whose blocks k_rows works on
+    size_t row_segs_cap = 0;
+    bool step_rows = true;                 // k_step's blocks are those of the partial rows and form them
+    int nblk = 0, nrows = 0;
     int nblk_pair = 0;                     // blocks [0, nblk_pair) belong to clouds in pair mode
     double* part = nullptr;
     size_t part_rows_cap = 0;
@@ -1448,47 +1626,95 @@ void check_cloud(m1lya_batch* b, int c)
     if (c < 0 || c >= b->n) bfail(b, M1LYA_ERR_ARG, "cloud index out of range");
 }
 
-// Work table of the current tile shape: per cloud, row segments of seg_len cells,
-// wpb of them (same i range, consecutive rows) per block; blocks never mix clouds.  The
-// blocks of clouds in pair mode come first: they are launched on their own.
+// Segment length for the batch's clouds (pair: those of N_ν <= 32, which have a launch of their
+// own).  A block takes its cells plus about one for its setup and first interface; a CU works
+// through its share of the blocks, two at a time in 1.45 times one block's time (one at a time with
+// four bins per lane).  The length of the least estimated time, the longest among equals; the
+// default tiles stay unless shorter ones save a quarter: their partial rows cost a launch, and a chip
+// whose CUs hold one block or two gains less than the estimate (sweep of 16, 400 blocks: 231 us, as
+// 512 blocks of 11 to 13 cells).
+// us per step: 32x32x64 30 at 1 cell, 104 at 16; 64x64x128 45 at 1, 140; 128x128x128 87 at 4, 158;
+// 100x84x194 145 at 5, 326; the 256x256x128 cone cloud keeps 16.
+int auto_segment(const m1lya_batch* b, bool pair)
+{
+    int best_seg = kSegLen;
+    double best = 0.0;
+    for (int seg = kSegLen; seg >= 1; --seg) {
+        long blocks = 0;
+        for (const Cloud& cl : b->cl)
+            if ((cl.pair != 0) == pair) blocks += (long)((cl.nr + seg - 1) / seg) * ((cl.nz + kRowWaves - 1) / kRowWaves);
+        constexpr int kCUs = 256;
+        const long per_cu = (blocks + kCUs - 1) / kCUs;
+        const bool single = b->wide && !pair;
+        const double rounds = single ? (double)per_cu : 1.45 * (double)(per_cu / 2) + (double)(per_cu % 2);
+        const double cost = rounds * (seg + (pair ? 2.0 : 1.0));
+        if (seg == kSegLen) best = 0.75 * cost;
+        else if (cost < best) { best = cost; best_seg = seg; }
+    }
+    return best_seg;
+}
+
+// Work tables.  Per cloud, row segments of one length, wpb of them (same i range, consecutive
+// rows) per block; blocks never mix clouds.  The blocks of clouds in pair mode come first: they are
+// launched on their own.  With segments of the caller's choice, or of the default length, a block
+// is a partial row of its cloud; else the rows are those of the default tiles.
 void build_tiles(m1lya_batch* b)
 {
-    std::vector<Seg> segs;
-    int blk = 0;
     std::vector<int> order;
     for (int pass = 0; pass < 2; ++pass)
         for (int c = 0; c < b->n; ++c)
             if ((b->cl[c].pair != 0) == (pass == 0)) order.push_back(c);
-    int nblk_pair = 0;
-    for (int c : order) {
-        Cloud& cl = b->cl[c];
-        cl.blk0 = blk;
-        const int nseg_r = (cl.nr + b->seg_len - 1) / b->seg_len;
-        for (int j0 = 0; j0 < cl.nz; j0 += b->wpb)
-            for (int s = 0; s < nseg_r; ++s) {
-                // rows j0+w >= N_Z are ghost rows: their wavefronts only take part in
-                // the Z exchange of the block
-                for (int w = 0; w < b->wpb; ++w)
-                    segs.push_back(Seg{c, j0 + w, s * b->seg_len, std::min(cl.nr, (s + 1) * b->seg_len)});
-                ++blk;
-            }
-        cl.blk1 = blk;
-        if (cl.pair) nblk_pair = blk;
+    auto table = [&](const int (&len)[2], int wpb, std::vector<Seg>& segs, bool rows) {
+        int blk = 0, nblk_pair = 0;
+        for (int c : order) {
+            Cloud& cl = b->cl[c];
+            const int L = len[cl.pair != 0], nseg_r = (cl.nr + L - 1) / L;
+            if (rows) cl.row0 = blk;
+            for (int j0 = 0; j0 < cl.nz; j0 += wpb)
+                for (int s = 0; s < nseg_r; ++s) {
+                    // rows j0+w >= N_Z are ghost rows: their wavefronts only take part in
+                    // the Z exchange of the block
+                    for (int w = 0; w < wpb; ++w) segs.push_back(Seg{c, j0 + w, s * L, std::min(cl.nr, (s + 1) * L)});
+                    ++blk;
+                }
+            if (rows) cl.row1 = blk;
+            if (cl.pair) nblk_pair = blk;
+        }
+        return std::make_pair(blk, nblk_pair);
+    };
+    auto push = [&](const std::vector<Seg>& segs, Seg*& d, size_t& cap) {
+        if (segs.size() > cap) {
+            bfree(b, d);
+            d = nullptr;
+            d = balloc<Seg>(b, segs.size());
+            cap = segs.size();
+        }
+        bchk(b, hipMemcpy(d, segs.data(), segs.size() * sizeof(Seg), hipMemcpyHostToDevice), "segments");
+    };
+    const int len_rows[2] = {kSegLen, kSegLen};
+    int len[2] = {b->seg_len, b->seg_len};   // clouds out of / in pair mode
+    if (b->auto_tiles) {
+        bool any[2] = {false, false};
+        for (const Cloud& cl : b->cl) any[cl.pair != 0] = true;
+        for (int p = 0; p < 2; ++p) len[p] = any[p] ? auto_segment(b, p != 0) : kSegLen;
+        b->wpb = kRowWaves;
+        b->seg_len = len[any[0] ? 0 : 1];
     }
-    b->nblk = blk;
-    b->nblk_pair = nblk_pair;
-    b->grid = (blk + 7) / 8 * 8;
-    if (segs.size() > b->segs_cap) {
-        bfree(b, b->d_segs);
-        b->d_segs = balloc<Seg>(b, segs.size());
-        b->segs_cap = segs.size();
+    b->step_rows = !b->auto_tiles || (len[0] == kSegLen && len[1] == kSegLen);
+    std::vector<Seg> segs, row_segs;
+    std::tie(b->nblk, b->nblk_pair) = table(len, b->wpb, segs, b->step_rows);
+    b->nrows = b->nblk;
+    push(segs, b->d_segs, b->segs_cap);
+    if (!b->step_rows) {
+        b->nrows = table(len_rows, kRowWaves, row_segs, true).first;
+        push(row_segs, b->d_row_segs, b->row_segs_cap);
     }
-    if ((size_t)blk > b->part_rows_cap) {
+    if ((size_t)b->nrows > b->part_rows_cap) {
         bfree(b, b->part);
-        b->part = balloc<double>(b, (size_t)blk * kPartStride);
-        b->part_rows_cap = blk;
+        b->part = nullptr;
+        b->part = balloc<double>(b, (size_t)b->nrows * kPartStride);
+        b->part_rows_cap = b->nrows;
     }
-    bchk(b, hipMemcpy(b->d_segs, segs.data(), segs.size() * sizeof(Seg), hipMemcpyHostToDevice), "segments");
     b->segs = std::move(segs);
     b->cl_dirty = true;
     drop_graphs(b);
@@ -1602,10 +1828,10 @@ void launch_step_kernels(m1lya_batch* b, int parity)
         const dim3 grid((b->nblk_pair + 7) / 8 * 8);
         if (b->shear)
             hipLaunchKernelGGL((k_step<true, 1, true>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, 0, b->nblk_pair,
-                               b->wpb, parity, b->krange, b->part, b->ctrl);
+                               b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
         else
             hipLaunchKernelGGL((k_step<false, 1, true>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, 0,
-                               b->nblk_pair, b->wpb, parity, b->krange, b->part, b->ctrl);
+                               b->nblk_pair, b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
         p.done();
     }
     if (b->nblk > b->nblk_pair) {
@@ -1619,17 +1845,23 @@ void launch_step_kernels(m1lya_batch* b, int parity)
         if (b->wide) {
             if (b->shear)
                 hipLaunchKernelGGL((k_step<true, 4, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
-                                   b->wpb, parity, b->krange, b->part, b->ctrl);
+                                   b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
             else
                 hipLaunchKernelGGL((k_step<false, 4, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
-                                   b->wpb, parity, b->krange, b->part, b->ctrl);
+                                   b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
         } else if (b->shear) {
             hipLaunchKernelGGL((k_step<true, 2, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
-                               b->wpb, parity, b->krange, b->part, b->ctrl);
+                               b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
         } else {
             hipLaunchKernelGGL((k_step<false, 2, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
-                               b->wpb, parity, b->krange, b->part, b->ctrl);
+                               b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
         }
+        p.done();
+    }
+    if (!b->step_rows) {
+        BProf p(b, "k_rows");
+        hipLaunchKernelGGL(k_rows, dim3((b->nrows + 7) / 8 * 8, b->max_R + 2), dim3(64 * kRowWaves), 0, s, b->d_cl, b->A,
+                           b->d_row_segs, b->nrows, kRowWaves, parity ^ 1, 1, b->part, b->ctrl);
         p.done();
     }
     {
@@ -1649,9 +1881,9 @@ void compute_krange(m1lya_batch* b)
 {
     sync_clouds(b);
     hipStream_t s = b->stream;
-    hipLaunchKernelGGL(k_active_rows, dim3(b->grid), dim3(64 * b->wpb), 0, s, b->d_cl, b->A, b->d_segs, b->nblk,
-                       b->wpb, b->parity, b->part);
-    bchk(b, hipGetLastError(), "k_active_rows");
+    hipLaunchKernelGGL(k_rows, dim3((b->nrows + 7) / 8 * 8, b->max_R + 2), dim3(64 * b->wpb), 0, s, b->d_cl, b->A,
+                       b->step_rows ? b->d_segs : b->d_row_segs, b->nrows, b->wpb, b->parity, 0, b->part, b->ctrl);
+    bchk(b, hipGetLastError(), "k_rows");
     hipLaunchKernelGGL(k_reduce, dim3((2 * kMaxBins + kNScal + 63) / 64, b->n, kSlices), dim3(256), 0, s, b->d_cl,
                        b->part, b->red, b->ctrl);
     bchk(b, hipGetLastError(), "k_reduce");
@@ -1817,6 +2049,7 @@ int m1lya_batch_create(int n_clouds, const int* n_nu, const int* n_r, const int*
             cl.R = cl.nn <= 64 ? 1 : cl.nn <= 128 ? 2 : 4;
             cl.pair = cl.nn <= 32;
             if (cl.R == 4) b->wide = true;
+            b->max_R = std::max(b->max_R, cl.R);
             const size_t ncell = (size_t)cl.nr * cl.nz;
             cl.o3 = (long long)b->n3; b->n3 += ncell * cl.nn;
             cl.oc = (long long)b->nc; b->nc += ncell;
@@ -1855,6 +2088,7 @@ int m1lya_batch_create(int n_clouds, const int* n_nu, const int* n_r, const int*
         b->scalars = balloc<double>(b, (size_t)n_clouds * 8);
         b->ctrl = balloc<Ctrl>(b, 1);
         b->steady = balloc<int>(b, (size_t)n_clouds);
+        A.bad = balloc<int>(b, (size_t)n_clouds);
         build_tiles(b);
     });
     if (rc != M1LYA_OK) {
@@ -2273,6 +2507,7 @@ int m1lya_batch_set_tiles(m1lya_batch* b, int seg_len, int waves_per_block)
         if (seg_len < 1 || seg_len > 64) bfail(b, M1LYA_ERR_ARG, "seg_len out of range [1, 64]");
         if (waves_per_block < 1 || waves_per_block > kMaxWaves) bfail(b, M1LYA_ERR_ARG, "waves_per_block must be 1..8");
         bchk(b, hipStreamSynchronize(b->stream), "hipStreamSynchronize");
+        b->auto_tiles = false;
         b->seg_len = seg_len;
         b->wpb = waves_per_block;
         build_tiles(b);
@@ -2297,8 +2532,8 @@ int m1lya_batch_set_graph(m1lya_batch* b, int on)
     });
 }
 
-// Times every tile shape of the candidate set on the live batch and keeps the
-// fastest.  State, active-bin ranges and buffer parity are restored, so the call
+// Times every tile shape of the candidate set, and the one that the batch's sizes give, on the
+// live batch and keeps the fastest.  State, active-bin ranges and buffer parity are restored, so the call
 // does not advance the simulation (the step scalars are those of the last trial).
 // Everything m1lya_batch_autotune changes, put back on every exit: the trial buffers and
 // events are released, profiling is restored, and unless the sweep finished the tile shape,
@@ -2312,10 +2547,10 @@ struct AutotuneScope {
     int* sK = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int prof, seg, wpb, parity;
-    bool saved = false, finished = false;
+    bool auto_tiles, saved = false, finished = false;
 
     explicit AutotuneScope(m1lya_batch* bb)
-        : b(bb), prof(bb->profiling), seg(bb->seg_len), wpb(bb->wpb), parity(bb->parity) {}
+        : b(bb), prof(bb->profiling), seg(bb->seg_len), wpb(bb->wpb), parity(bb->parity), auto_tiles(bb->auto_tiles) {}
 
     void copy(void* dst, const void* src, size_t n)
     {
@@ -2348,7 +2583,8 @@ struct AutotuneScope {
             // an error left a trial candidate in place: best effort back to the entry state,
             // the error itself is what the call reports
             try {
-                if (b->seg_len != seg || b->wpb != wpb) {
+                if (b->seg_len != seg || b->wpb != wpb || b->auto_tiles != auto_tiles) {
+                    b->auto_tiles = auto_tiles;
                     b->seg_len = seg;
                     b->wpb = wpb;
                     build_tiles(b);
@@ -2388,9 +2624,9 @@ int m1lya_batch_autotune(m1lya_batch* b, int trial_steps, int* seg_len, int* wav
         // occupancy, on 256 rows of 256 cells) and the lengths that give 3 or 6 wavefronts
         // per SIMD on 256-cell rows; 2, 4 or 8 wavefronts per block (taller blocks share
         // more Z interfaces and halo rows, shorter ones fit more blocks per CU)
-        static const int seg_opts[] = {6, 8, 11, 16, 22, 32, 43, 64};
+        static const int seg_opts[] = {0, 6, 8, 11, 16, 22, 32, 43, 64};
         static const int wpb_opts[] = {2, 4, 8};
-        int best_s = b->seg_len, best_w = b->wpb;
+        int best_s = b->auto_tiles ? 0 : b->seg_len, best_w = b->wpb;
         double best = 1e300;
         bchk(b, hipEventCreate(&scope.e0), "hipEventCreate");
         bchk(b, hipEventCreate(&scope.e1), "hipEventCreate");
@@ -2399,6 +2635,9 @@ int m1lya_batch_autotune(m1lya_batch* b, int trial_steps, int* seg_len, int* wav
         for (int pass = 0; pass < 2; ++pass)
         for (int s : seg_opts)
             for (int w : wpb_opts) {
+                // segment length 0: the length that follows from the sizes, once
+                if (s == 0 && w != wpb_opts[0]) continue;
+                b->auto_tiles = s == 0;
                 b->seg_len = s;
                 b->wpb = w;
                 build_tiles(b);
@@ -2422,6 +2661,7 @@ int m1lya_batch_autotune(m1lya_batch* b, int trial_steps, int* seg_len, int* wav
                     best_w = w;
                 }
             }
+        b->auto_tiles = best_s == 0;
         b->seg_len = best_s;
         b->wpb = best_w;
         build_tiles(b);
@@ -2429,8 +2669,8 @@ int m1lya_batch_autotune(m1lya_batch* b, int trial_steps, int* seg_len, int* wav
         scope.restore();
         bchk(b, hipStreamSynchronize(b->stream), "hipStreamSynchronize");
         scope.finished = true;
-        if (seg_len) *seg_len = best_s;
-        if (waves_per_block) *waves_per_block = best_w;
+        if (seg_len) *seg_len = b->seg_len;
+        if (waves_per_block) *waves_per_block = b->wpb;
         if (best_ms) *best_ms = best;
     });
 }
