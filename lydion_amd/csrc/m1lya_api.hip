@@ -13,6 +13,7 @@
 
 #include "../../include/m1lya.h"
 #include "m1lya_internal.h"
+#include "m1lya_transfer.h"
 
 using namespace m1;
 
@@ -88,6 +89,7 @@ struct m1lya_ctx {
     size_t history_cap = 0;
 
     std::vector<void*> allocs;
+    m1t::Download down;
     std::string err;
 
     int profiling = 0;   // 0 off, 1 every launch, 2 the fused step's column kernel only
@@ -446,6 +448,16 @@ void replay_step(m1lya_ctx* c, double c_tilde, double dt, double z_center, int b
     c->fij_stale = true;
 }
 
+// Copies to the host behind the stream's work; complete on return if large, else once the
+// stream is synchronised.
+void download(m1lya_ctx* c, double* host, const double* src, size_t n, const char* what)
+{
+    if (n * sizeof(double) >= m1t::kMinBytes && m1t::pageable(host))
+        hipchk(c, c->down.run(host, src, n, 1.0, c->device, c->stream), what);
+    else
+        hipchk(c, hipMemcpyAsync(host, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream), what);
+}
+
 template <class F>
 int guarded(m1lya_ctx* c, F&& f)
 {
@@ -545,6 +557,7 @@ void m1lya_destroy(m1lya_ctx* c)
         (void)hipEventDestroy(p.e1);
     }
     for (hipEvent_t e : c->pool) (void)hipEventDestroy(e);
+    c->down.release();
     for (void* p : c->allocs) (void)hipFree(p);
     if (c->history) (void)hipFree(c->history);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -666,8 +679,7 @@ int m1lya_download(m1lya_ctx* c, int field, double* host, size_t count)
         if (count != fi.count)
             fail(c, M1LYA_ERR_ARG, "field " + std::to_string(field) + ": count " + std::to_string(count) +
                                        " != " + std::to_string(fi.count));
-        hipchk(c, hipMemcpyAsync(host, fi.ptr, count * sizeof(double), hipMemcpyDeviceToHost, c->stream),
-               "download");
+        download(c, host, fi.ptr, count, "download");
         hipchk(c, hipStreamSynchronize(c->stream), "sync");
         check_err_flag(c, "step");
     });
@@ -1417,12 +1429,9 @@ int m1lya_adjoint_run(m1lya_ctx* c, int n_steps, double c_tilde, double dt, doub
         if (Lsum > 0.0 && obj != 0.0) launch_adj_axpy_cell(st, gcell + 2 * nc, c->dV, -obj / Lsum * kFourPi, (int)nc);
         if (objective) *objective = obj;
         if (history) std::memcpy(history, hh.data(), hh.size() * sizeof(double));
-        if (grad_state)
-            hipchk(c, hipMemcpyAsync(grad_state, lam, B3 * sizeof(double), hipMemcpyDeviceToHost, st), "grad");
-        if (grad_cell)
-            hipchk(c, hipMemcpyAsync(grad_cell, gcell, 5 * nc * sizeof(double), hipMemcpyDeviceToHost, st), "grad");
-        if (grad_bin)
-            hipchk(c, hipMemcpyAsync(grad_bin, gbin, 3 * n3 * sizeof(double), hipMemcpyDeviceToHost, st), "grad");
+        if (grad_state) download(c, grad_state, lam, B3, "grad");
+        if (grad_cell) download(c, grad_cell, gcell, 5 * nc, "grad");
+        if (grad_bin) download(c, grad_bin, gbin, 3 * n3, "grad");
         hipchk(c, hipStreamSynchronize(st), "sync");
         check_err_flag(c, "adjoint");
     });

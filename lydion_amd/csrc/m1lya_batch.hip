@@ -40,6 +40,7 @@
 #include "../../include/m1lya.h"
 #include "m1lya_fast.h"
 #include "m1lya_internal.h"
+#include "m1lya_transfer.h"
 
 // FP contraction is on only inside the FP32 advection (m1lya_fast.h and the cell update
 // below).  The FP64 emission, frequency factors, solve and reductions round as written:
@@ -1563,6 +1564,7 @@ struct m1lya_batch {
     };
     std::vector<Pending> pending;         // event pairs not yet read
     std::vector<hipEvent_t> event_pool;
+    m1t::Download down;
 };
 
 namespace {
@@ -2109,6 +2111,7 @@ void m1lya_batch_destroy(m1lya_batch* b)
         (void)hipEventDestroy(p.e1);
     }
     for (hipEvent_t e : b->event_pool) (void)hipEventDestroy(e);
+    b->down.release();
     for (void* p : b->allocs) (void)hipFree(p);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
@@ -2420,6 +2423,10 @@ int m1lya_batch_download(m1lya_batch* b, int cloud, int field, double* host, siz
             if (count != n) bfail(b, M1LYA_ERR_ARG, "field " + std::to_string(field) + ": wrong count");
         };
         auto down32 = [&](const float* src, size_t n, double scale) {
+            if (n * sizeof(double) >= m1t::kMinBytes) {
+                bchk(b, b->down.run(host, src, n, scale, b->device, b->stream), "download");
+                return;
+            }
             std::vector<float> h(n);
             bchk(b, hipMemcpy(h.data(), src, n * sizeof(float), hipMemcpyDeviceToHost), "download");
             for (size_t t = 0; t < n; ++t) host[t] = (double)h[t] * scale;
