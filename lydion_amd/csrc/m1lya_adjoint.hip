@@ -7,7 +7,7 @@
 // with its flux correction; the scalars are Update_f_Lyα_MF_L_Lyα!
 // (src/ConstantsAndFunctions.jl:588-674) and the escaping spectrum of
 // Compute_f_esc_Lyα_Cylindrical (:969-993).  Given the cotangent of X_{n+1},
-// three kernels produce the cotangent of X_n and accumulate those of the
+// the kernels below produce the cotangent of X_n and accumulate those of the
 // coefficient fields:
 //
 //   k_adj_column    one wavefront per cell, lanes over bins: E and C in
@@ -20,7 +20,10 @@
 //                   reverse (floors, causality limit, aberration, D:∇u and
 //                   K_ϕϕ terms); writes the cotangent of each cell's
 //                   flux-divergence sums and the cell's local cotangent.
-//   k_adj_gather    one thread per (bin, cell): adds, over the eight
+//   k_adj_march,    the interfaces in reverse mode, one direction at a time (below).
+//   k_adj_tile
+//   k_adj_gather    the same by dual numbers (mode 1, the reference of the tests):
+//                   one thread per (bin, cell): adds, over the eight
 //                   interfaces whose stencil holds the cell, the derivative of
 //                   the interface outputs along the cell's J, H_r, H_Z and α_F
 //                   contracted with the interface cotangents (which come from
@@ -328,164 +331,305 @@ __global__ __launch_bounds__(256, 2) void k_adj_gather(AdjAdvArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// Interface contributions through reverse-mode interfaces.  k_adj_face: thread per
-// (bin, interface); the interface cotangents come from the two cells it separates,
-// m1a::face_vjp turns them into cotangents of the interface's 14 inputs (J, H_r, H_Z
-// of its four stencil slots, α_F on its two sides), stored as planes of fpart.
-// k_adj_gather_rev: thread per (bin, cell); sums, over the <= 8 interfaces whose
-// stencil holds the cell, the slots that read it, through the ghost map of each
-// boundary (mirror: -1 on the normal flux; outflow clip: 0 or 1), and the α_F sides
-// that are the cell.  Same contributions as k_adj_gather's dual-number passes, in a
-// fixed order, without atomics.
+// Interface contributions through reverse-mode interfaces.  A wavefront, lanes over bins, marches
+// over the interfaces of a segment of a row (DIR 0) or a column (DIR 1).  The cotangents of an
+// interface's outputs come from the two cells it separates; m1a::face_vjp turns them into those of
+// its inputs (J, H_r, H_Z of its four stencil slots, α_F on its two sides), which are added to the
+// cells that the slots read, through the ghost map of each boundary (mirror: -1 on the normal flux;
+// outflow clip: 0 or 1).  The four cells of the stencil move along in registers, their sums in LDS
+// (no lane reads another's): a cell is loaded and its ratios H/J are formed once per direction, and its sums are
+// written once, when the last interface that reads it has passed.  Same contributions as
+// k_adj_gather's dual-number passes, in a fixed order that does not depend on the segments, without
+// atomics.  DIR 0 leaves its sums in fpart (four planes), DIR 1 continues them and adds the result
+// to the cotangent of the state.  Bound by the instructions of face_vjp at two wavefronts per SIMD;
+// the loads of an interface are issued one interface ahead.  128x128x128, us per step: 117 + 119,
+// against 168 + 141 + 152 for a thread per interface that left its 14 input cotangents in memory for
+// a gather per cell (1 GB of traffic).
 // ---------------------------------------------------------------------------
 namespace {
-
-struct FacePlanes {
-    size_t base, plane;   // plane p of interface index q at fpart[base + p * plane + q * nn + k]
-};
-
-__device__ __forceinline__ FacePlanes face_planes(int dir, int nn, int nr, int nz)
-{
-    const size_t nfr = (size_t)nz * (nr + 1) * nn, nfz = (size_t)nr * (nz + 1) * nn;
-    return dir == 0 ? FacePlanes{0, nfr} : FacePlanes{14 * nfr, nfz};
-}
 
 // Ghost map of stencil cell c along one direction (as tload_r / tload_z): the source
 // cell, and in fac the derivative of the slot's normal flux component (H_r along r,
 // H_Z along Z) with respect to the source's; J and the other component map with 1.
-// vnorm: the source's normal component, which decides the outflow clips.
-__device__ __forceinline__ int ghost_src(int c, int n, int dir, int low_reflect, int high_reflect, double vnorm,
+// vnorm(cell): the cell's normal component, which decides the outflow clips.
+template <class Vnorm>
+__device__ __forceinline__ int ghost_src(int c, int n, int dir, int low_reflect, int high_reflect, Vnorm vnorm,
                                          double& fac)
 {
     fac = 1.0;
     if (c < 0) {
         if (dir == 0 || low_reflect) { fac = -1.0; return -c - 1; }
-        fac = (0.0 < vnorm) ? 0.0 : 1.0;   // min(H_Z, 0) at an open bottom
+        fac = (0.0 < vnorm(0)) ? 0.0 : 1.0;   // min(H_Z, 0) at an open bottom
         return 0;
     }
     if (c < n) return c;
     if (high_reflect) { fac = -1.0; return 2 * n - 1 - c; }
-    fac = (0.0 > vnorm) ? 0.0 : 1.0;       // max(H, 0) at an open outer / top boundary
+    fac = (0.0 > vnorm(n - 1)) ? 0.0 : 1.0;   // max(H, 0) at an open outer / top boundary
     return n - 1;
+}
+
+// 1 / max(J, Jeps) and the ratios H / J of a stencil cell
+__device__ __forceinline__ void face_ratios(double J, double Hr, double Hz, double& iJ, double& fr, double& fz)
+{
+    const double Jm = m1a::facevjp::pass_max(J, kJeps) ? J : kJeps;
+    iJ = recip(Jm);
+    if (__builtin_expect(!(Jm < 0x1p500), 0)) iJ = 1.0 / Jm;
+    fr = Hr * iJ;
+    fz = Hz * iJ;
 }
 
 }  // namespace
 
-template <int DIR>
-__global__ __launch_bounds__(256, 2) void k_adj_face(AdjAdvArgs a)
+template <int DIR, bool HLL>
+__global__ __launch_bounds__(256, 2) void k_adj_march(AdjAdvArgs a, int seg)
 {
+    __shared__ double sums[4][4][4][64];
     const int nn = a.nn, nr = a.g.nr, nz = a.g.nz;
+    const int n = DIR == 0 ? nr : nz, lines = DIR == 0 ? nz : nr;
     const int k = blockIdx.x * 64 + threadIdx.x;
-    // DIR 0: interface f = 0..N_r of row j; DIR 1: interface f = 0..N_Z of column i
-    const int f = DIR == 0 ? (int)(blockIdx.y * 4 + threadIdx.y) : (int)blockIdx.z;
-    const int i = DIR == 0 ? 0 : (int)(blockIdx.y * 4 + threadIdx.y);
-    const int j = DIR == 0 ? (int)blockIdx.z : 0;
-    const int nf = DIR == 0 ? nr : nz;
-    if (k >= nn || f > nf || (DIR == 1 && i >= nr)) return;
+    const int line = __builtin_amdgcn_readfirstlane(blockIdx.y * 4 + threadIdx.y);
+    const int c0 = blockIdx.z * seg, c1 = min(n, c0 + seg);
+    if (k >= nn || line >= lines) return;
     if (k < a.krange[0] || k > a.krange[1]) return;
     const double cdt = a.cdt;
-    double lF[3] = {0.0, 0.0, 0.0}, lkL = 0.0, lkR = 0.0;
-    if (f >= 1) {
-        const int cl = DIR == 0 ? j * nr + (f - 1) : (f - 1) * nr + i;
-        const double A = DIR == 0 ? a.g.A_r[(size_t)j * (nr + 1) + f] : a.g.A_z[(size_t)f * nr + i];
-        const double s = -cdt * a.g.inv_dV[cl] * A;
-        const size_t q = (size_t)cl * nn + k;
-        lF[0] += s * a.pJ[q]; lF[1] += s * a.pHr[q]; lF[2] += s * a.pHz[q];
-        if (DIR == 0) lkL = 0.5 * cdt * a.g.inv_r_cell[f - 1] * a.pHr[q];
-    }
-    if (f <= nf - 1) {
-        const int cr = DIR == 0 ? j * nr + f : f * nr + i;
-        const double A = DIR == 0 ? a.g.A_r[(size_t)j * (nr + 1) + f] : a.g.A_z[(size_t)f * nr + i];
-        const double s = cdt * a.g.inv_dV[cr] * A;
-        const size_t q = (size_t)cr * nn + k;
-        lF[0] += s * a.pJ[q]; lF[1] += s * a.pHr[q]; lF[2] += s * a.pHz[q];
-        if (DIR == 0) lkR = 0.5 * cdt * a.g.inv_r_cell[f] * a.pHr[q];
-    }
-    const FacePlanes P = face_planes(DIR, nn, nr, nz);
-    const size_t q0 = P.base + (size_t)(DIR == 0 ? j * (nr + 1) + f : f * nr + i) * nn + k;
-    m1a::FaceGrad g;
-    if (lF[0] == 0.0 && lF[1] == 0.0 && lF[2] == 0.0 && lkL == 0.0 && lkR == 0.0) {
+    const size_t n3 = (size_t)nr * nz * nn;
+    const int low_reflect = DIR == 0 ? 1 : (a.bc_z_bot == BC_REFLECT);
+    const int high_reflect = DIR == 0 ? (a.bc_r_right == BC_REFLECT) : (a.bc_z_top == BC_REFLECT);
+    auto cell = [&](int c) { return DIR == 0 ? line * nr + c : c * nr + line; };
+    auto at = [&](int c) { return (size_t)cell(c) * nn + k; };
+    auto vnorm = [&](int c) { return DIR == 0 ? a.Hr[at(c)] : a.Hz[at(c)]; };
+
+    // cells f-2 .. f+1 of interface f, ghosts included: the state and the ratios; their sums are
+    // in the lane's part of sums, slot cell mod 4
+    double J[4], iJ[4], fr[4], fz[4];
+    auto sum = [&](int c) { return &sums[threadIdx.y][c & 3][0][threadIdx.x]; };
+    // a cell on its way into the stencil, and its sums so far if it is one of the segment's
+    struct Ahead {
+        double J, Hr, Hz, sum[4];
+    };
+    auto load = [&](int c) {
+        Ahead x;
+        if (DIR == 0) tload_r<double>(a.J, a.Hr, a.Hz, nn, nr, line, k, c, a.bc_r_right, -1, -1, x.J, x.Hr, x.Hz);
+        else tload_z<double>(a.J, a.Hr, a.Hz, nn, nr, nz, line, k, c, a.bc_z_bot, a.bc_z_top, -1, -1, x.J, x.Hr, x.Hz);
 #pragma unroll
-        for (int m = 0; m < 4; ++m) { g.J[m] = 0.0; g.Hr[m] = 0.0; g.Hz[m] = 0.0; }
-        g.aF_L = 0.0; g.aF_R = 0.0;
-    } else {
-        double J[4], Hr[4], Hz[4];
-        const int cells[4] = {f - 1, f, f + 1, f - 2};
-        double aFL, aFR, u;
-        const double* iv;
-        if (DIR == 0) {
+        for (int m = 0; m < 4; ++m)
+            x.sum[m] = (DIR == 1 && c >= c0 && c < c1) ? a.fpart[(size_t)m * n3 + at(c)] : 0.0;
+        return x;
+    };
+    auto enter = [&](const Ahead& x, int c, int w) {
+        J[w] = x.J;
+        face_ratios(x.J, x.Hr, x.Hz, iJ[w], fr[w], fz[w]);
+        double* o = sum(c);
 #pragma unroll
-            for (int m = 0; m < 4; ++m)
-                tload_r<double>(a.J, a.Hr, a.Hz, nn, nr, j, k, cells[m], a.bc_r_right, -1, -1, J[m], Hr[m], Hz[m]);
-            iv = a.g.ivr + (size_t)f * 5;
-            aFL = a.aF[((size_t)j * nr + max(f - 1, 0)) * nn + k];
-            aFR = a.aF[((size_t)j * nr + min(f, nr - 1)) * nn + k];
-            u = a.v.ur_star[(size_t)j * (nr + 1) + f] * kInvC;
-        } else {
+        for (int m = 0; m < 4; ++m) o[64 * m] = x.sum[m];
+    };
+    const int f0 = max(c0 - 1, 0), f1 = min(c1 + 1, n);
 #pragma unroll
-            for (int m = 0; m < 4; ++m)
-                tload_z<double>(a.J, a.Hr, a.Hz, nn, nr, nz, i, k, cells[m], a.bc_z_bot, a.bc_z_top, -1, -1, J[m],
-                                Hr[m], Hz[m]);
-            iv = a.g.ivz + (size_t)f * 5;
-            aFL = a.aF[((size_t)max(f - 1, 0) * nr + i) * nn + k];
-            aFR = a.aF[((size_t)min(f, nz - 1) * nr + i) * nn + k];
-            u = a.v.uz_star[(size_t)f * nr + i] * kInvC;
+    for (int w = 1; w < 4; ++w) enter(load(f0 - 3 + w), f0 - 3 + w, w);
+    // the loads of interface f + 1 are issued before f is worked on
+    Ahead next = load(f0 + 1);
+    double aFL = a.aF[at(max(f0 - 1, 0))], aFR = a.aF[at(f0)];
+    double pJ = 0.0, pHr = 0.0, pHz = 0.0;   // cotangents of the flux divergence of cell f-1
+    if (f0 >= 1) { pJ = a.pJ[at(f0 - 1)]; pHr = a.pHr[at(f0 - 1)]; pHz = a.pHz[at(f0 - 1)]; }
+    double nJ = a.pJ[at(f0)], nHr = a.pHr[at(f0)], nHz = a.pHz[at(f0)];   // of cell f
+#pragma unroll 1
+    for (int f = f0; f <= c1 + 1; ++f) {
+#pragma unroll
+        for (int w = 0; w < 3; ++w) {
+            J[w] = J[w + 1]; iJ[w] = iJ[w + 1]; fr[w] = fr[w + 1]; fz[w] = fz[w + 1];
         }
-        g = m1a::face_vjp(DIR, a.hll, DIR == 0 && f == 0, J, Hr, Hz, iv, aFL, aFR, u, lF[0], lF[1], lF[2], lkL, lkR);
-    }
+        double old[4] = {0.0, 0.0, 0.0, 0.0};
+        if (DIR == 1 && f - 2 >= c0) {
+            const size_t q = at(f - 2);
+            old[0] = a.oJ[q]; old[1] = a.oHr[q]; old[2] = a.oHz[q]; old[3] = a.gaF[q];
+        }
+        if (f <= n) {
+            enter(next, f + 1, 3);
+            const int fn = min(f + 1, f1);
+            next = load(fn + 1);
+            const size_t qn = at(min(fn, n - 1));
+            const double aFn = a.aF[qn], mJ = a.pJ[qn], mHr = a.pHr[qn], mHz = a.pHz[qn];
+            double lF[3] = {0.0, 0.0, 0.0}, lkL = 0.0, lkR = 0.0;
+            const double A = DIR == 0 ? a.g.A_r[(size_t)line * (nr + 1) + f] : a.g.A_z[(size_t)f * nr + line];
+            if (f >= 1) {
+                const double s = -cdt * a.g.inv_dV[cell(f - 1)] * A;
+                lF[0] += s * pJ; lF[1] += s * pHr; lF[2] += s * pHz;
+                if (DIR == 0) lkL = 0.5 * cdt * a.g.inv_r_cell[f - 1] * pHr;
+            }
+            if (f <= n - 1) {
+                pJ = nJ; pHr = nHr; pHz = nHz;
+                const double s = cdt * a.g.inv_dV[cell(f)] * A;
+                lF[0] += s * pJ; lF[1] += s * pHr; lF[2] += s * pHz;
+                if (DIR == 0) lkR = 0.5 * cdt * a.g.inv_r_cell[f] * pHr;
+            }
+            nJ = mJ; nHr = mHr; nHz = mHz;
+            if (!(lF[0] == 0.0 && lF[1] == 0.0 && lF[2] == 0.0 && lkL == 0.0 && lkR == 0.0)) {
+                const double u = (DIR == 0 ? a.v.ur_star[(size_t)line * (nr + 1) + f]
+                                           : a.v.uz_star[(size_t)f * nr + line]) * kInvC;
+                // slots in the reference's order: cells f-1, f, f+1, f-2
+                const double sJ[4] = {J[1], J[2], J[3], J[0]}, si[4] = {iJ[1], iJ[2], iJ[3], iJ[0]};
+                const double sr[4] = {fr[1], fr[2], fr[3], fr[0]}, sz[4] = {fz[1], fz[2], fz[3], fz[0]};
+                const m1a::FaceGrad g =
+                    m1a::face_vjp(DIR, HLL, DIR == 0 && f == 0, sJ, si, sr, sz,
+                                  (DIR == 0 ? a.g.ivr : a.g.ivz) + (size_t)f * 5, aFL, aFR, u, lF[0], lF[1], lF[2],
+                                  lkL, lkR);
+                if (f >= 2 && f + 1 < n) {
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        a.fpart[q0 + (size_t)(3 * m) * P.plane] = g.J[m];
-        a.fpart[q0 + (size_t)(3 * m + 1) * P.plane] = g.Hr[m];
-        a.fpart[q0 + (size_t)(3 * m + 2) * P.plane] = g.Hz[m];
+                    for (int m = 0; m < 4; ++m) {
+                        double* o = sum(m == 3 ? f - 2 : f - 1 + m);
+                        o[0] += g.J[m];
+                        o[64] += g.Hr[m];
+                        o[128] += g.Hz[m];
+                    }
+                    sum(f - 1)[192] += g.aF_L;
+                    sum(f)[192] += g.aF_R;
+                } else {
+                    const int cells[4] = {f - 1, f, f + 1, f - 2};
+#pragma unroll
+                    for (int m = 0; m < 4; ++m) {
+                        double fac;
+                        const int src = ghost_src(cells[m], n, DIR, low_reflect, high_reflect, vnorm, fac);
+                        double* o = sum(src);
+                        o[0] += g.J[m];
+                        o[64] += DIR == 0 ? fac * g.Hr[m] : g.Hr[m];
+                        o[128] += DIR == 0 ? g.Hz[m] : fac * g.Hz[m];
+                    }
+                    sum(max(f - 1, 0))[192] += g.aF_L;
+                    sum(min(f, n - 1))[192] += g.aF_R;
+                }
+            }
+            aFL = aFR;
+            aFR = aFn;
+        }
+        if (f - 2 >= c0) {
+            const size_t q = at(f - 2);
+            const double* o = sum(f - 2);
+            if (DIR == 0) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) a.fpart[(size_t)m * n3 + q] = o[64 * m];
+            } else {
+                a.oJ[q] = old[0] + o[0];
+                a.oHr[q] = old[1] + o[64];
+                a.oHz[q] = old[2] + o[128];
+                a.gaF[q] = old[3] + o[192];
+            }
+        }
     }
-    a.fpart[q0 + (size_t)12 * P.plane] = g.aF_L;
-    a.fpart[q0 + (size_t)13 * P.plane] = g.aF_R;
 }
 
-__global__ __launch_bounds__(256) void k_adj_gather_rev(AdjAdvArgs a)
+// The same sums for grids too small to march over: a block of eight wavefronts takes the
+// kTileFaces interfaces around kTileFaces - 3 cells of a line, two interfaces a wavefront, and the
+// cells gather their slots from LDS in the order of the march (the results have the same bits).
+// 45x61x64, both directions: 40 us, 58 by marches, 49 by way of memory.
+constexpr int kTileFaces = 16, kTileWaves = 8;
+
+template <int DIR, bool HLL>
+__global__ __launch_bounds__(64 * kTileWaves, 2) void k_adj_tile(AdjAdvArgs a, int seg)
 {
+    __shared__ double part[kTileFaces][14][64];
     const int nn = a.nn, nr = a.g.nr, nz = a.g.nz;
+    const int n = DIR == 0 ? nr : nz;
     const int k = blockIdx.x * 64 + threadIdx.x;
-    const int i = blockIdx.y * 4 + threadIdx.y;
-    const int j = blockIdx.z;
-    if (k >= nn || i >= nr) return;
-    if (k < a.krange[0] || k > a.krange[1]) return;
-    const size_t idx = ((size_t)j * nr + i) * nn + k;
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    const int line = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int c0 = blockIdx.z * seg, c1 = min(n, c0 + seg);
+    const bool act = k < nn && k >= a.krange[0] && k <= a.krange[1];
+    const double cdt = a.cdt;
+    const size_t n3 = (size_t)nr * nz * nn;
+    auto cell = [&](int c) { return DIR == 0 ? line * nr + c : c * nr + line; };
+    auto at = [&](int c) { return (size_t)cell(c) * nn + k; };
+    if (act) {
 #pragma unroll 1
-    for (int dir = 0; dir < 2; ++dir) {
-        const FacePlanes P = face_planes(dir, nn, nr, nz);
-        const int tc = dir == 0 ? i : j;
-        const int n = dir == 0 ? nr : nz;
-        const int low_reflect = dir == 0 ? 1 : (a.bc_z_bot == BC_REFLECT);
-        const int high_reflect = dir == 0 ? (a.bc_r_right == BC_REFLECT) : (a.bc_z_top == BC_REFLECT);
-        const double vnorm = dir == 0 ? a.Hr[idx] : a.Hz[idx];
+        for (int s = wave; s < kTileFaces; s += kTileWaves) {
+            const int f = c0 - 1 + s;
+            if (f < 0 || f > min(c1 + 1, n)) continue;
+            const double A = DIR == 0 ? a.g.A_r[(size_t)line * (nr + 1) + f] : a.g.A_z[(size_t)f * nr + line];
+            double lF[3] = {0.0, 0.0, 0.0}, lkL = 0.0, lkR = 0.0;
+            if (f >= 1) {
+                const double w = -cdt * a.g.inv_dV[cell(f - 1)] * A;
+                const size_t q = at(f - 1);
+                lF[0] += w * a.pJ[q]; lF[1] += w * a.pHr[q]; lF[2] += w * a.pHz[q];
+                if (DIR == 0) lkL = 0.5 * cdt * a.g.inv_r_cell[f - 1] * a.pHr[q];
+            }
+            if (f <= n - 1) {
+                const double w = cdt * a.g.inv_dV[cell(f)] * A;
+                const size_t q = at(f);
+                lF[0] += w * a.pJ[q]; lF[1] += w * a.pHr[q]; lF[2] += w * a.pHz[q];
+                if (DIR == 0) lkR = 0.5 * cdt * a.g.inv_r_cell[f] * a.pHr[q];
+            }
+            m1a::FaceGrad g;
+            if (lF[0] == 0.0 && lF[1] == 0.0 && lF[2] == 0.0 && lkL == 0.0 && lkR == 0.0) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) { g.J[m] = 0.0; g.Hr[m] = 0.0; g.Hz[m] = 0.0; }
+                g.aF_L = 0.0; g.aF_R = 0.0;
+            } else {
+                const int cells[4] = {f - 1, f, f + 1, f - 2};
+                double J[4], iJ[4], fr[4], fz[4];
+#pragma unroll
+                for (int m = 0; m < 4; ++m) {
+                    double vr, vz;
+                    if (DIR == 0)
+                        tload_r<double>(a.J, a.Hr, a.Hz, nn, nr, line, k, cells[m], a.bc_r_right, -1, -1, J[m], vr, vz);
+                    else
+                        tload_z<double>(a.J, a.Hr, a.Hz, nn, nr, nz, line, k, cells[m], a.bc_z_bot, a.bc_z_top, -1, -1,
+                                        J[m], vr, vz);
+                    face_ratios(J[m], vr, vz, iJ[m], fr[m], fz[m]);
+                }
+                const double aFL = a.aF[at(max(f - 1, 0))], aFR = a.aF[at(min(f, n - 1))];
+                const double u = (DIR == 0 ? a.v.ur_star[(size_t)line * (nr + 1) + f]
+                                           : a.v.uz_star[(size_t)f * nr + line]) * kInvC;
+                g = m1a::face_vjp(DIR, HLL, DIR == 0 && f == 0, J, iJ, fr, fz,
+                                  (DIR == 0 ? a.g.ivr : a.g.ivz) + (size_t)f * 5, aFL, aFR, u, lF[0], lF[1], lF[2],
+                                  lkL, lkR);
+            }
+            double* o = &part[s][0][threadIdx.x];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                o[64 * (3 * m)] = g.J[m];
+                o[64 * (3 * m + 1)] = g.Hr[m];
+                o[64 * (3 * m + 2)] = g.Hz[m];
+            }
+            o[64 * 12] = g.aF_L;
+            o[64 * 13] = g.aF_R;
+        }
+    }
+    __syncthreads();
+    if (!act) return;
+    const int low_reflect = DIR == 0 ? 1 : (a.bc_z_bot == BC_REFLECT);
+    const int high_reflect = DIR == 0 ? (a.bc_r_right == BC_REFLECT) : (a.bc_z_top == BC_REFLECT);
+    auto vnorm = [&](int c) { return DIR == 0 ? a.Hr[at(c)] : a.Hz[at(c)]; };
 #pragma unroll 1
-        for (int t = 0; t < 4; ++t) {
-            const int f = tc - 1 + t;
-            if (f < 0 || f > n) continue;
-            const size_t q0 = P.base + (size_t)(dir == 0 ? j * (nr + 1) + f : f * nr + i) * nn + k;
+    for (int c = c0 + wave; c < c1; c += kTileWaves) {
+        const size_t q = at(c);
+        double acc[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc[m] = DIR == 1 ? a.fpart[(size_t)m * n3 + q] : 0.0;
+#pragma unroll 1
+        for (int f = max(c - 1, 0); f <= min(c + 2, n); ++f) {
+            const double* o = &part[f - (c0 - 1)][0][threadIdx.x];
             const int cells[4] = {f - 1, f, f + 1, f - 2};
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 double fac;
-                const int src = ghost_src(cells[m], n, dir, low_reflect, high_reflect, vnorm, fac);
-                if (src != tc) continue;
-                acc[0] += a.fpart[q0 + (size_t)(3 * m) * P.plane];
-                const double gr = a.fpart[q0 + (size_t)(3 * m + 1) * P.plane];
-                const double gz = a.fpart[q0 + (size_t)(3 * m + 2) * P.plane];
-                if (dir == 0) { acc[1] += fac * gr; acc[2] += gz; }
-                else { acc[1] += gr; acc[2] += fac * gz; }
+                if (ghost_src(cells[m], n, DIR, low_reflect, high_reflect, vnorm, fac) != c) continue;
+                const double gr = o[64 * (3 * m + 1)], gz = o[64 * (3 * m + 2)];
+                acc[0] += o[64 * (3 * m)];
+                acc[1] += DIR == 0 ? fac * gr : gr;
+                acc[2] += DIR == 0 ? gz : fac * gz;
             }
-            if (max(f - 1, 0) == tc) acc[3] += a.fpart[q0 + (size_t)12 * P.plane];
-            if (min(f, n - 1) == tc) acc[3] += a.fpart[q0 + (size_t)13 * P.plane];
+            if (max(f - 1, 0) == c) acc[3] += o[64 * 12];
+            if (min(f, n - 1) == c) acc[3] += o[64 * 13];
+        }
+        if (DIR == 0) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) a.fpart[(size_t)m * n3 + q] = acc[m];
+        } else {
+            a.oJ[q] += acc[0];
+            a.oHr[q] += acc[1];
+            a.oHz[q] += acc[2];
+            a.gaF[q] += acc[3];
         }
     }
-    a.oJ[idx] += acc[0];
-    a.oHr[idx] += acc[1];
-    a.oHz[idx] += acc[2];
-    a.gaF[idx] += acc[3];
 }
 
 // ---------------------------------------------------------------------------
@@ -871,6 +1015,38 @@ void launch_adj_column(hipStream_t s, const AdjColArgs& a)
     hipLaunchKernelGGL(k_adj_column, dim3(ncell), dim3(64), lds, s, a);
 }
 
+// The interfaces of one direction.  In units of one interface by a wavefront that has its SIMD to
+// itself (4.3 us; two at a time take 1.28), a march takes its segment's cells, three interfaces more
+// and about one to start, on the wavefronts a SIMD gets (256 VGPRs allow two at a time); a block of
+// k_adj_tile takes two pairs of interfaces and 0.8 for its sums, one block to a CU, and the launch one
+// to start.  The least estimated time: on 128x128x128 the march by 16 cells (r: estimated 110 us,
+// measured 117; tiles 150), on 45x61x64 the tiles (19 us, 19; the march 28).
+template <int DIR>
+static void launch_adj_faces(hipStream_t s, const AdjAdvArgs& a)
+{
+    constexpr int kCUs = 256, kSimds = 4 * kCUs, kSegMax = 32;
+    const int n = DIR == 0 ? a.g.nr : a.g.nz, lines = DIR == 0 ? a.g.nz : a.g.nr;
+    const int chunks = (a.nn + 63) / 64, groups = (lines + 3) / 4;
+    int seg = kSegMax;
+    double best = 0.0;
+    for (int t = kSegMax; t >= 1; --t) {
+        const long per_simd = ((long)chunks * groups * 4 * ((n + t - 1) / t) + kSimds - 1) / kSimds;
+        const double cost = (1.28 * (double)(per_simd / 2) + (double)(per_simd % 2)) * (t + 4);
+        if (t == kSegMax || cost < best) { best = cost; seg = t; }
+    }
+    const int tiles = (n + kTileFaces - 4) / (kTileFaces - 3), tile_seg = (n + tiles - 1) / tiles;
+    const long per_cu = ((long)chunks * lines * tiles + kCUs - 1) / kCUs;
+    if (3.36 * (double)per_cu + 1.0 < best) {
+        const dim3 grid(chunks, lines, tiles), block(64, kTileWaves);
+        if (a.hll) hipLaunchKernelGGL((k_adj_tile<DIR, true>), grid, block, 0, s, a, tile_seg);
+        else hipLaunchKernelGGL((k_adj_tile<DIR, false>), grid, block, 0, s, a, tile_seg);
+        return;
+    }
+    const dim3 grid(chunks, groups, (n + seg - 1) / seg), block(64, 4);
+    if (a.hll) hipLaunchKernelGGL((k_adj_march<DIR, true>), grid, block, 0, s, a, seg);
+    else hipLaunchKernelGGL((k_adj_march<DIR, false>), grid, block, 0, s, a, seg);
+}
+
 void launch_adj_advect(hipStream_t s, const AdjAdvArgs& a)
 {
     dim3 grid((a.nn + 63) / 64, (a.g.nr + 3) / 4, a.g.nz);
@@ -881,9 +1057,8 @@ void launch_adj_advect(hipStream_t s, const AdjAdvArgs& a)
         hipLaunchKernelGGL(k_adj_gather, grid, dim3(64, 4), 0, s, a);
         return;
     }
-    hipLaunchKernelGGL(k_adj_face<0>, dim3((a.nn + 63) / 64, (a.g.nr + 1 + 3) / 4, a.g.nz), dim3(64, 4), 0, s, a);
-    hipLaunchKernelGGL(k_adj_face<1>, dim3((a.nn + 63) / 64, (a.g.nr + 3) / 4, a.g.nz + 1), dim3(64, 4), 0, s, a);
-    hipLaunchKernelGGL(k_adj_gather_rev, grid, dim3(64, 4), 0, s, a);
+    launch_adj_faces<0>(s, a);
+    launch_adj_faces<1>(s, a);
 }
 
 void launch_adj_spectrum(hipStream_t s, const double* Hr, const double* Hz, const double* A_r, const double* A_z,

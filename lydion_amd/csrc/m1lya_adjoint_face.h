@@ -6,7 +6,8 @@
 // sides) it returns the cotangents of its inputs, the four stencil cells' J, H_r,
 // H_Z and the two α_F values.  At a kink (limiter, max/min, clamp) it takes the
 // derivative of the branch the value selects, as the dual-number evaluation does,
-// so the two agree to rounding.  Forward formulas: src/AdvectJandH.jl:81-118,
+// so the two agree to rounding.  Where a wavefront's divisors are away from the ends of the
+// exponent range, quotients over one divisor share its reciprocal (m1::quot, the IEEE quotient).  Forward formulas: src/AdvectJandH.jl:81-118,
 // 155-204, 276-282, 359-473, 499-522; src/M1Closure.jl:28-33, 91-119, 273-296.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -37,7 +38,7 @@ __device__ __forceinline__ double minmod_f(double A, double B, int& which)
 // Compute_D_Edd_from_f_n forward, with the intermediates its reverse needs
 struct EddF {
     bool on, pass_f;
-    double fc, SQ, den, chi, b, nr, nz;
+    double fc, SQ, den, rden, chi, b, nr, nz;
     double rr, zz, rz;
 };
 
@@ -47,17 +48,18 @@ __device__ __forceinline__ EddF edd_f_n(double f, double nr, double nz)
     e.on = f > kFmin;
     e.nr = nr; e.nz = nz;
     if (!e.on) {
-        e.pass_f = false; e.fc = 0.0; e.SQ = 0.0; e.den = 1.0; e.chi = 0.0; e.b = 0.0;
+        e.pass_f = false; e.fc = 0.0; e.SQ = 1.0; e.den = 1.0; e.rden = 1.0; e.chi = 0.0; e.b = 0.0;
         e.rr = kOneThird; e.zz = kOneThird; e.rz = 0.0;
         return e;
     }
     e.pass_f = !(kFmax < f);                 // tmin(f, kFmax)
     e.fc = e.pass_f ? f : kFmax;
     const double f2 = e.fc * e.fc;
-    e.SQ = sqrt(4.0 - 3.0 * f2);
+    e.SQ = m1::root(4.0 - 3.0 * f2);   // in [1, 2]
     const double num = 3.0 + 4.0 * f2;
     e.den = 5.0 + 2.0 * e.SQ;
-    e.chi = num / e.den;
+    e.rden = m1::rcp_nr(e.den);
+    e.chi = m1::quot(num, e.den, e.rden);
     const double a = (1.0 - e.chi) * 0.5;
     e.b = (3.0 * e.chi - 1.0) * 0.5;
     const double b_nr = e.b * nr;
@@ -77,10 +79,9 @@ __device__ __forceinline__ void edd_f_n_rev(const EddF& e, double lrr, double lz
     lnr += lrr * 2.0 * e.b * e.nr + lrz * e.b * e.nz;
     lnz += lzz * 2.0 * e.b * e.nz + lrz * e.b * e.nr;
     const double lchi = -0.5 * la + 1.5 * lb;
-    const double lnum = lchi / e.den;
-    const double lden = -lchi * e.chi / e.den;
-    const double lSQ = 2.0 * lden;
-    const double lt = e.SQ > 0.0 ? 0.5 * lSQ / e.SQ : 0.0;   // t = 4 - 3 f²
+    const double lnum = m1::quot(lchi, e.den, e.rden);
+    const double lden = m1::quot(-lchi * e.chi, e.den, e.rden);
+    const double lt = m1::quot(lden, e.SQ);                  // t = 4 - 3 f²
     const double lf2 = 4.0 * lnum - 3.0 * lt;
     if (e.pass_f) lf += 2.0 * e.fc * lf2;
 }
@@ -107,8 +108,8 @@ __device__ __forceinline__ EigF eig_f(double f0, double mu0)
     const double muf = e.mu * e.f;
     const double q = 4.0 - 3.0 * e.f2;
     e.pq = !(0.0 > q);
-    e.SQ = sqrt(e.pq ? q : 0.0);
-    e.inv_SQ = 1.0 / e.SQ;
+    e.SQ = m1::root(e.pq ? q : 0.0);   // f <= kFmax: the argument is above 1
+    e.inv_SQ = m1::recip(e.SQ);
     const double r = kTwoThirds * (4.0 - 3.0 * e.f2 - e.SQ) + 2.0 * e.mu2 * (2.0 - e.f2 - e.SQ);
     e.pr = !(0.0 > r);
     e.Q = e.pr ? r : 0.0;
@@ -136,7 +137,7 @@ __device__ __forceinline__ void eig_rev(const EigF& e, double ll1, double ll3, d
     double lf2 = lr * (-3.0 * kTwoThirds - 2.0 * e.mu2);
     const double lmu2 = lr * 2.0 * (2.0 - e.f2 - e.SQ);
     lSQ += lr * (-kTwoThirds - 2.0 * e.mu2);
-    const double lqv = e.SQ > 0.0 ? 0.5 * lSQ / e.SQ : 0.0;
+    const double lqv = m1::quot(0.5 * lSQ, e.SQ);
     const double lq = e.pq ? lqv : 0.0;
     lf2 += -3.0 * lq;
     const double lf = 2.0 * e.f * lf2 + lmuf * e.mu;
@@ -148,10 +149,12 @@ __device__ __forceinline__ void eig_rev(const EigF& e, double ll1, double ll3, d
 }  // namespace facevjp
 
 // One interface and its vector-Jacobian product.  lFJ, lFHr, lFHz: cotangents of the
-// three fluxes; lkL, lkR: of the two K_ϕϕ outputs (tface's kphi_L, kphi_R).
-__device__ inline FaceGrad face_vjp(int dir, int hll, bool axis, const double (&J)[4], const double (&Hr)[4],
-                                    const double (&Hz)[4], const double* iv, double aF_L, double aF_R,
-                                    double u_over_c, double lFJ, double lFHr, double lFHz, double lkL, double lkR)
+// three fluxes; lkL, lkR: of the two K_ϕϕ outputs (tface's kphi_L, kphi_R; used along r).  The
+// stencil cells come with iJ = 1 / max(J, Jeps), fr = H_r iJ and fz = H_Z iJ.
+__device__ __forceinline__ FaceGrad face_vjp(int dir, int hll, bool axis, const double (&J)[4],
+                                             const double (&iJ)[4], const double (&fr)[4], const double (&fz)[4],
+                                             const double* iv, double aF_L, double aF_R, double u_over_c, double lFJ,
+                                             double lFHr, double lFHz, double lkL, double lkR)
 {
     using namespace facevjp;
     FaceGrad g;
@@ -161,15 +164,6 @@ __device__ inline FaceGrad face_vjp(int dir, int hll, bool axis, const double (&
     // ================= forward (treconstruct) =================
     const double dL = iv[0], dR = iv[1], c01 = iv[2], c12 = iv[3], c23 = iv[4];
     const double tau_L = aF_L * dL, tau_R = aF_R * dR;
-    bool pJ[4];
-    double iJ[4], fr[4], fz[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-        pJ[m] = pass_max(J[m], kJeps);
-        iJ[m] = 1.0 / (pJ[m] ? J[m] : kJeps);
-        fr[m] = Hr[m] * iJ[m];
-        fz[m] = Hz[m] * iJ[m];
-    }
     const double dJc = (J[1] - J[0]) * c12;
     int wJL, wJR, wrL, wrR, wzL, wzR;
     const double dJL = minmod_f((J[0] - J[3]) * c01, dJc, wJL);
@@ -186,15 +180,30 @@ __device__ inline FaceGrad face_vjp(int dir, int hll, bool axis, const double (&
     const double J_L = pJL ? JL0 : kJeps, J_R = pJR ? JR0 : kJeps;
     const double frL0 = fr[0] + dfrL * dL, frR0 = fr[1] - dfrR * dR;
     const double fzL0 = fz[0] + dfzL * dL, fzR0 = fz[1] - dfzR * dR;
-    const double fL0 = sqrt(frL0 * frL0 + fzL0 * fzL0);
-    const double fR0 = sqrt(frR0 * frR0 + fzR0 * fzR0);
+    const double fL2 = frL0 * frL0 + fzL0 * fzL0, fR2 = frR0 * frR0 + fzR0 * fzR0;
+    const double tau = tau_L + tau_R;
+    auto mid = [](double x) { return x >= 0x1p-400 && x <= 0x1p400; };
+    const bool plain = !__any(!((mid(fL2) || fL2 == 0.0) && (mid(fR2) || fR2 == 0.0) && mid(tau)));
+    auto over = [&](double n, double d, double r) { return plain ? m1::quot(n, d, r) : n / d; };
+    double fL0, fR0, rfL, rfR;
+    if (plain) {
+        fL0 = fL2 > 0.0 ? m1::root(fL2) : 0.0;
+        fR0 = fR2 > 0.0 ? m1::root(fR2) : 0.0;
+        rfL = m1::recip(fL0);
+        rfR = m1::recip(fR0);
+    } else {
+        fL0 = sqrt(fL2);
+        fR0 = sqrt(fR2);
+        rfL = 1.0 / fL0;
+        rfR = 1.0 / fR0;
+    }
     const bool nL = fL0 > 1.0, nR = fR0 > 1.0;   // limited to |f| = 1
-    const double ifL0 = nL ? 1.0 / fL0 : 1.0, ifR0 = nR ? 1.0 / fR0 : 1.0;
+    const double ifL0 = nL ? rfL : 1.0, ifR0 = nR ? rfR : 1.0;
     const double frL = nL ? frL0 * ifL0 : frL0, fzL = nL ? fzL0 * ifL0 : fzL0;
     const double frR = nR ? frR0 * ifR0 : frR0, fzR = nR ? fzR0 * ifR0 : fzR0;
     const double f_L = nL ? 1.0 : fL0, f_R = nR ? 1.0 : fR0;
     const bool dnL = f_L > 0.0, dnR = f_R > 0.0;
-    const double invnL = dnL ? 1.0 / f_L : 0.0, invnR = dnR ? 1.0 / f_R : 0.0;
+    const double invnL = nL ? 1.0 : (dnL ? rfL : 0.0), invnR = nR ? 1.0 : (dnR ? rfR : 0.0);
     const double nr_L = dnL ? frL * invnL : 0.0, nz_L = dnL ? fzL * invnL : 0.0;
     const double nr_R = dnR ? frR * invnR : 0.0, nz_R = dnR ? fzR * invnR : 0.0;
     const double HrL = frL * J_L, HrR = frR * J_R, HzL = fzL * J_L, HzR = fzR * J_R;
@@ -211,13 +220,14 @@ __device__ inline FaceGrad face_vjp(int dir, int hll, bool axis, const double (&
         FHr_L = DL.rz * J_L; FHr_R = DR.rz * J_R;
         FHz_L = DL.zz * J_L; FHz_R = DR.zz * J_R;
     }
-    const double tau = tau_L + tau_R;
     const double num = 0.2 + tau;
     const double dnm = num + tau * tau;
-    const double eps = num / dnm;
+    const double rdnm = m1::rcp_nr(dnm);
+    const double eps = over(num, dnm, rdnm);
     const bool ptau = pass_max(tau, 1e-300);
     const double tau_eff = ptau ? tau : 1e-300;
-    const double FJd = -kOneThird * (J[1] - J[0]) / tau_eff;
+    const double rtau = m1::rcp_nr(tau_eff);
+    const double FJd = over(-kOneThird * (J[1] - J[0]), tau_eff, rtau);
 
     // ================= reverse =================
     // upwind term: F += u (up ? right : left)
@@ -242,7 +252,7 @@ __device__ inline FaceGrad face_vjp(int dir, int hll, bool axis, const double (&
         const double S_L = pSL ? m1 : 0.0;
         const double dS0 = S_R - S_L;
         const bool pdS = pass_max(dS0, 1e-300);
-        const double inv_dS = 1.0 / (pdS ? dS0 : 1e-300);
+        const double inv_dS = m1::recip(pdS ? dS0 : 1e-300);
         const double SRSL = S_R * S_L;
         const double NJ = S_R * FJ_L - S_L * FJ_R + SRSL * (J_R - J_L);
         const double NHr = S_R * FHr_L - S_L * FHr_R + SRSL * (HrR - HrL);
@@ -293,60 +303,59 @@ __device__ inline FaceGrad face_vjp(int dir, int hll, bool axis, const double (&
         leps += -0.5 * (lFHr * (HrR - HrL) + lFHz * (HzR - HzL));
     }
     // eps = num / (num + tau²), FJd = -(1/3)(J1 - J0)/tau_eff
-    const double lnum = leps / dnm - leps * eps / dnm;
-    const double ltau_q = -leps * eps / dnm * 2.0 * tau;
+    const double lepe = over(leps * eps, dnm, rdnm);
+    const double lnum = over(leps, dnm, rdnm) - lepe;
+    const double ltau_q = -lepe * 2.0 * tau;
     double ltau = lnum + ltau_q;
-    const double lJdiff = -kOneThird * lFJd / tau_eff;
+    const double lJdiff = over(-kOneThird * lFJd, tau_eff, rtau);
     g.J[1] += lJdiff;
     g.J[0] -= lJdiff;
-    if (ptau) ltau += -lFJd * FJd / tau_eff;
+    if (ptau) ltau += over(-lFJd * FJd, tau_eff, rtau);
     g.aF_L = ltau * dL;
     g.aF_R = ltau * dR;
 
-    // K_ϕϕ outputs
-    {
+    // K_ϕϕ outputs (r only): 1 - D_rr - D_ZZ times J, clamped.  (The closure's cotangents go back on
+    // their own here, not with those of the side fluxes: the gradient along α_F of thin cells is a
+    // difference of nearly equal terms, and another order of rounding shows in it at 1e-10.)
+    if (dir == 0) {
         const double xL = 1.0 - DL.rr - DL.zz;
+        lJ_L += lkL * clamp_f(xL, 0.0, 1.0);
         if (pass_clamp(xL, 0.0, 1.0)) {
-            lJ_L += lkL * xL;
             const double lx = lkL * J_L;
             edd_f_n_rev(DL, -lx, -lx, 0.0, lfL, lnrL, lnzL);
-        } else {
-            lJ_L += lkL * clamp_f(xL, 0.0, 1.0);
         }
-    }
-    if (axis) {
-        // Compute_K_ϕϕ_InnerAxis(J_R, HzR)
-        const bool pa = pass_max(J_R, kJeps);
-        const double Ja = pa ? J_R : kJeps;
-        const double fz0 = HzR / Ja;
-        const bool pfz = pass_clamp(fz0, -1.0, 1.0);
-        const double fzc = clamp_f(fz0, -1.0, 1.0);
-        const double f = fzc < 0.0 ? -fzc : fzc;
-        double nzc = 0.0;
-        if (f > 0.0) nzc = (fzc > 0.0) ? 1.0 : ((fzc < 0.0) ? -1.0 : fzc);
-        const EddF DA = edd_f_n(f, 0.0, nzc);
-        const double x = 1.0 - DA.rr - DA.zz;
-        double lJa = 0.0, lf = 0.0, lnr_d = 0.0, lnz_d = 0.0;
-        if (pass_clamp(x, 0.0, 1.0)) {
-            lJa += lkR * x;
-            const double lx = lkR * Ja;
-            edd_f_n_rev(DA, -lx, -lx, 0.0, lf, lnr_d, lnz_d);
+        if (axis) {
+            // Compute_K_ϕϕ_InnerAxis(J_R, HzR)
+            const bool pa = pass_max(J_R, kJeps);
+            const double Ja = pa ? J_R : kJeps;
+            const double fz0 = HzR / Ja;
+            const bool pfz = pass_clamp(fz0, -1.0, 1.0);
+            const double fzc = clamp_f(fz0, -1.0, 1.0);
+            const double f = fzc < 0.0 ? -fzc : fzc;
+            double nzc = 0.0;
+            if (f > 0.0) nzc = (fzc > 0.0) ? 1.0 : ((fzc < 0.0) ? -1.0 : fzc);
+            const EddF DA = edd_f_n(f, 0.0, nzc);
+            const double x = 1.0 - DA.rr - DA.zz;
+            double lJa = 0.0, lf = 0.0, lnr_d = 0.0, lnz_d = 0.0;
+            if (pass_clamp(x, 0.0, 1.0)) {
+                lJa += lkR * x;
+                const double lx = lkR * Ja;
+                edd_f_n_rev(DA, -lx, -lx, 0.0, lf, lnr_d, lnz_d);
+            } else {
+                lJa += lkR * clamp_f(x, 0.0, 1.0);
+            }
+            const double lfzc = fzc < 0.0 ? -lf : lf;
+            const double lfz0 = pfz ? lfzc : 0.0;
+            lHzR += lfz0 / Ja;
+            lJa += -lfz0 * fz0 / Ja;
+            if (pa) lJ_R += lJa;
         } else {
-            lJa += lkR * clamp_f(x, 0.0, 1.0);
-        }
-        const double lfzc = fzc < 0.0 ? -lf : lf;
-        const double lfz0 = pfz ? lfzc : 0.0;
-        lHzR += lfz0 / Ja;
-        lJa += -lfz0 * fz0 / Ja;
-        if (pa) lJ_R += lJa;
-    } else {
-        const double xR = 1.0 - DR.rr - DR.zz;
-        if (pass_clamp(xR, 0.0, 1.0)) {
-            lJ_R += lkR * xR;
-            const double lx = lkR * J_R;
-            edd_f_n_rev(DR, -lx, -lx, 0.0, lfR, lnrR, lnzR);
-        } else {
+            const double xR = 1.0 - DR.rr - DR.zz;
             lJ_R += lkR * clamp_f(xR, 0.0, 1.0);
+            if (pass_clamp(xR, 0.0, 1.0)) {
+                const double lx = lkR * J_R;
+                edd_f_n_rev(DR, -lx, -lx, 0.0, lfR, lnrR, lnzR);
+            }
         }
     }
 
@@ -399,8 +408,8 @@ __device__ inline FaceGrad face_vjp(int dir, int hll, bool axis, const double (&
         lfrR0 = lfrR; lfzR0 = lfzR; lfR0 = lfR;
     }
     // f0 = sqrt(fr0² + fz0²)
-    if (fL0 > 0.0) { lfrL0 += lfL0 * frL0 / fL0; lfzL0 += lfL0 * fzL0 / fL0; }
-    if (fR0 > 0.0) { lfrR0 += lfR0 * frR0 / fR0; lfzR0 += lfR0 * fzR0 / fR0; }
+    if (fL0 > 0.0) { lfrL0 += over(lfL0 * frL0, fL0, rfL); lfzL0 += over(lfL0 * fzL0, fL0, rfL); }
+    if (fR0 > 0.0) { lfrR0 += over(lfR0 * frR0, fR0, rfR); lfzR0 += over(lfR0 * fzR0, fR0, rfR); }
     // J_L = max(J0 + dJL dL, Jeps), J_R = max(J1 - dJR dR, Jeps)
     const double lJL0 = pJL ? lJ_L : 0.0, lJR0 = pJR ? lJ_R : 0.0;
     g.J[0] += lJL0;
@@ -432,7 +441,7 @@ __device__ inline FaceGrad face_vjp(int dir, int hll, bool axis, const double (&
     for (int m = 0; m < 4; ++m) {
         g.Hr[m] += lfr[m] * iJ[m];
         g.Hz[m] += lfz[m] * iJ[m];
-        if (pJ[m]) g.J[m] += -(lfr[m] * fr[m] + lfz[m] * fz[m]) * iJ[m];
+        if (pass_max(J[m], kJeps)) g.J[m] += -(lfr[m] * fr[m] + lfz[m] * fz[m]) * iJ[m];
     }
     return g;
 }

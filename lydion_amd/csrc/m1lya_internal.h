@@ -164,15 +164,12 @@ struct AdjAdvArgs {
     double cdt;
     int bc_r_right, bc_z_bot, bc_z_top, hll;
     const int* krange;
-    double* fpart;        // reverse-mode interfaces: 14 planes of per-face input cotangents
+    double* fpart;        // reverse-mode interfaces: the r direction's sums per cell, four planes
     int mode;             // 0 interfaces in reverse mode; 1 dual-number passes per cell
 };
 
 // doubles of AdjAdvArgs::fpart for an N_r x N_Z x N_ν grid
-inline size_t adj_face_part_size(int nn, int nr, int nz)
-{
-    return (size_t)14 * ((size_t)nz * (nr + 1) + (size_t)nr * (nz + 1)) * nn;
-}
+inline size_t adj_face_part_size(int nn, int nr, int nz) { return (size_t)4 * nr * nz * nn; }
 
 struct AdjColArgs {
     int nn, nr, nz, recoil;
