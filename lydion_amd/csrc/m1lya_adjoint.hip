@@ -156,13 +156,40 @@ __device__ m1a::FaceT<T> face_at(const AdjAdvArgs& a, int dir, int f, int i, int
     return m1a::tface<T>(dir, a.hll, dir == 0 && f == 0, st, iv, aFL, aFR, u);
 }
 
+// Values of interface f of row j (r, dir 0) or column i (Z, dir 1) at bin k: the forward sweep's
+// arithmetic, kphi_R at the axis being that of cell 0.
+template <int DIR>
+__device__ __forceinline__ FaceResult face_values(const AdjAdvArgs& a, int f, int i, int j, int k)
+{
+    const int nn = a.nn, nr = a.g.nr, nz = a.g.nz;
+    Stencil st;
+    const int cells[4] = {f - 1, f, f + 1, f - 2};
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        double vr, vz;
+        if (DIR == 0) tload_r<double>(a.J, a.Hr, a.Hz, nn, nr, j, k, cells[m], a.bc_r_right, -1, -1, st.J[m], vr, vz);
+        else tload_z<double>(a.J, a.Hr, a.Hz, nn, nr, nz, i, k, cells[m], a.bc_z_bot, a.bc_z_top, -1, -1, st.J[m], vr, vz);
+        flux_ratios(st.J[m], vr, vz, st.fr[m], st.fz[m]);
+    }
+    const int n = DIR == 0 ? nr : nz, cl = max(f - 1, 0), cr = min(f, n - 1);
+    const double aFL = a.aF[(DIR == 0 ? (size_t)j * nr + cl : (size_t)cl * nr + i) * nn + k];
+    const double aFR = a.aF[(DIR == 0 ? (size_t)j * nr + cr : (size_t)cr * nr + i) * nn + k];
+    const double u = (DIR == 0 ? a.v.ur_star[(size_t)j * (nr + 1) + f] : a.v.uz_star[(size_t)f * nr + i]) * kInvC;
+    FaceResult r = interface_flux(DIR, a.hll, st, (DIR == 0 ? a.g.ivr : a.g.ivz) + (size_t)f * 5, aFL, aFR, u);
+    if (DIR == 0 && f == 0) r.kphi_R = kphi_inner_axis(r.J_R, r.Hz_R);
+    return r;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
 // Cell update of AdvectJandH_Cylindrical! (src/AdvectJandH.jl:1302-1382) in reverse.
 // ---------------------------------------------------------------------------
 // Block of 64 bins x BI x BJ cells, a wavefront per cell; the forward values of each interface
-// are evaluated once per block and reach the two cells that share it through LDS.
+// are evaluated once per block and reach the two cells that share it through LDS.  Bound by FP64
+// instructions, 2.75 interfaces per cell among them: with the forward sweep's divisions and the
+// interfaces dealt out three to a wavefront (two to four when each cell took its own) 156 us on
+// 128x128x128, was 171.
 template <int BI, int BJ>
 __global__ __launch_bounds__(64 * BI * BJ) void k_adj_cell(AdjAdvArgs a)
 {
@@ -174,22 +201,28 @@ __global__ __launch_bounds__(64 * BI * BJ) void k_adj_cell(AdjAdvArgs a)
     const int i = blockIdx.y * BI + il;
     const int j = blockIdx.z * BJ + jl;
     const bool cell_ok = k < nn && i < nr && j < nz;
-    const bool act = cell_ok && k >= a.krange[0] && k <= a.krange[1];
-    if (act) {
-        auto put_r = [&](int f, int slot) {
-            const m1a::FaceT<double> r = face_at<double>(a, 0, f, i, j, k, -1, -1);
-            double* o = &rF[jl][slot][0][lane];
-            o[0] = r.FJ; o[64] = r.FHr; o[128] = r.FHz; o[192] = r.kphi_L; o[256] = r.kphi_R;
-        };
-        auto put_z = [&](int g, int slot) {
-            const m1a::FaceT<double> r = face_at<double>(a, 1, g, i, j, k, -1, -1);
-            double* o = &zF[slot][il][0][lane];
-            o[0] = r.FJ; o[64] = r.FHr; o[128] = r.FHz;
-        };
-        put_r(i, il);
-        if (il == BI - 1 || i == nr - 1) put_r(i + 1, il + 1);
-        put_z(j, jl);
-        if (jl == BJ - 1 || j == nz - 1) put_z(j + 1, jl + 1);
+    const bool bin_act = k < nn && k >= a.krange[0] && k <= a.krange[1];
+    const bool act = cell_ok && bin_act;
+    if (bin_act) {
+        // the block's interfaces, dealt out evenly over its wavefronts
+        constexpr int kR = BJ * (BI + 1), kZ = (BJ + 1) * BI;
+        const int i0 = blockIdx.y * BI, j0 = blockIdx.z * BJ;
+#pragma unroll 1
+        for (int t = __builtin_amdgcn_readfirstlane(jl * BI + il); t < kR + kZ; t += BI * BJ) {
+            if (t < kR) {
+                const int row = t / (BI + 1), slot = t % (BI + 1);
+                if (i0 + slot > nr || j0 + row >= nz) continue;
+                const FaceResult r = face_values<0>(a, i0 + slot, 0, j0 + row, k);
+                double* o = &rF[row][slot][0][lane];
+                o[0] = r.F.J; o[64] = r.F.Hr; o[128] = r.F.Hz; o[192] = r.kphi_L; o[256] = r.kphi_R;
+            } else {
+                const int slot = (t - kR) / BI, col = (t - kR) % BI;
+                if (j0 + slot > nz || i0 + col >= nr) continue;
+                const FaceResult r = face_values<1>(a, j0 + slot, i0 + col, 0, k);
+                double* o = &zF[slot][col][0][lane];
+                o[0] = r.F.J; o[64] = r.F.Hr; o[128] = r.F.Hz;
+            }
+        }
     }
     __syncthreads();
     if (!cell_ok) return;
@@ -256,7 +289,8 @@ __global__ __launch_bounds__(64 * BI * BJ) void k_adj_cell(AdjAdvArgs a)
     lHzs += lHzn2;
     // D:∇u of the cell's own closure
     if (lDdu != 0.0) {
-#pragma unroll 1
+        // unrolled, so that the three passes share their values
+#pragma unroll
         for (int var = 0; var < 3; ++var) {
             Dl tJ(Js, var == 0 ? 1.0 : 0.0), tHr(Hrs, var == 1 ? 1.0 : 0.0), tHz(Hzs, var == 2 ? 1.0 : 0.0);
             m1a::EddT<Dl> Dd = m1a::tD_edd(tHr, tHz, tJ);
@@ -702,7 +736,14 @@ __device__ __forceinline__ double wsum(double v)
 }
 }  // namespace
 
-__global__ __launch_bounds__(64) void k_adj_column(AdjColArgs a)
+// MODE: rows differentiated in reverse mode (0) or by dual numbers (1), a kernel each: together they
+// took 214 VGPRs, reverse mode alone 123.  Latency bound (chains of a solve, few wavefronts): the
+// wavefronts in flight are as many as LDS holds, eleven rows of N_ν each (the rows' derivatives
+// take the place of the solved rows, and the serial solve's factors exist above 128 rows only):
+// fourteen on a CU at 128 bins, where sixteen rows and 214 VGPRs allowed eight.  128x128x128: 209 us,
+// was 262; 45x61x64: 31 us, was 40.
+template <int MODE>
+__global__ __launch_bounds__(64, MODE == 0 ? 4 : 2) void k_adj_column(AdjColArgs a)
 {
     extern __shared__ double lds[];
     const int nn = a.nn, nr = a.nr;
@@ -718,14 +759,13 @@ __global__ __launch_bounds__(64) void k_adj_column(AdjColArgs a)
     double* rC = lds + 5 * nn;
     double* x = lds + 6 * nn;
     double* mu = lds + 7 * nn;
-    double* cp = lds + 8 * nn;
-    double* cq = lds + 9 * nn;
-    double* lJ = lds + 10 * nn;    // cotangent of E's output, then of the advection output
-    double* lHr = lds + 11 * nn;
-    double* lHz = lds + 12 * nn;
-    double* gm = lds + 13 * nn;    // row k's derivative contributions to Hvoigt at k-1, k, k+1
-    double* g0 = lds + 14 * nn;
-    double* gp = lds + 15 * nn;
+    double* lJ = lds + 8 * nn;     // cotangent of E's output, then of the advection output
+    double* lHr = lds + 9 * nn;
+    double* lHz = lds + 10 * nn;
+    double* cp = lds + 11 * nn;    // of more than 128 rows only
+    double* cq = lds + 12 * nn;
+    // row k's derivative contributions to Hvoigt at k-1, k, k+1, in the place of the rows once solved
+    double *gm = rA, *g0 = rB, *gp = rC;
     const double ct = a.c_tilde, dt = a.dt, dw = a.dw;
     const double fpc_ict = (kFourPi / kC) * (1.0 / ct);
     const double ac = a.alpha_c[c], al = a.alpha[c], pd = a.pd[c], jsv = a.js[c];
@@ -745,7 +785,6 @@ __global__ __launch_bounds__(64) void k_adj_column(AdjColArgs a)
         X2z[k] = h1z / denH;
         sr += a.dnu[k] * (h1r - X2r[k]);
         sz += a.dnu[k] * (h1z - X2z[k]);
-        gm[k] = 0.0; g0[k] = 0.0; gp[k] = 0.0;
     }
     sr = wsum(sr);
     sz = wsum(sz);
@@ -863,6 +902,8 @@ __global__ __launch_bounds__(64) void k_adj_column(AdjColArgs a)
 
     // ---- matrix cotangents contracted with each row's local derivatives ----
     double lPREF = 0.0, lREC = 0.0;
+    for (int k = lane; k < nn; k += 64) { gm[k] = 0.0; g0[k] = 0.0; gp[k] = 0.0; }
+    __syncthreads();
     for (int k = lane + 1; k <= nn - 2; k += 64) {
         const int r = k - 1;
         const double m_r = mu[r];
@@ -876,7 +917,7 @@ __global__ __launch_bounds__(64) void k_adj_column(AdjColArgs a)
         const m1a::RowConst rc = row_const(k);
         // derivatives along the six inputs: reverse mode, or (mode 1) two per dual pass
         double g[6];
-        if (a.mode == 0) {
+        if (MODE == 0) {
             m1a::freq_row_vjp(rc, Hv[k - 1], Hv[k], Hv[k + 1], PREFACT, RECOIL_0, VEL, lFkp, lFk, lFkm, g);
         } else {
 #pragma unroll 1
@@ -1011,8 +1052,9 @@ __global__ void k_adj_axpy_cell(double* y, const double* dV, double s, int n)
 void launch_adj_column(hipStream_t s, const AdjColArgs& a)
 {
     const int ncell = a.nr * a.nz;
-    const size_t lds = 16 * (size_t)a.nn * sizeof(double);
-    hipLaunchKernelGGL(k_adj_column, dim3(ncell), dim3(64), lds, s, a);
+    const size_t lds = (a.nn - 2 <= 128 ? 11 : 13) * (size_t)a.nn * sizeof(double);
+    if (a.mode == 0) hipLaunchKernelGGL(k_adj_column<0>, dim3(ncell), dim3(64), lds, s, a);
+    else hipLaunchKernelGGL(k_adj_column<1>, dim3(ncell), dim3(64), lds, s, a);
 }
 
 // The interfaces of one direction.  In units of one interface by a wavefront that has its SIMD to

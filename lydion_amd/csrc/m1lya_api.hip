@@ -1265,7 +1265,7 @@ int m1lya_adjoint_run(m1lya_ctx* c, int n_steps, double c_tilde, double dt, doub
         if (n_steps < 1) fail(c, M1LYA_ERR_ARG, "n_steps < 1");
         if (checkpoint_every < 0) fail(c, M1LYA_ERR_ARG, "checkpoint_every < 0");
         if (!(c_tilde > 0.0) || !(dt > 0.0)) fail(c, M1LYA_ERR_ARG, "c_tilde and dt must be > 0");
-        // the reverse column kernel keeps 16 rows of N_ν doubles in LDS (32 KiB at 256 bins)
+        // the reverse column kernel keeps up to 13 rows of N_ν doubles in LDS (26 KiB at 256 bins)
         if (c->nn > kMaxBinsAdjoint)
             fail(c, M1LYA_ERR_DIMS, "the adjoint supports N_ν <= " + std::to_string(kMaxBinsAdjoint));
         const size_t n3 = c->n3, nc = c->ncell, B3 = 3 * n3;
