@@ -448,18 +448,14 @@ constexpr size_t step_lds_bytes(int wpb, int nq)
 
 // kPair (with NQ = 1, clouds of N_ν <= 32): the two halves of a wavefront hold two neighbouring
 // cells of its row, i (lanes 0-31) and i+1 (lanes 32-63), one bin per lane, so that such clouds
-// fill every lane; the march advances two cells at a time.  The launch covers the blocks
-// [blk0, blk1) of the batch.  rows: the block forms its partial row; without it (short segments)
-// k_rows does.
+// fill every lane; the march advances two cells at a time.  lb: the block of the batch.  rows: the
+// block forms its partial row; without it (short segments) k_rows does.
 template <bool kShear, int NQ, bool kPair>
-__global__ __launch_bounds__(64 * kMaxWaves, NQ <= 2 ? 4 : 2) void k_step(const Cloud* __restrict__ clouds, Arrays A,
-                                                            const Seg* __restrict__ segs, int blk0, int blk1,
-                                                            int wpb, int parity, int rows,
-                                                            const int* __restrict__ krange,
-                                                            double* __restrict__ part, const Ctrl* __restrict__ ctrl)
+__device__ __forceinline__ void step_block(const Cloud* __restrict__ clouds, const Arrays& A,
+                                           const Seg* __restrict__ segs, int lb, int wpb, int parity, int rows,
+                                           const int* __restrict__ krange, double* __restrict__ part)
 {
     static_assert(!kPair || NQ == 1, "pair mode holds one bin per lane");
-    if (ctrl->halt) return;
     constexpr int kB = 64 * NQ;          // bins a wavefront holds
     constexpr int kSh = 2 * kB + 8;      // LDS row of the per-wavefront sums
     extern __shared__ __align__(16) unsigned char smem[];
@@ -468,8 +464,6 @@ __global__ __launch_bounds__(64 * kMaxWaves, NQ <= 2 ? 4 : 2) void k_step(const 
     double (*sacc)[2 * kNScal] = reinterpret_cast<double (*)[2 * kNScal]>(&sh[wpb][0]);
     float (*zrow)[3][kB] = reinterpret_cast<float (*)[3][kB]>(&sacc[wpb][0]);
     float (*zflx)[3][kB] = zrow + (wpb + 4);
-    const int lb = blk0 + xcd_block(blockIdx.x, gridDim.x);
-    if (lb >= blk1) return;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Seg sg = segs[(size_t)lb * wpb + wave];
@@ -1122,6 +1116,42 @@ __global__ __launch_bounds__(64 * kMaxWaves, NQ <= 2 ? 4 : 2) void k_step(const 
         KSum s{0, 0};
         for (int w = 0; w < wpb; ++w) s.add(sh[w][t]);
         part[(size_t)lb * kPartStride + t] = s.value();
+    }
+}
+
+// The step of the blocks [blk0, blk1) of the batch.
+template <bool kShear, int NQ, bool kPair>
+__global__ __launch_bounds__(64 * kMaxWaves, NQ <= 2 ? 4 : 2) void k_step(const Cloud* __restrict__ clouds, Arrays A,
+                                                            const Seg* __restrict__ segs, int blk0, int blk1,
+                                                            int wpb, int parity, int rows,
+                                                            const int* __restrict__ krange,
+                                                            double* __restrict__ part, const Ctrl* __restrict__ ctrl)
+{
+    if (ctrl->halt) return;
+    const int lb = blk0 + xcd_block(blockIdx.x, gridDim.x);
+    if (lb >= blk1) return;
+    step_block<kShear, NQ, kPair>(clouds, A, segs, lb, wpb, parity, rows, krange, part);
+}
+
+// Both kinds of blocks in one launch: the wavefronts' blocks of one cell (grid0 of them, rounded up
+// to the XCDs, the longer ones) first, those of two cells behind them, so that neither kind's last
+// wave of blocks leaves CUs idle.  Sweep of 16 (400 and 1680 blocks): 486 us, 234 + 284 by a launch
+// each.
+template <bool kShear>
+__global__ __launch_bounds__(64 * kMaxWaves, 4) void k_step_mixed(const Cloud* __restrict__ clouds, Arrays A,
+                                                                  const Seg* __restrict__ segs, int nblk_pair,
+                                                                  int nblk, int grid0, int wpb, int parity, int rows,
+                                                                  const int* __restrict__ krange,
+                                                                  double* __restrict__ part,
+                                                                  const Ctrl* __restrict__ ctrl)
+{
+    if (ctrl->halt) return;
+    if ((int)blockIdx.x < grid0) {
+        const int lb = nblk_pair + xcd_block(blockIdx.x, grid0);
+        if (lb < nblk) step_block<kShear, 2, false>(clouds, A, segs, lb, wpb, parity, rows, krange, part);
+    } else {
+        const int lb = xcd_block(blockIdx.x - grid0, gridDim.x - grid0);
+        if (lb < nblk_pair) step_block<kShear, 1, true>(clouds, A, segs, lb, wpb, parity, rows, krange, part);
     }
 }
 
@@ -1823,42 +1853,57 @@ void launch_step_kernels(m1lya_batch* b, int parity)
 {
     hipStream_t s = b->stream;
     const dim3 block(64 * b->wpb);
-    if (b->nblk_pair > 0) {
-        // clouds of N_ν <= 32, two cells per wavefront
-        BProf p(b, "k_step_pair", true);
-        const size_t lds = step_lds_bytes(b->wpb, 1);
-        const dim3 grid((b->nblk_pair + 7) / 8 * 8);
+    // both kinds of blocks share a launch (clouds of more than 128 bins, whose blocks leave room for
+    // half as many wavefronts, have their own; so has each kind when launches are timed)
+    if (b->nblk_pair > 0 && b->nblk > b->nblk_pair && !b->wide && !b->profiling) {
+        const int grid0 = (b->nblk - b->nblk_pair + 7) / 8 * 8;
+        const dim3 grid(grid0 + (b->nblk_pair + 7) / 8 * 8);
+        const size_t lds = std::max(step_lds_bytes(b->wpb, 1), step_lds_bytes(b->wpb, 2));
         if (b->shear)
-            hipLaunchKernelGGL((k_step<true, 1, true>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, 0, b->nblk_pair,
-                               b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
+            hipLaunchKernelGGL((k_step_mixed<true>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b->nblk_pair,
+                               b->nblk, grid0, b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
         else
-            hipLaunchKernelGGL((k_step<false, 1, true>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, 0,
-                               b->nblk_pair, b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
-        p.done();
-    }
-    if (b->nblk > b->nblk_pair) {
-        BProf p(b, "k_step", true);
-        // the variant with the reference-row path for sheared / anisotropic velocity gradients only
-        // when a cell of the batch needs it: it costs registers the common path does not pay for
-        // and the four-bins-per-lane variant only when a cloud has more than 128 bins
-        const size_t lds = step_lds_bytes(b->wpb, b->wide ? 4 : 2);
-        const int b0 = b->nblk_pair, b1 = b->nblk;
-        const dim3 grid((b1 - b0 + 7) / 8 * 8);
-        if (b->wide) {
+            hipLaunchKernelGGL((k_step_mixed<false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b->nblk_pair,
+                               b->nblk, grid0, b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
+        bchk(b, hipGetLastError(), "k_step_mixed");
+    } else {
+        if (b->nblk_pair > 0) {
+            // clouds of N_ν <= 32, two cells per wavefront
+            BProf p(b, "k_step_pair", true);
+            const size_t lds = step_lds_bytes(b->wpb, 1);
+            const dim3 grid((b->nblk_pair + 7) / 8 * 8);
             if (b->shear)
-                hipLaunchKernelGGL((k_step<true, 4, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
-                                   b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
+                hipLaunchKernelGGL((k_step<true, 1, true>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, 0,
+                                   b->nblk_pair, b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
             else
-                hipLaunchKernelGGL((k_step<false, 4, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
-                                   b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
-        } else if (b->shear) {
-            hipLaunchKernelGGL((k_step<true, 2, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
-                               b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
-        } else {
-            hipLaunchKernelGGL((k_step<false, 2, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
-                               b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
+                hipLaunchKernelGGL((k_step<false, 1, true>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, 0,
+                                   b->nblk_pair, b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
+            p.done();
         }
-        p.done();
+        if (b->nblk > b->nblk_pair) {
+            BProf p(b, "k_step", true);
+            // the variant with the reference-row path for sheared / anisotropic velocity gradients only
+            // when a cell of the batch needs it: it costs registers the common path does not pay for
+            // and the four-bins-per-lane variant only when a cloud has more than 128 bins
+            const size_t lds = step_lds_bytes(b->wpb, b->wide ? 4 : 2);
+            const int b0 = b->nblk_pair, b1 = b->nblk;
+            const dim3 grid((b1 - b0 + 7) / 8 * 8);
+            if (b->wide) {
+                if (b->shear)
+                    hipLaunchKernelGGL((k_step<true, 4, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
+                                       b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
+                else
+                    hipLaunchKernelGGL((k_step<false, 4, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
+                                       b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
+            } else if (b->shear) {
+                hipLaunchKernelGGL((k_step<true, 2, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
+                                   b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
+            } else {
+                hipLaunchKernelGGL((k_step<false, 2, false>), grid, block, lds, s, b->d_cl, b->A, b->d_segs, b0, b1,
+                                   b->wpb, parity, b->step_rows ? 1 : 0, b->krange, b->part, b->ctrl);
+            }
+            p.done();
+        }
     }
     if (!b->step_rows) {
         BProf p(b, "k_rows");

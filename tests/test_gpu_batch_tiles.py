@@ -61,3 +61,39 @@ def test_sized_tiles_report_a_non_finite_state(lut):
         errors.append(str(e.value))
         b.close()
     assert errors[0] == errors[1]
+
+
+@pytest.mark.parametrize("shear", [False, True])
+@pytest.mark.parametrize("tiles", [None, (16, 8), (5, 3)])
+def test_both_kinds_of_blocks_in_one_launch(lut, tiles, shear):
+    """Clouds of one and of two cells per wavefront in a batch step in one launch, or in one each when
+    launches are timed; either way every cloud has the bits that it has alone."""
+    sizes = [(31, 20, 32), (40, 33, 66), (7, 50, 18), (29, 17, 128)]
+    clouds = [developed_state(small_cloud(n_r=r, n_z=z, n_nu=n, tau0=1e7, umax=100.0, lut=lut)) for r, z, n in sizes]
+    if shear:
+        for c in clouds:
+            c.lya["duz_dr"] = c.lya["duz_dr"] + 0.3 * c.lya["dur_dr"]
+
+    def run(cs, profiling, graph):
+        b = M1LyaBatch(cs)
+        if tiles:
+            b.set_tiles(*tiles)
+        b.set_graph(graph)
+        b.set_profiling(profiling)
+        h = b.run_steps(5)
+        state = [[b.download(i, k) for k in STATE] for i in range(len(cs))]
+        names = set(b.kernel_stats())
+        b.close()
+        return h, state, names
+
+    h0, s0, _ = run(clouds, 0, False)
+    for profiling, graph in ((1, False), (0, True)):
+        h, s, names = run(clouds, profiling, graph)
+        assert not profiling or {"k_step", "k_step_pair"} <= names
+        assert np.array_equal(h, h0)
+        assert all(np.array_equal(x, y) for a, b in zip(s, s0) for x, y in zip(a, b))
+    for i, c in enumerate(clouds):
+        # caller-set tiles give the row's sums their own partition; the state is free of it
+        h, s, _ = run([c], 0, False)
+        assert np.array_equal(h[:, 0], h0[:, i])
+        assert all(np.array_equal(x, y) for x, y in zip(s[0], s0[i]))
