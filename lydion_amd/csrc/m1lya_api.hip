@@ -452,8 +452,10 @@ void replay_step(m1lya_ctx* c, double c_tilde, double dt, double z_center, int b
 // stream is synchronised.
 void download(m1lya_ctx* c, double* host, const double* src, size_t n, const char* what)
 {
-    if (n * sizeof(double) >= m1t::kMinBytes && m1t::pageable(host))
-        hipchk(c, c->down.run(host, src, n, 1.0, c->device, c->stream), what);
+    hipError_t e;
+    if (n * sizeof(double) >= m1t::kMinBytes && m1t::pageable(host) &&
+        c->down.run(host, src, n, 1.0, c->device, c->stream, e))
+        hipchk(c, e, what);
     else
         hipchk(c, hipMemcpyAsync(host, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream), what);
 }

@@ -2468,8 +2468,9 @@ int m1lya_batch_download(m1lya_batch* b, int cloud, int field, double* host, siz
             if (count != n) bfail(b, M1LYA_ERR_ARG, "field " + std::to_string(field) + ": wrong count");
         };
         auto down32 = [&](const float* src, size_t n, double scale) {
-            if (n * sizeof(double) >= m1t::kMinBytes) {
-                bchk(b, b->down.run(host, src, n, scale, b->device, b->stream), "download");
+            hipError_t e;
+            if (n * sizeof(double) >= m1t::kMinBytes && b->down.run(host, src, n, scale, b->device, b->stream, e)) {
+                bchk(b, e, "download");
                 return;
             }
             std::vector<float> h(n);

@@ -55,28 +55,37 @@ public:
     }
 
     // host[0 .. n) = src[0 .. n), FP32 values times scale, once the stream's work so far is done;
-    // returns when the copy is complete.
+    // returns when the copy is complete, its outcome in result.  False: there is no pinned memory to
+    // be had, and nothing was copied.
     template <class T>
-    hipError_t run(double* host, const T* src, size_t n, double scale, int device, hipStream_t stream)
+    bool run(double* host, const T* src, size_t n, double scale, int device, hipStream_t stream, hipError_t& result)
     {
         std::lock_guard<std::mutex> hold(lock);
         constexpr size_t kElems = kChunkBytes / sizeof(T);
         const size_t chunks = (n + kElems - 1) / kElems;
         const unsigned cpus = std::max(1u, std::thread::hardware_concurrency());
-        const int workers = (int)std::min<size_t>(std::min<size_t>(kWorkers, cpus), chunks);
+        const int most = (int)std::min<size_t>(std::min<size_t>(kWorkers, cpus), chunks);
         int current = device;
         (void)hipGetDevice(&current);
-        hipError_t e = current != device ? hipSetDevice(device) : hipSuccess;
-        for (int w = 0; e == hipSuccess && w < workers; ++w) {
-            if (!buf[w]) e = hipHostMalloc(&buf[w], kChunkBytes, hipHostMallocDefault);
-            if (e == hipSuccess && !ev[w]) e = hipEventCreateWithFlags(&ev[w], hipEventDisableTiming);
-        }
-        if (e == hipSuccess) e = copy(host, src, n, scale, device, stream, workers, chunks);
+        result = current != device ? hipSetDevice(device) : hipSuccess;
+        int workers = 0;
+        while (result == hipSuccess && workers < most && slot(workers)) ++workers;
+        if (result == hipSuccess && workers > 0) result = copy(host, src, n, scale, device, stream, workers, chunks);
         if (current != device) (void)hipSetDevice(current);
-        return e;
+        return result != hipSuccess || workers > 0;
     }
 
 private:
+    // Worker w's buffer and event
+    bool slot(int w)
+    {
+        if (!buf[w] && hipHostMalloc(&buf[w], kChunkBytes, hipHostMallocDefault) != hipSuccess) buf[w] = nullptr;
+        if (buf[w] && !ev[w] && hipEventCreateWithFlags(&ev[w], hipEventDisableTiming) != hipSuccess) ev[w] = nullptr;
+        if (buf[w] && ev[w]) return true;
+        (void)hipGetLastError();
+        return false;
+    }
+
     template <class T>
     hipError_t copy(double* host, const T* src, size_t n, double scale, int device, hipStream_t stream, int workers,
                     size_t chunks)
