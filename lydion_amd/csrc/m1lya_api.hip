@@ -526,8 +526,9 @@ int m1lya_create(int n_nu, int n_r, int n_z, int precision, m1lya_ctx** out)
         c->A_z = dalloc(c, (size_t)n_r * (n_z + 1));
         c->inv_r_cell = dalloc(c, n_r); c->rcom = dalloc(c, n_r); c->zcom = dalloc(c, n_z);
         c->ivr = dalloc(c, (size_t)(n_r + 1) * 5); c->ivz = dalloc(c, (size_t)(n_z + 1) * 5);
-        c->nu = dalloc(c, n_nu + 1); c->nuC = dalloc(c, n_nu); c->dnu = dalloc(c, n_nu);
-        c->inv_dnu = dalloc(c, n_nu); c->inv_nuC = dalloc(c, n_nu);
+        const int nb = (n_nu + 63) / 64 * 64;   // the column kernel's lanes read past the last bin
+        c->nu = dalloc(c, nb + 1); c->nuC = dalloc(c, nb); c->dnu = dalloc(c, nb);
+        c->inv_dnu = dalloc(c, nb); c->inv_nuC = dalloc(c, nb);
         c->col = column_shape(n_nu, nc);
         c->act_blocks = (int)std::min<size_t>(nc, 1024);
         c->pstride = 2 * n_nu + 8;

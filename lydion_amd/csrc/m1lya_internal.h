@@ -9,7 +9,7 @@ namespace m1 {
 
 // Most cell columns per wavefront in the column kernel (lane-per-column dgtsv).
 constexpr int kColumnW = 4;
-// Largest N_ν of the FP64 context (nine bins per lane, one column per wavefront).
+// Largest N_ν of the FP64 context (nine bins per lane in the column kernel).
 constexpr int kMaxBinsFP64 = 576;
 constexpr int kMaxBinsAdjoint = 256;
 
@@ -239,13 +239,18 @@ void launch_advect(hipStream_t s, const AdvectArgs& a);
 // alone, so that the partition of the fused reductions, and with it their bits, does not depend
 // on the device.
 //
-// Four wavefronts per block fill 64 KB of LDS with the rows of w·nw columns (16 up to 128 bins, 8
-// up to 256); wider grids keep one wavefront and one column of up to 18 KB.  The grid is exactly
-// one wave of resident blocks (kColumnBlocks / nw on MI355X: 8 wavefronts per CU, 256 CUs), so
-// that every block loops over the same number of column groups and they all start together: a
-// larger one left a partial second wave starting late.  While fewer cells than one such wave
-// holds are there, w is halved, so that the columns spread over more blocks.
-constexpr int kColumnBlocks = 2048;
+// A column takes five arrays of N_ν-2 rows of LDS, and the w·nw columns of a block as many as leave
+// room for two blocks in a CU's 160 KB: 81 KB for 16 columns of 128 bins, 82 KB for 8 of 256 and for
+// 4 of 512, 69 KB for 3 of 576.  Blocks of several wavefronts above 256 bins too: a column's solve
+// is a chain that takes a wavefront's issue slots however few of its lanes solve, so that eight
+// one-wavefront blocks on a CU ran two chains on each SIMD (870 cycles a row, 380 for a chain alone).
+// 45x61x320: 158 us, 265 by one-wavefront blocks; 128x128x542: 1.49 ms, 1.90 by one-wavefront
+// blocks that spread the bins of a wavefront and shared no term between rows.
+//
+// The grid is at most one wave of resident blocks (two per CU at 256 VGPRs), which loop over the
+// column groups: a larger one left a partial second wave starting late.  While fewer cells than one
+// such wave holds are there, w is halved, so that the columns spread over more blocks.
+constexpr int kColumnBlocks = 512;
 struct ColumnShape {
     int w, nw, blocks;
 };

@@ -594,6 +594,25 @@ __device__ __forceinline__ void one_minus_phi(double P, double r, double& o, dou
     chi = small ? (sgn < 0 ? 1.0 : -1.0) - 0.5 * P : quot(1.0 - e, P, r);
 }
 
+// AbsorptionUpdateJorH (src/ConstantsAndFunctions.jl:451-462) for J and the two components of H,
+// which share their divisor.
+__device__ __forceinline__ void absorb(double aJ, double dJdt, double aH, double ct, double dt, double& J, double& Hr,
+                                       double& Hz)
+{
+    const double den = 1.0 + aH * ct * dt, rden = rcp_nr(den);
+    double jn = quot(J + dJdt * dt, 1.0 + aJ * ct * dt);
+    double hrn = quot(Hr + 0.0 * dt, den, rden);
+    double hzn = quot(Hz + 0.0 * dt, den, rden);
+    // numerators whose residual could underflow, and divisors out of range
+    if (__builtin_expect(!(fabs(Hr) > 0x1p-900) || !(fabs(Hz) > 0x1p-900) || !(fabs(den) < 0x1p500) ||
+                             !(fabs(aJ) * ct * dt < 0x1p500), 0)) {
+        hrn = (Hr + 0.0 * dt) / den;
+        hzn = (Hz + 0.0 * dt) / den;
+        jn = (J + dJdt * dt) / (1.0 + aJ * ct * dt);
+    }
+    J = jn; Hr = hrn; Hz = hzn;
+}
+
 // The KPL consecutive bins of a lane, from k0; bins past N_ν are left as they are.
 template <int KPL>
 __device__ __forceinline__ void load_bins(const double* __restrict__ p, int k0, int nn, double (&v)[KPL])
@@ -630,20 +649,23 @@ __device__ __forceinline__ void store_bins(double* __restrict__ p, int k0, int n
 //   P1 (lanes over k): emission/absorption (src/ConstantsAndFunctions.jl:483-573),
 //       frequency factors (src/FreqFactors.jl:142-278), tridiagonal rows to LDS
 //       (src/UpdateLyaJandH.jl:178-227);
-//   P2 (lane per column): dgtsv on the LDS columns, all W·NW of them by the block's first
-//       wavefront: the elimination is a serial chain per column, so the issue cost of P2 is
+//   P2 (lane per column): dgtsv on the LDS columns, all W·NW of them by one wavefront of the
+//       block: the elimination is a serial chain per column, so the issue cost of P2 is
 //       one wavefront instruction per row step for as many columns as lanes take part;
 //   P3 (lanes over k): J floor, H rescale and causality, old copies
 //       (src/UpdateLyaJandH.jl:335-379), plus the fused step's reductions.
 // A lane holds KPL consecutive bins, so that a row's neighbours k-1 and k+1 are mostly the
 // lane's own: what a bin contributes to three rows (its diffusion coefficient's reciprocal, its
-// drift, and in cells at rest its exponentials too) is formed once and passed on.
+// drift, and in cells at rest its exponentials too) is formed once and passed on, through a window
+// of two bins: 247 registers and no spills at four bins per lane, where all the bins' terms at once
+// took 256 and 284 bytes of scratch, and 360 to 512 from five bins on (one wavefront per SIMD).
+// 90x90x194: 140 us, 165 with all terms at once.
 // What bounds it: instruction issue in P1 and P3 (two wavefronts per SIMD, whose loads are not
 // all covered), and P2's one wavefront per block.  256x256x128 cone cloud: 592 -> 397 us (P1 and
 // P3 alone 410 -> 240 us: shared factors, divisions without range handling, one pass of per-cell
 // terms per column group); 77x90x194: 251 -> 179 us; 32x32x64: 33 -> 18 us (columns spread over
 // four times the blocks).  Loads three or four rows ahead in P2 measured no better than two.
-// LDS per block: 5 arrays x (N_ν-2) rows x W·NW columns (odd row stride, so the
+// LDS per block: 5 arrays x (N_ν-2) rows x W·NW columns (odd row stride, so that the
 // lane-per-column sweep is bank-conflict free).
 // ------------------------------------------------------------------------
 // kFused: the instantiation for the fused step's phases (emission, frequency factors, solve,
@@ -651,8 +673,11 @@ __device__ __forceinline__ void store_bins(double* __restrict__ p, int k0, int n
 // only COL_CONV is read from the arguments.
 constexpr int kFusedFlags = COL_EMIT | COL_FREQ | COL_SOLVE | COL_HCORR | COL_FUSED;
 
+// Most bins per lane at which k_column also serves the calls without a solve.
+constexpr int kBinsPerLaneAll = 4;
+
 template <int W, int KPL, int NW, bool kFused>
-__global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a)
+__global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
 {
     extern __shared__ double lds[];
     const int nn = a.nn, nr = a.nr, nz = a.nz;
@@ -662,8 +687,9 @@ __global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a
     const int k0 = lane * KPL;   // the lane's bins are k0 .. k0 + KPL - 1
     constexpr int WB = W * NW;   // columns of the block
     const int flags = kFused ? (kFusedFlags | (a.flags & COL_CONV)) : a.flags;
-    const bool EMIT = flags & COL_EMIT, FREQ = flags & COL_FREQ, STOREF = flags & COL_STORE_F;
-    const bool SOLVE = flags & COL_SOLVE, HCORR = flags & COL_HCORR, FUSED = flags & COL_FUSED;
+    constexpr bool kWide = KPL > kBinsPerLaneAll;   // calls without a solve go to k_bins
+    const bool EMIT = (kFused || !kWide) && (flags & COL_EMIT), FREQ = flags & COL_FREQ, STOREF = flags & COL_STORE_F;
+    const bool SOLVE = kWide || (flags & COL_SOLVE), HCORR = kWide || (flags & COL_HCORR), FUSED = flags & COL_FUSED;
     const bool CONV = flags & COL_CONV;
     if (a.halt && *a.halt) return;
     const int S = col_stride(nn);
@@ -689,23 +715,28 @@ __global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a
     const double fpc_ict = (kFourPi / kC) * inv_ct;
     const double inv_dt = 1.0 / dt;
 
-    // the grid's constants of the lane's bins: widths of the two halves, Δν, 1/Δν, 2/νC.  Up to two
-    // bins per lane they stay in registers; beyond, they are loaded again for every column.
-    double hR[KPL], hL[KPL], dnu[KPL], idn[KPL], two[KPL];
-    auto load_grid = [&](bool factors) {
+    // the grid's constants of the lane's bins: Δν, widths of the two halves, 1/Δν, 2/νC.  Up to two
+    // bins per lane they stay in registers; beyond, they are read where a row needs them.
+    constexpr bool kKeep = KPL <= 2;
+    constexpr int kGrid = kKeep ? KPL : 1;
+    double g_dnu[kGrid], g_hR[kGrid], g_hL[kGrid], g_idn[kGrid], g_two[kGrid];
+    if (kKeep) {
 #pragma unroll
-        for (int q = 0; q < KPL; ++q) {
-            const int k = min(k0 + q, nn - 1);
-            dnu[q] = a.dnu[k];
-            if (!factors) continue;
+        for (int q = 0; q < kGrid; ++q) {
+            const int k = k0 + q;
             const double nuC = a.nuC[k];
-            hR[q] = a.nu[k + 1] - nuC;
-            hL[q] = nuC - a.nu[k];
-            idn[q] = a.inv_dnu[k];
-            two[q] = 2.0 * a.inv_nuC[k];
+            g_dnu[q] = a.dnu[k];
+            g_hR[q] = a.nu[k + 1] - nuC;
+            g_hL[q] = nuC - a.nu[k];
+            g_idn[q] = a.inv_dnu[k];
+            g_two[q] = 2.0 * a.inv_nuC[k];
         }
-    };
-    if (KPL <= 2) load_grid(true);
+    }
+    auto grid_dnu = [&](int q) { return kKeep ? g_dnu[kKeep ? q : 0] : a.dnu[k0 + q]; };
+    auto grid_hR = [&](int q) { return kKeep ? g_hR[kKeep ? q : 0] : a.nu[k0 + q + 1] - a.nuC[k0 + q]; };
+    auto grid_hL = [&](int q) { return kKeep ? g_hL[kKeep ? q : 0] : a.nuC[k0 + q] - a.nu[k0 + q]; };
+    auto grid_idn = [&](int q) { return kKeep ? g_idn[kKeep ? q : 0] : a.inv_dnu[k0 + q]; };
+    auto grid_two = [&](int q) { return kKeep ? g_two[kKeep ? q : 0] : 2.0 * a.inv_nuC[k0 + q]; };
     double e1[KPL], e10[KPL];
 #pragma unroll
     for (int kk = 0; kk < KPL; ++kk) { e1[kk] = 0.0; e10[kk] = 0.0; }
@@ -724,7 +755,6 @@ __global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a
             const int c = grp * WB + lc;
             if (c >= ncells) continue;
             const size_t base = (size_t)c * nn;
-            if (KPL > 2) load_grid(true);
             double Jcur[KPL], hv[KPL];
 #pragma unroll
             for (int q = 0; q < KPL; ++q) { Jo[w][q] = 1.0; Hr[w][q] = 0.5; Hz[w][q] = 0.5; hv[q] = 1.0; }   // bins past N_ν
@@ -741,29 +771,12 @@ __global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a
                 load_bins<KPL>(a.aF + base, k0, nn, aF);
 #pragma unroll
                 for (int q = 0; q < KPL; ++q) {
-                    // AbsorptionUpdateJorH (src/ConstantsAndFunctions.jl:451-462); the two
-                    // components of H share their divisor
-                    const double aJ = ac + al_pd * hv[q];
-                    const double dJdt = js_ct * ph[q];
-                    const double jn = quot(Jo[w][q] + dJdt * dt, 1.0 + aJ * ct * dt);
-                    const double den = 1.0 + aF[q] * ct * dt, rden = rcp_nr(den);
                     const double hr = Hr[w][q], hz = Hz[w][q];
-                    double hrn = quot(hr + 0.0 * dt, den, rden);
-                    double hzn = quot(hz + 0.0 * dt, den, rden);
-                    // numerators whose residual could underflow, and divisors out of range
-                    if (__builtin_expect(!(fabs(hr) > 0x1p-900) || !(fabs(hz) > 0x1p-900) || !(fabs(den) < 0x1p500) ||
-                                             !(fabs(aJ) * ct * dt < 0x1p500), 0)) {
-                        hrn = (hr + 0.0 * dt) / den;
-                        hzn = (hz + 0.0 * dt) / den;
-                        Jcur[q] = (Jo[w][q] + dJdt * dt) / (1.0 + aJ * ct * dt);
-                    } else {
-                        Jcur[q] = jn;
-                    }
+                    absorb(ac + al_pd * hv[q], js_ct * ph[q], aF[q], ct, dt, Jo[w][q], Hr[w][q], Hz[w][q]);
                     if (k0 + q < nn) {
-                        sr += dnu[q] * (hr - hrn);
-                        sz += dnu[q] * (hz - hzn);
+                        sr += grid_dnu(q) * (hr - Hr[w][q]);
+                        sz += grid_dnu(q) * (hz - Hz[w][q]);
                     }
-                    Jo[w][q] = Jcur[q]; Hr[w][q] = hrn; Hz[w][q] = hzn;
                 }
                 sr = wave_sum_dpp(sr);
                 sz = wave_sum_dpp(sz);
@@ -782,7 +795,20 @@ __global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a
                 load_bins<KPL>(a.J + base, k0, nn, Jcur);
             }
             if (FREQ || SOLVE) {
-                double Fkp[KPL], Fk[KPL], Fkm[KPL];
+                // rows of FrequencyUpdateJLyα! (src/UpdateLyaJandH.jl:200-215) in gtsv form:
+                // dl <- A[2:end], du <- C[1:end-1] (src/TridiagonalSolver.jl:45-46)
+                bool wild = !(dw >= kTameMin);
+                auto put_row = [&](int q, double Fkp, double Fk, double Fkm) {
+                    const int k = k0 + q, row = k - 1;
+                    if (k < 1 || k > nn - 2) return;
+                    if (STOREF) { a.Fkp[base + k] = Fkp; a.Fk[base + k] = Fk; a.Fkm[base + k] = Fkm; }
+                    if (!SOLVE) return;
+                    sD[(size_t)lc * S + row] = -(Fk + dw);
+                    sB[(size_t)lc * S + row] = -dw * Jo[w][q];
+                    if (row >= 1) sDL[(size_t)lc * S + row - 1] = Fkm;
+                    if (row <= n - 2) sDU[(size_t)lc * S + row] = Fkp;
+                    wild |= (row >= 1 && !(fabs(Fkm) >= kTameMin)) || !(fabs(Fkp) + fabs(Fk + dw) + fabs(Fkm) < kTameMax);
+                };
                 if (FREQ) {
                     const double dnuD = a.dnuD ? a.dnuD[c] : 0.0;
                     const double PREFACT = 0.5 * dmax(a.alpha[c], a.alpha_floor) * (dnuD * dnuD);
@@ -793,107 +819,128 @@ __global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a
                     // ϕϕ entries are >= 0): the cell's bins skip the closure, and a bin's exponents
                     // are the same in the three rows it enters
                     const bool still = durdr == 0.0 && durdz == 0.0 && duzdr == 0.0 && duzdz == 0.0 && urr == 0.0;
-                    double VEL[KPL];
+                    auto vel = [&](double J, double hr, double hz) {
+                        if (still) return 0.0;
+                        return D_colon_grad_u(D_edd(hr, hz, J), durdr, durdz, duzdr, duzdz, urr) * kInvC;
+                    };
+                    unsigned redo = 0;   // bins whose factors are infinite or NaN
+                    auto end_row = [&](int q, double Fkp, double Fk, double Fkm) {
+                        if (!(fabs(Fkp) + fabs(Fk) + fabs(Fkm) < 0x1p500)) redo |= 1u << q;
+                        else put_row(q, Fkp, Fk, Fkm);
+                    };
                     // per bin: the recoil drift, the half-widths over K
-                    double S0[KPL], qR[KPL], qL[KPL];
-#pragma unroll
-                    for (int q = 0; q < KPL; ++q) {
+                    auto bin = [&](int q, double& S0, double& qR, double& qL) {
                         const double K = PREFACT * hv[q];
                         const double iK = recip(K);
-                        S0[q] = a.recoil ? K * (RECOIL_0 - two[q]) : -0.0;
-                        qR[q] = hR[q] * iK;
-                        qL[q] = hL[q] * iK;
-                        VEL[q] = 0.0;
-                    }
+                        S0 = a.recoil ? K * (RECOIL_0 - grid_two(q)) : -0.0;
+                        qR = grid_hR(q) * iK;
+                        qL = grid_hL(q) * iK;
+                    };
+                    // The lane's rows in order, each from the terms of its own bin and of the bins beside
+                    // it, which a window of two bins hands on; the lane's first and last bins' terms go to
+                    // the lanes beside it beforehand.  (All bins' terms at once are sixteen registers a
+                    // bin: 256 at three bins per lane, and spills beyond.)
                     if (still) {
                         // rows share what their bins form: A = χL(P) q, exp(-P), χR(P) q, exp(P) over
                         // the right half, χR(P') q' and exp(P') over the left half
-                        double A[KPL], oL[KPL], B[KPL], oR[KPL], Bl[KPL], oRl[KPL];
-#pragma unroll
-                        for (int q = 0; q < KPL; ++q) {
-                            const double C = 0.0 + S0[q];
-                            const double P = dclamp(C * qR[q], -kPmax, kPmax);
-                            const double Pl = dclamp(C * qL[q], -kPmax, kPmax);
+                        auto right = [&](double S0, double qR, double& A, double& oL, double& B, double& oR) {
+                            const double C = 0.0 + S0;
+                            const double P = dclamp(C * qR, -kPmax, kPmax);
                             const double rP = rcp_nr(P);
                             double x;
-                            one_minus_phi<-1>(P, rP, oL[q], x);
-                            A[q] = x * qR[q];
-                            one_minus_phi<1>(P, rP, oR[q], x);
-                            B[q] = x * qR[q];
-                            one_minus_phi<1>(Pl, rcp_nr(Pl), oRl[q], x);
-                            Bl[q] = x * qL[q];
-                        }
-                        const double A_p = prev_lane(A[KPL - 1]), oL_p = prev_lane(oL[KPL - 1]);
-                        const double Bl_n = next_lane(Bl[0]), oRl_n = next_lane(oRl[0]);
+                            one_minus_phi<-1>(P, rP, oL, x);
+                            A = x * qR;
+                            one_minus_phi<1>(P, rP, oR, x);
+                            B = x * qR;
+                        };
+                        auto left = [&](double S0, double qL, double& Bl, double& oRl) {
+                            const double C = 0.0 + S0;
+                            const double Pl = dclamp(C * qL, -kPmax, kPmax);
+                            double x;
+                            one_minus_phi<1>(Pl, rcp_nr(Pl), oRl, x);
+                            Bl = x * qL;
+                        };
+                        double S0, qR, qL, Bl, oRl, A_e, oL_e, B_e, oR_e;
+                        bin(KPL - 1, S0, qR, qL);
+                        right(S0, qR, A_e, oL_e, B_e, oR_e);
+                        if (KPL > 1) bin(0, S0, qR, qL);
+                        left(S0, qL, Bl, oRl);
+                        double Am = prev_lane(A_e), oLm = prev_lane(oL_e);
+                        const double Bl_n = next_lane(Bl), oRl_n = next_lane(oRl);
 #pragma unroll
                         for (int q = 0; q < KPL; ++q) {
-                            const double Am = q > 0 ? A[q > 0 ? q - 1 : 0] : A_p, oLm = q > 0 ? oL[q > 0 ? q - 1 : 0] : oL_p;
-                            const double Bp = q + 1 < KPL ? Bl[q + 1 < KPL ? q + 1 : 0] : Bl_n;
-                            const double oRp = q + 1 < KPL ? oRl[q + 1 < KPL ? q + 1 : 0] : oRl_n;
-                            const double den_kp = idn[q] * recip(A[q] - Bp);
-                            const double den_km = idn[q] * recip(Am - B[q]);
-                            Fkp[q] = oRp * den_kp;
-                            Fkm[q] = oLm * den_km;
-                            Fk[q] = oL[q] * den_kp + oR[q] * den_km;
+                            double A = A_e, oL = oL_e, B = B_e, oR = oR_e, Bp = Bl_n, oRp = oRl_n;
+                            if (q + 1 < KPL) {
+                                right(S0, qR, A, oL, B, oR);
+                                bin(q + 1, S0, qR, qL);
+                                left(S0, qL, Bp, oRp);
+                            }
+                            const double den_kp = grid_idn(q) * recip(A - Bp);
+                            const double den_km = grid_idn(q) * recip(Am - B);
+                            end_row(q, oRp * den_kp, oL * den_kp + oR * den_km, oLm * den_km);
+                            Am = A;
+                            oLm = oL;
                         }
                     } else {
                         // every row with its own bin's VEL in the exponents of its three bins
-                        const double S_p = prev_lane(S0[KPL - 1]), qR_p = prev_lane(qR[KPL - 1]);
-                        const double S_n = next_lane(S0[0]), qL_n = next_lane(qL[0]);
+                        double S0, qR, qL, S_e, qR_e;
+                        bin(KPL - 1, S_e, qR_e, qL);
+                        S0 = S_e;
+                        qR = qR_e;
+                        if (KPL > 1) bin(0, S0, qR, qL);
+                        double Sm = prev_lane(S_e), qm = prev_lane(qR_e);
+                        const double S_n = next_lane(S0), qL_n = next_lane(qL);
 #pragma unroll
                         for (int q = 0; q < KPL; ++q) {
                             const int k = min(max(k0 + q, 1), nn - 2);
-                            const Edd D = D_edd(Hr[w][q], Hz[w][q], Jcur[q]);
-                            VEL[q] = D_colon_grad_u(D, durdr, durdz, duzdr, duzdz, urr) * kInvC;
-                            const double Sm = q > 0 ? S0[q > 0 ? q - 1 : 0] : S_p, qm = q > 0 ? qR[q > 0 ? q - 1 : 0] : qR_p;
-                            const double Sp = q + 1 < KPL ? S0[q + 1 < KPL ? q + 1 : 0] : S_n;
-                            const double qp = q + 1 < KPL ? qL[q + 1 < KPL ? q + 1 : 0] : qL_n;
-                            const double Pkp = dclamp((VEL[q] * a.nuC[k + 1] + Sp) * qp, -kPmax, kPmax);
-                            const double Pk = dclamp((VEL[q] * a.nuC[k] + S0[q]) * qR[q], -kPmax, kPmax);
-                            const double Pkm = dclamp((VEL[q] * a.nuC[k - 1] + Sm) * qm, -kPmax, kPmax);
+                            double Sp = S_n, qp = qL_n, qRp = qR;
+                            if (q + 1 < KPL) bin(q + 1, Sp, qRp, qp);
+                            const double VEL = vel(EMIT ? Jo[w][q] : Jcur[q], Hr[w][q], Hz[w][q]);
+                            const double Pkp = dclamp((VEL * a.nuC[k + 1] + Sp) * qp, -kPmax, kPmax);
+                            const double Pk = dclamp((VEL * a.nuC[k] + S0) * qR, -kPmax, kPmax);
+                            const double Pkm = dclamp((VEL * a.nuC[k - 1] + Sm) * qm, -kPmax, kPmax);
                             double oRkp, xRkp, oLk, xLk, oRk, xRk, oLkm, xLkm;
                             const double rPk = rcp_nr(Pk);
                             one_minus_phi<1>(Pkp, rcp_nr(Pkp), oRkp, xRkp);
                             one_minus_phi<-1>(Pk, rPk, oLk, xLk);
                             one_minus_phi<1>(Pk, rPk, oRk, xRk);
                             one_minus_phi<-1>(Pkm, rcp_nr(Pkm), oLkm, xLkm);
-                            const double den_kp = idn[q] * recip(xLk * qR[q] - xRkp * qp);
-                            const double den_km = idn[q] * recip(xLkm * qm - xRk * qR[q]);
-                            Fkp[q] = oRkp * den_kp;
-                            Fkm[q] = oLkm * den_km;
-                            Fk[q] = oLk * den_kp + oRk * den_km;
+                            const double den_kp = grid_idn(q) * recip(xLk * qR - xRkp * qp);
+                            const double den_km = grid_idn(q) * recip(xLkm * qm - xRk * qR);
+                            end_row(q, oRkp * den_kp, oLk * den_kp + oRk * den_km, oLkm * den_km);
+                            Sm = S0;
+                            qm = qR;
+                            S0 = Sp;
+                            qR = qRp;
                         }
                     }
+                    redo &= k0 > 0 ? ~0u : ~1u;
+                    if (k0 + KPL > nn - 1) redo &= k0 < nn - 1 ? (1u << (nn - 1 - k0)) - 1 : 0u;
+                    // infinite or NaN factors: the row again in the general form
+                    if (__builtin_expect(redo != 0, 0)) {
+#pragma unroll 1
+                        for (int q = 0; q < KPL; ++q) {
+                            const int k = k0 + q;
+                            if (!(redo >> q & 1)) continue;
+                            double J = 0.0, hr = 0.0, hz = 0.0;
 #pragma unroll
-                    for (int q = 0; q < KPL; ++q) {
-                        const int k = k0 + q;
-                        // infinite or NaN factors: the row again in the general form
-                        if (__builtin_expect(k >= 1 && k <= nn - 2 && !(fabs(Fkp[q]) + fabs(Fk[q]) + fabs(Fkm[q]) < 0x1p500), 0))
-                            freq_row_general(a, base + k, k, VEL[q], PREFACT, RECOIL_0, Fkp[q], Fk[q], Fkm[q]);
-                        if (STOREF && k >= 1 && k <= nn - 2) {
-                            a.Fkp[base + k] = Fkp[q]; a.Fk[base + k] = Fk[q]; a.Fkm[base + k] = Fkm[q];
+                            for (int m = 0; m < KPL; ++m)
+                                if (m == q) { J = EMIT ? Jo[w][m] : Jcur[m]; hr = Hr[w][m]; hz = Hz[w][m]; }
+                            double Fkp, Fk, Fkm;
+                            freq_row_general(a, base + k, k, vel(J, hr, hz), PREFACT, RECOIL_0, Fkp, Fk, Fkm);
+#pragma unroll
+                            for (int m = 0; m < KPL; ++m)
+                                if (m == q) put_row(m, Fkp, Fk, Fkm);
                         }
                     }
                 } else {
-                    load_bins<KPL>(a.Fkp + base, k0, nn, Fkp);
-                    load_bins<KPL>(a.Fk + base, k0, nn, Fk);
-                    load_bins<KPL>(a.Fkm + base, k0, nn, Fkm);
-                }
-                if (SOLVE) {
-                    // rows of FrequencyUpdateJLyα! (src/UpdateLyaJandH.jl:200-215) in gtsv form:
-                    // dl <- A[2:end], du <- C[1:end-1] (src/TridiagonalSolver.jl:45-46)
-                    bool wild = !(dw >= kTameMin);
 #pragma unroll
                     for (int q = 0; q < KPL; ++q) {
-                        const int k = k0 + q, row = k - 1;
-                        if (k < 1 || k > nn - 2) continue;
-                        sD[(size_t)lc * S + row] = -(Fk[q] + dw);
-                        sB[(size_t)lc * S + row] = -dw * Jo[w][q];
-                        if (row >= 1) sDL[(size_t)lc * S + row - 1] = Fkm[q];
-                        if (row <= n - 2) sDU[(size_t)lc * S + row] = Fkp[q];
-                        wild |= (row >= 1 && !(fabs(Fkm[q]) >= kTameMin)) ||
-                                !(fabs(Fkp[q]) + fabs(Fk[q] + dw) + fabs(Fkm[q]) < kTameMax);
+                        const int k = k0 + q;
+                        if (k >= 1 && k <= nn - 2) put_row(q, a.Fkp[base + k], a.Fk[base + k], a.Fkm[base + k]);
                     }
+                }
+                if (SOLVE) {
                     const bool any_wild = __any(wild);
                     if (lane == 0) s_wild[lc] = any_wild;
                 }
@@ -954,15 +1001,16 @@ __global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a
             const int i = c % nr, j = c / nr;
             const double dV = a.dV ? a.dV[c] : 0.0;
             double jn[KPL], Js[KPL], esc = 0.0;
-            if (KPL > 2) load_grid(false);
             const bool edge = FUSED && (i == nr - 1 || j == nz - 1 || (j == 0 && a.bc_z_bot == BC_OUTFLOW));
-            if (SOLVE && !FUSED) load_bins<KPL>(a.J + base, k0, nn, jn);
             if (FUSED && CONV) load_bins<KPL>(a.J_old + base, k0, nn, Js);
 #pragma unroll
             for (int q = 0; q < KPL; ++q) {
                 const int k = k0 + q;
-                if (!(SOLVE && !FUSED) || k >= nn) jn[q] = Jo[w][q];
-                if (SOLVE && k >= 1 && k <= nn - 2) jn[q] = sB[(size_t)lc * S + (k - 1)];
+                jn[q] = Jo[w][q];
+                if (SOLVE) {
+                    if (k >= 1 && k <= nn - 2) jn[q] = sB[(size_t)lc * S + (k - 1)];
+                    else if (!FUSED && k < nn) jn[q] = a.J[base + k];
+                }
                 double hr = Hr[w][q], hz = Hz[w][q];
                 // the floor below would hide a NaN in J (max(NaN, Jeps) = Jeps): test first
                 if (FUSED && k < nn) bad += !(__builtin_isfinite(jn[q]) && __builtin_isfinite(hr) && __builtin_isfinite(hz));
@@ -984,14 +1032,14 @@ __global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a
                 }
                 Hr[w][q] = hr; Hz[w][q] = hz;
                 if (FUSED && k < nn) {
-                    if (CONV) conv += dnu[q] * fabs(jn[q] - Js[q]) * dV;
-                    e1[q] += dnu[q] * dmax(jn[q] - kJeps, 0.0) * dV;
-                    e10[q] += dnu[q] * dmax(jn[q] - 10 * kJeps, 0.0) * dV;
+                    if (CONV) conv += grid_dnu(q) * fabs(jn[q] - Js[q]) * dV;
+                    e1[q] += grid_dnu(q) * dmax(jn[q] - kJeps, 0.0) * dV;
+                    e10[q] += grid_dnu(q) * dmax(jn[q] - 10 * kJeps, 0.0) * dV;
                     // Compute_f_esc_Cylindrical terms (src/ConstantsAndFunctions.jl:937-953)
                     if (edge) {
-                        if (i == nr - 1) esc += dnu[q] * (a.A_r[(size_t)j * (nr + 1) + nr] * kFourPi * dmax(hr, 0.0));
-                        if (j == nz - 1) esc += dnu[q] * (a.A_z[(size_t)nz * nr + i] * kFourPi * dmax(hz, 0.0));
-                        if (j == 0 && a.bc_z_bot == BC_OUTFLOW) esc += dnu[q] * (a.A_z[i] * kFourPi * dmax(-hz, 0.0));
+                        if (i == nr - 1) esc += grid_dnu(q) * (a.A_r[(size_t)j * (nr + 1) + nr] * kFourPi * dmax(hr, 0.0));
+                        if (j == nz - 1) esc += grid_dnu(q) * (a.A_z[(size_t)nz * nr + i] * kFourPi * dmax(hz, 0.0));
+                        if (j == 0 && a.bc_z_bot == BC_OUTFLOW) esc += grid_dnu(q) * (a.A_z[i] * kFourPi * dmax(-hz, 0.0));
                     }
                 }
             }
@@ -1030,6 +1078,55 @@ __global__ __launch_bounds__(64 * NW, NW > 1 ? 2 : 1) void k_column(ColumnArgs a
 #pragma unroll
             for (int w = 1; w < NW; ++w) v += lds[(size_t)w * ncol + t];
             prow[t] = v;
+        }
+    }
+}
+
+// Emission / absorption alone, or the frequency factors alone, above 256 bins: lanes over bins, one
+// wavefront per cell.  Without a solve no lane needs its neighbours' terms, and k_column's
+// consecutive bins per lane (up to nine) cost a cache line per bin and lane.  45x61x542 at rest:
+// emission 28.6 us, 69 by k_column; factors 23 us, 65.
+__global__ __launch_bounds__(256) void k_bins(ColumnArgs a)
+{
+    const int nn = a.nn, ncells = a.nr * a.nz;
+    const int lane = threadIdx.x & 63;
+    const int c = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (c >= ncells) return;
+    const size_t base = (size_t)c * nn;
+    if (a.flags & COL_EMIT) {
+        const double ct = a.c_tilde, dt = a.dt, inv_ct = 1.0 / ct, fpc_ict = (kFourPi / kC) * inv_ct;
+        const double ac = a.alpha_c[c], al_pd = a.alpha[c] * a.pd[c], js_ct = a.js[c] * ct;
+        double sr = 0.0, sz = 0.0;
+        for (int k = lane; k < nn; k += 64) {
+            const size_t idx = base + k;
+            const double hr = a.Hr[idx], hz = a.Hz[idx];
+            double J = a.J_old[idx], hrn = hr, hzn = hz;
+            absorb(ac + al_pd * a.Hv[idx], js_ct * a.phi[idx], a.aF[idx], ct, dt, J, hrn, hzn);
+            sr += a.dnu[k] * (hr - hrn);
+            sz += a.dnu[k] * (hz - hzn);
+            a.J[idx] = J; a.Hr[idx] = hrn; a.Hz[idx] = hzn;
+            a.J_old[idx] = J; a.Hr_old[idx] = hrn; a.Hz_old[idx] = hzn;
+        }
+        sr = wave_sum_dpp(sr);
+        sz = wave_sum_dpp(sz);
+        if (lane == 0) {
+            a.drhou_r[c] += fpc_ict * sr;
+            a.drhou_z[c] += fpc_ict * sz;
+        }
+    }
+    if (a.flags & COL_FREQ) {
+        const double dnuD = a.dnuD[c], PREFACT = 0.5 * dmax(a.alpha[c], a.alpha_floor) * (dnuD * dnuD);
+        const double RECOIL_0 = kHoverKB / a.T[c];
+        const double durdr = a.dur_dr[c], durdz = a.dur_dz[c], duzdr = a.duz_dr[c], duzdz = a.duz_dz[c];
+        const double urr = a.ur_over_r[c];
+        const bool still = durdr == 0.0 && durdz == 0.0 && duzdr == 0.0 && duzdz == 0.0 && urr == 0.0;
+        for (int k = lane; k < nn; k += 64) {
+            if (k < 1 || k > nn - 2) continue;
+            const size_t idx = base + k;
+            double VEL = 0.0;
+            if (!still)
+                VEL = D_colon_grad_u(D_edd(a.Hr[idx], a.Hz[idx], a.J[idx]), durdr, durdz, duzdr, duzdz, urr) * kInvC;
+            freq_row_general(a, idx, k, VEL, PREFACT, RECOIL_0, a.Fkp[idx], a.Fk[idx], a.Fkm[idx]);
         }
     }
 }
@@ -1259,12 +1356,18 @@ void launch_advect(hipStream_t s, const AdvectArgs& a)
     hipLaunchKernelGGL((k_advect<WPB>), grid, dim3(64 * WPB), 0, s, a, seg);
 }
 
+// Dynamic LDS of a k_column block: the rows of its columns, and after them each wavefront's sums.
+static size_t column_lds(int nn, int w, int nw)
+{
+    const size_t rows = 5 * (size_t)col_stride(nn) * w * nw + 2 * kColPad;
+    const size_t sums = (size_t)nw * (2 * nn + kStepSums);
+    return std::max(rows, sums) * sizeof(double);
+}
+
 template <int W, int KPL, int NW>
 static void launch_column_t(hipStream_t s, const ColumnArgs& a, int nblocks)
 {
-    const size_t rows = 5 * (size_t)col_stride(a.nn) * W * NW + 2 * kColPad;
-    const size_t sums = (size_t)NW * (2 * a.nn + kStepSums);
-    const size_t lds = std::max(rows, sums) * sizeof(double);
+    const size_t lds = column_lds(a.nn, W, NW);
     if ((a.flags & ~COL_CONV) == kFusedFlags)
         hipLaunchKernelGGL((k_column<W, KPL, NW, true>), dim3(nblocks), dim3(64 * NW), lds, s, a);
     else
@@ -1274,11 +1377,11 @@ static void launch_column_t(hipStream_t s, const ColumnArgs& a, int nblocks)
 ColumnShape column_shape(int nn, size_t ncells)
 {
     ColumnShape c;
-    c.nw = nn <= 256 ? 4 : 1;
+    c.nw = nn <= 512 ? 4 : 3;
     c.w = nn <= 128 ? kColumnW : (nn <= 256 ? 2 : 1);
-    while (c.w > 1 && ncells < (size_t)c.w * c.nw * 512) c.w /= 2;
+    while (c.w > 1 && ncells < (size_t)c.w * c.nw * kColumnBlocks) c.w /= 2;
     const size_t groups = (ncells + (size_t)c.w * c.nw - 1) / ((size_t)c.w * c.nw);
-    c.blocks = (int)std::max<size_t>(1, std::min<size_t>(groups, (size_t)kColumnBlocks / c.nw));
+    c.blocks = (int)std::max<size_t>(1, std::min<size_t>(groups, kColumnBlocks));
     return c;
 }
 
@@ -1294,16 +1397,20 @@ static void launch_column_w(hipStream_t s, const ColumnArgs& a, const ColumnShap
 
 void launch_column(hipStream_t s, const ColumnArgs& a, const ColumnShape& c)
 {
+    if (a.nn > 64 * kBinsPerLaneAll && !(a.flags & COL_SOLVE)) {
+        hipLaunchKernelGGL(k_bins, dim3((a.nr * a.nz + 3) / 4), dim3(256), 0, s, a);
+        return;
+    }
     switch ((a.nn + 63) / 64) {
     case 1: launch_column_w<1>(s, a, c); break;
     case 2: launch_column_w<2>(s, a, c); break;
     case 3: launch_column_w<3>(s, a, c); break;
     case 4: launch_column_w<4>(s, a, c); break;
-    case 5: launch_column_t<1, 5, 1>(s, a, c.blocks); break;
-    case 6: launch_column_t<1, 6, 1>(s, a, c.blocks); break;
-    case 7: launch_column_t<1, 7, 1>(s, a, c.blocks); break;
-    case 8: launch_column_t<1, 8, 1>(s, a, c.blocks); break;
-    default: launch_column_t<1, 9, 1>(s, a, c.blocks); break;
+    case 5: launch_column_t<1, 5, 4>(s, a, c.blocks); break;
+    case 6: launch_column_t<1, 6, 4>(s, a, c.blocks); break;
+    case 7: launch_column_t<1, 7, 4>(s, a, c.blocks); break;
+    case 8: launch_column_t<1, 8, 4>(s, a, c.blocks); break;
+    default: launch_column_t<1, 9, 3>(s, a, c.blocks); break;
     }
 }
 
