@@ -4,11 +4,10 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include "m1lya_device.h"
+#include "m1lya_shape.h"
 
 namespace m1 {
 
-// Most cell columns per wavefront in the column kernel (lane-per-column dgtsv).
-constexpr int kColumnW = 4;
 // Largest N_ν of the FP64 context (nine bins per lane in the column kernel).
 constexpr int kMaxBinsFP64 = 576;
 constexpr int kMaxBinsAdjoint = 256;
@@ -234,27 +233,6 @@ void launch_reduce_cols(hipStream_t s, const double* part, int nrows, int stride
                         const int* halt = nullptr);
 void launch_active_final(hipStream_t s, const double* red, int nn, int kcmin, int kcmax, int* krange);
 void launch_advect(hipStream_t s, const AdvectArgs& a);
-// Shape of the column kernel's launch: w cell columns per wavefront, nw wavefronts per block
-// (the block shares its dgtsv phase), blocks of the grid.  It depends on the grid's dimensions
-// alone, so that the partition of the fused reductions, and with it their bits, does not depend
-// on the device.
-//
-// A column takes five arrays of N_ν-2 rows of LDS, and the w·nw columns of a block as many as leave
-// room for two blocks in a CU's 160 KB: 81 KB for 16 columns of 128 bins, 82 KB for 8 of 256 and for
-// 4 of 512, 69 KB for 3 of 576.  Blocks of several wavefronts above 256 bins too: a column's solve
-// is a chain that takes a wavefront's issue slots however few of its lanes solve, so that eight
-// one-wavefront blocks on a CU ran two chains on each SIMD (870 cycles a row, 380 for a chain alone).
-// 45x61x320: 158 us, 265 by one-wavefront blocks; 128x128x542: 1.49 ms, 1.90 by one-wavefront
-// blocks that spread the bins of a wavefront and shared no term between rows.
-//
-// The grid is at most one wave of resident blocks (two per CU at 256 VGPRs), which loop over the
-// column groups: a larger one left a partial second wave starting late.  While fewer cells than one
-// such wave holds are there, w is halved, so that the columns spread over more blocks.
-constexpr int kColumnBlocks = 512;
-struct ColumnShape {
-    int w, nw, blocks;
-};
-ColumnShape column_shape(int nn, size_t ncells);
 void launch_column(hipStream_t s, const ColumnArgs& a, const ColumnShape& c);
 // Step scalars {M_F, net, out, L, f_esc, kmin, kmax, ΔJ/J}; ΔJ/J is 0 unless the column
 // kernel ran with COL_CONV.  ctl may be null (no halt, no count); tol > 0 sets ctl->halt

@@ -1374,17 +1374,6 @@ static void launch_column_t(hipStream_t s, const ColumnArgs& a, int nblocks)
         hipLaunchKernelGGL((k_column<W, KPL, NW, false>), dim3(nblocks), dim3(64 * NW), lds, s, a);
 }
 
-ColumnShape column_shape(int nn, size_t ncells)
-{
-    ColumnShape c;
-    c.nw = nn <= 512 ? 4 : 3;
-    c.w = nn <= 128 ? kColumnW : (nn <= 256 ? 2 : 1);
-    while (c.w > 1 && ncells < (size_t)c.w * c.nw * kColumnBlocks) c.w /= 2;
-    const size_t groups = (ncells + (size_t)c.w * c.nw - 1) / ((size_t)c.w * c.nw);
-    c.blocks = (int)std::max<size_t>(1, std::min<size_t>(groups, kColumnBlocks));
-    return c;
-}
-
 template <int KPL>
 static void launch_column_w(hipStream_t s, const ColumnArgs& a, const ColumnShape& c)
 {
