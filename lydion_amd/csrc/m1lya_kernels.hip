@@ -824,6 +824,9 @@ __global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
                         return D_colon_grad_u(D_edd(hr, hz, J), durdr, durdz, duzdr, duzdz, urr) * kInvC;
                     };
                     unsigned redo = 0;   // bins whose factors are infinite or NaN
+                    double VELs[kGrid];  // up to two bins per lane: kept for the rows formed again
+#pragma unroll
+                    for (int q = 0; q < kGrid; ++q) VELs[q] = 0.0;
                     auto end_row = [&](int q, double Fkp, double Fk, double Fkm) {
                         if (!(fabs(Fkp) + fabs(Fk) + fabs(Fkm) < 0x1p500)) redo |= 1u << q;
                         else put_row(q, Fkp, Fk, Fkm);
@@ -896,6 +899,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
                             double Sp = S_n, qp = qL_n, qRp = qR;
                             if (q + 1 < KPL) bin(q + 1, Sp, qRp, qp);
                             const double VEL = vel(EMIT ? Jo[w][q] : Jcur[q], Hr[w][q], Hz[w][q]);
+                            if (kKeep) VELs[kKeep ? q : 0] = VEL;
                             const double Pkp = dclamp((VEL * a.nuC[k + 1] + Sp) * qp, -kPmax, kPmax);
                             const double Pk = dclamp((VEL * a.nuC[k] + S0) * qR, -kPmax, kPmax);
                             const double Pkm = dclamp((VEL * a.nuC[k - 1] + Sm) * qm, -kPmax, kPmax);
@@ -922,12 +926,16 @@ __global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
                         for (int q = 0; q < KPL; ++q) {
                             const int k = k0 + q;
                             if (!(redo >> q & 1)) continue;
-                            double J = 0.0, hr = 0.0, hz = 0.0;
+                            double VEL = 0.0, J = 0.0, hr = 0.0, hz = 0.0;
 #pragma unroll
-                            for (int m = 0; m < KPL; ++m)
-                                if (m == q) { J = EMIT ? Jo[w][m] : Jcur[m]; hr = Hr[w][m]; hz = Hz[w][m]; }
+                            for (int m = 0; m < KPL; ++m) {
+                                if (m != q) continue;
+                                if (kKeep) VEL = VELs[kKeep ? m : 0];
+                                else { J = EMIT ? Jo[w][m] : Jcur[m]; hr = Hr[w][m]; hz = Hz[w][m]; }
+                            }
+                            if (!kKeep) VEL = vel(J, hr, hz);
                             double Fkp, Fk, Fkm;
-                            freq_row_general(a, base + k, k, vel(J, hr, hz), PREFACT, RECOIL_0, Fkp, Fk, Fkm);
+                            freq_row_general(a, base + k, k, VEL, PREFACT, RECOIL_0, Fkp, Fk, Fkm);
 #pragma unroll
                             for (int m = 0; m < KPL; ++m)
                                 if (m == q) put_row(m, Fkp, Fk, Fkm);
