@@ -1119,9 +1119,11 @@ __device__ __forceinline__ void step_block(const Cloud* __restrict__ clouds, con
     }
 }
 
-// The step of the blocks [blk0, blk1) of the batch.
+// The step of the blocks [blk0, blk1) of the batch.  Two cells per wavefront at rest fit in 96 VGPRs,
+// so that five of the wavefronts of blocks of four (or fewer) share a SIMD: 32 clouds of 128x128x32
+// in tiles of 16x4, 523 us, 594 at 97 VGPRs and four.
 template <bool kShear, int NQ, bool kPair>
-__global__ __launch_bounds__(64 * kMaxWaves, NQ <= 2 ? 4 : 2) void k_step(const Cloud* __restrict__ clouds, Arrays A,
+__global__ __launch_bounds__(64 * kMaxWaves, NQ > 2 ? 2 : kPair && !kShear ? 5 : 4) void k_step(const Cloud* __restrict__ clouds, Arrays A,
                                                             const Seg* __restrict__ segs, int blk0, int blk1,
                                                             int wpb, int parity, int rows,
                                                             const int* __restrict__ krange,
@@ -1687,9 +1689,9 @@ int auto_segment(const m1lya_batch* b, bool pair)
 }
 
 // Work tables.  Per cloud, row segments of one length, wpb of them (same i range, consecutive
-// rows) per block; blocks never mix clouds.  The blocks of clouds in pair mode come first: they are
-// launched on their own.  With segments of the caller's choice, or of the default length, a block
-// is a partial row of its cloud; else the rows are those of the default tiles.
+// rows) per block; blocks never mix clouds.  The blocks of clouds in pair mode come first.  With
+// segments of the caller's choice, or of the default length, a block is a partial row of its cloud;
+// else the rows are those of the default tiles.
 void build_tiles(m1lya_batch* b)
 {
     std::vector<int> order;
@@ -1849,13 +1851,30 @@ void collect_stats(m1lya_batch* b)
     b->pending.clear();
 }
 
+// Whether one launch takes both kinds of blocks.  It saves the first kind's last, partial round of
+// blocks.  But in it the blocks of two cells per wavefront get the registers and the LDS of the
+// others, so that with fewer than eight wavefronts per block fewer of them are resident (per CU, of
+// 4, 2 and 1 wavefronts: 4, 6 and 8 instead of 5, 10 and 16).  Apart once that costs more than one
+// and a half rounds of them: over sweeps of 4 to 64 clouds in tiles of 8 to 32 cells by 1 to 8 rows,
+// together saves up to 31 % below that, apart up to 34 % above (32 clouds of 128x128x32 and one of
+// 64x64x64 in tiles of 16x1: 793 us, 1192 together).  Clouds of more than 128 bins, whose blocks
+// leave room for half as many wavefronts, have their own launch; so has each kind when launches are
+// timed.
+bool step_mixed(const m1lya_batch* b)
+{
+    if (b->nblk_pair == 0 || b->nblk == b->nblk_pair || b->wide || b->profiling) return false;
+    auto resident = [&](int waves, int nq) {
+        return (double)std::min<size_t>(waves / b->wpb, (160 << 10) / step_lds_bytes(b->wpb, nq));
+    };
+    const double lost = 1.0 / resident(16, 2) - 1.0 / resident(b->shear ? 16 : 20, 1);
+    return (double)b->nblk_pair / 256.0 * lost <= 1.5;
+}
+
 void launch_step_kernels(m1lya_batch* b, int parity)
 {
     hipStream_t s = b->stream;
     const dim3 block(64 * b->wpb);
-    // both kinds of blocks share a launch (clouds of more than 128 bins, whose blocks leave room for
-    // half as many wavefronts, have their own; so has each kind when launches are timed)
-    if (b->nblk_pair > 0 && b->nblk > b->nblk_pair && !b->wide && !b->profiling) {
+    if (step_mixed(b)) {
         const int grid0 = (b->nblk - b->nblk_pair + 7) / 8 * 8;
         const dim3 grid(grid0 + (b->nblk_pair + 7) / 8 * 8);
         const size_t lds = std::max(step_lds_bytes(b->wpb, 1), step_lds_bytes(b->wpb, 2));

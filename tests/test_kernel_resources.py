@@ -44,3 +44,10 @@ def test_column_kernel_keeps_two_wavefronts_per_simd(kernels):
         # a few spilled registers at eight and nine bins per lane, next to none below
         wide = re.search(r"k_columnILi1ELi[89]", k)
         assert scratch <= (256 if wide else 72), (k, scratch)
+
+
+def test_paired_step_keeps_five_wavefronts_per_simd(kernels):
+    """Two cells per wavefront, no sheared gradients: tiles of four rows and fewer rely on 512 / 5
+    registers, in units of eight."""
+    pair = [v for k, v in kernels.items() if "k_stepILb0ELi1ELb1E" in k]
+    assert pair and all(vgprs <= 96 and scratch == 0 for vgprs, scratch in pair), pair
