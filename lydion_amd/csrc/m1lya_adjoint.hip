@@ -552,11 +552,10 @@ __global__ __launch_bounds__(256, 2) void k_adj_march(AdjAdvArgs a, int seg)
 }
 
 // The same sums for grids too small to march over: a block of eight wavefronts takes the
-// kTileFaces interfaces around kTileFaces - 3 cells of a line, two interfaces a wavefront, and the
-// cells gather their slots from LDS in the order of the march (the results have the same bits).
-// 45x61x64, both directions: 40 us, 58 by marches, 49 by way of memory.
-constexpr int kTileFaces = 16, kTileWaves = 8;
-
+// interfaces around the seg <= kTileFaces - 3 cells of a part of a line, at most two interfaces a
+// wavefront, and the cells gather their slots from LDS in the order of the march (the results have the same bits).
+// 45x61x64, both directions: 40 us, 58 by marches, 49 by way of memory; 24x24x32 by five cells a
+// block, both directions and k_adj_cell: 37 us, 51 by thirteen.
 template <int DIR, bool HLL>
 __global__ __launch_bounds__(64 * kTileWaves, 2) void k_adj_tile(AdjAdvArgs a, int seg)
 {
@@ -1057,36 +1056,21 @@ void launch_adj_column(hipStream_t s, const AdjColArgs& a)
     else hipLaunchKernelGGL(k_adj_column<1>, dim3(ncell), dim3(64), lds, s, a);
 }
 
-// The interfaces of one direction.  In units of one interface by a wavefront that has its SIMD to
-// itself (4.3 us; two at a time take 1.28), a march takes its segment's cells, three interfaces more
-// and about one to start, on the wavefronts a SIMD gets (256 VGPRs allow two at a time); a block of
-// k_adj_tile takes two pairs of interfaces and 0.8 for its sums, one block to a CU, and the launch one
-// to start.  The least estimated time: on 128x128x128 the march by 16 cells (r: estimated 110 us,
-// measured 117; tiles 150), on 45x61x64 the tiles (19 us, 19; the march 28).
+// The interfaces of one direction.
 template <int DIR>
 static void launch_adj_faces(hipStream_t s, const AdjAdvArgs& a)
 {
-    constexpr int kCUs = 256, kSimds = 4 * kCUs, kSegMax = 32;
-    const int n = DIR == 0 ? a.g.nr : a.g.nz, lines = DIR == 0 ? a.g.nz : a.g.nr;
-    const int chunks = (a.nn + 63) / 64, groups = (lines + 3) / 4;
-    int seg = kSegMax;
-    double best = 0.0;
-    for (int t = kSegMax; t >= 1; --t) {
-        const long per_simd = ((long)chunks * groups * 4 * ((n + t - 1) / t) + kSimds - 1) / kSimds;
-        const double cost = (1.28 * (double)(per_simd / 2) + (double)(per_simd % 2)) * (t + 4);
-        if (t == kSegMax || cost < best) { best = cost; seg = t; }
-    }
-    const int tiles = (n + kTileFaces - 4) / (kTileFaces - 3), tile_seg = (n + tiles - 1) / tiles;
-    const long per_cu = ((long)chunks * lines * tiles + kCUs - 1) / kCUs;
-    if (3.36 * (double)per_cu + 1.0 < best) {
-        const dim3 grid(chunks, lines, tiles), block(64, kTileWaves);
-        if (a.hll) hipLaunchKernelGGL((k_adj_tile<DIR, true>), grid, block, 0, s, a, tile_seg);
-        else hipLaunchKernelGGL((k_adj_tile<DIR, false>), grid, block, 0, s, a, tile_seg);
+    const int n = DIR == 0 ? a.g.nr : a.g.nz, lines = DIR == 0 ? a.g.nz : a.g.nr, chunks = (a.nn + 63) / 64;
+    const FaceShape f = face_shape(a.nn, n, lines, a.hll != 0);
+    if (f.tile) {
+        const dim3 grid(chunks, lines, (n + f.seg - 1) / f.seg), block(64, kTileWaves);
+        if (a.hll) hipLaunchKernelGGL((k_adj_tile<DIR, true>), grid, block, 0, s, a, f.seg);
+        else hipLaunchKernelGGL((k_adj_tile<DIR, false>), grid, block, 0, s, a, f.seg);
         return;
     }
-    const dim3 grid(chunks, groups, (n + seg - 1) / seg), block(64, 4);
-    if (a.hll) hipLaunchKernelGGL((k_adj_march<DIR, true>), grid, block, 0, s, a, seg);
-    else hipLaunchKernelGGL((k_adj_march<DIR, false>), grid, block, 0, s, a, seg);
+    const dim3 grid(chunks, (lines + 3) / 4, (n + f.seg - 1) / f.seg), block(64, 4);
+    if (a.hll) hipLaunchKernelGGL((k_adj_march<DIR, true>), grid, block, 0, s, a, f.seg);
+    else hipLaunchKernelGGL((k_adj_march<DIR, false>), grid, block, 0, s, a, f.seg);
 }
 
 void launch_adj_advect(hipStream_t s, const AdjAdvArgs& a)

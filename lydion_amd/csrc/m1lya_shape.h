@@ -1,5 +1,5 @@
-// m1lya_shape.h -- launch shape of the FP64 column kernel, from the grid's dimensions alone (host
-// arithmetic, no device code).
+// m1lya_shape.h -- launch shapes of the FP64 column kernel and of the reverse interfaces, from the
+// grid's dimensions and the flux method alone (host arithmetic, no device code).
 #pragma once
 #include <algorithm>
 #include <cstddef>
@@ -48,6 +48,47 @@ inline ColumnShape column_shape(int nn, size_t ncells)
     while (c.w > 1 && groups(c.w / 2) <= limit(c.w / 2)) c.w /= 2;
     c.blocks = (int)std::max<size_t>(1, std::min<size_t>(groups(c.w), kColumnBlocks));
     return c;
+}
+
+// Shape of the reverse interfaces along one direction (n cells on each of `lines` lines): blocks of
+// kTileWaves wavefronts that take the interfaces around seg cells (k_adj_tile), or wavefronts that
+// march over seg cells (k_adj_march).  The least estimated time, in units of one interface by a
+// wavefront that has its SIMD to itself (4.3 us by GLF).  A march takes its segment's cells, three
+// interfaces more and about one to start, on the wavefronts a SIMD gets (256 VGPRs allow two at a
+// time, in 1.28 times one's time).  A tile takes 2.2 where each of its wavefronts takes one interface
+// and 3.7 where it takes two, one block to a CU; its rounds of blocks count half by their number and
+// half by the work in them, and its launch takes one.  HLL makes an interface of a tile 1.2 times as long and one of a march,
+// which spills there, 1.47 times.
+// Both directions and the cells' own kernel, us, tiles / marches (the better seg of each), GLF and HLL:
+// 24x24x32 37 / 56, 43 / 71; 45x61x64 64 / 84, 75 / 115; 56x56x64 79 / 87, 93 / 117; 80x80x64 128 /
+// 132, 152 / 182; 63x64x128 147 / 136, 177 / 190; 128x96x64 202 / 182, 242 / 254; 100x110x128 331 /
+// 283, 391 / 396; 128x128x128 494 / 391, 581 / 550.
+constexpr int kTileFaces = 16, kTileWaves = 8;
+
+struct FaceShape {
+    bool tile;
+    int seg;
+};
+
+inline FaceShape face_shape(int nn, int n, int lines, bool hll)
+{
+    constexpr int kCUs = 256, kSimds = 4 * kCUs, kSegMax = 32;
+    const int chunks = (nn + 63) / 64, groups = (lines + 3) / 4;
+    FaceShape s{false, kSegMax};
+    double best = 0.0;
+    for (int t = kSegMax; t >= 1; --t) {
+        const long per_simd = ((long)chunks * groups * 4 * ((n + t - 1) / t) + kSimds - 1) / kSimds;
+        const double cost = (hll ? 1.47 : 1.0) * (1.28 * (double)(per_simd / 2) + (double)(per_simd % 2)) * (t + 4);
+        if (t == kSegMax || cost < best) { best = cost; s.seg = t; }
+    }
+    for (int faces = kTileFaces; faces >= kTileWaves; faces -= kTileWaves) {
+        const int tiles = (n + faces - 4) / (faces - 3);
+        const long blocks = (long)chunks * lines * tiles;
+        const double rounds = 0.5 * ((double)blocks / kCUs + (double)((blocks + kCUs - 1) / kCUs));
+        const double cost = (hll ? 1.2 : 1.0) * (1.0 + (faces > kTileWaves ? 3.7 : 2.2) * rounds);
+        if (cost < best) { best = cost; s = FaceShape{true, (n + tiles - 1) / tiles}; }
+    }
+    return s;
 }
 
 }  // namespace m1
