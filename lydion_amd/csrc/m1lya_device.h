@@ -221,8 +221,9 @@ struct Recon {
 // ReconstructInterface: src/AdvectJandH.jl:359-473.
 // iv = {ΔL, ΔR, 1/(x_i-x_{i-1}), 1/(x_{i+1}-x_i), 1/(x_{i+2}-x_{i+1})}
 // With f > 1 the limited direction (f_r, f_Z)/f is the direction itself, so that one reciprocal
-// of |f| serves the limiter and the direction.  A vanishing flux or a depth beyond 2^400 in any
-// lane sends the wavefront to the divisions and roots of any range.
+// of |f| serves the limiter and the direction.  A vanishing flux, a flux or a J near the top of the
+// range or beyond it, or a depth beyond 2^400 in any lane sends the wavefront to the divisions and
+// roots of any range.
 __device__ __forceinline__ Recon reconstruct(const Stencil& s, const double* iv, double aF_i, double aF_ip1)
 {
     const double dL = iv[0], dR = iv[1], inv_i_im1 = iv[2], inv_ip1_i = iv[3], inv_ip2_ip1 = iv[4];
@@ -231,7 +232,8 @@ __device__ __forceinline__ Recon reconstruct(const Stencil& s, const double* iv,
     const double fr_i = s.fr[0], fr_ip1 = s.fr[1], fr_ip2 = s.fr[2], fr_im1 = s.fr[3];
     const double fz_i = s.fz[0], fz_ip1 = s.fz[1], fz_ip2 = s.fz[2], fz_im1 = s.fz[3];
 
-    double dJc = (s.J[1] - s.J[0]) * inv_ip1_i;
+    const double dJ = s.J[1] - s.J[0];
+    double dJc = dJ * inv_ip1_i;
     double dJL = minmod((s.J[0] - s.J[3]) * inv_i_im1, dJc);
     double dJR = minmod((s.J[2] - s.J[1]) * inv_ip2_ip1, dJc);
     double dfrc = (fr_ip1 - fr_i) * inv_ip1_i;
@@ -241,7 +243,8 @@ __device__ __forceinline__ Recon reconstruct(const Stencil& s, const double* iv,
     double dfzL = minmod((fz_i - fz_im1) * inv_i_im1, dfzc);
     double dfzR = minmod((fz_ip2 - fz_ip1) * inv_ip2_ip1, dfzc);
 
-    // a NaN J leaves the flux ratios NaN, and with them every flux
+    // a NaN J leaves the flux ratios NaN, and with them every flux; one that an infinite J brings
+    // about here is kept below
     double J_L = dmax_num(s.J[0] + dJL * dL, kJeps);
     double J_R = dmax_num(s.J[1] - dJR * dR, kJeps);
     double fr_L = fr_i + dfrL * dL;
@@ -251,7 +254,8 @@ __device__ __forceinline__ Recon reconstruct(const Stencil& s, const double* iv,
 
     const double f2_L = fr_L * fr_L + fz_L * fz_L, f2_R = fr_R * fr_R + fz_R * fz_R;
     double f_L, f_R, inv_L, inv_R;
-    o.plain = !__any(!(f2_L >= 0x1p-700) || !(f2_R >= 0x1p-700) || !(o.tau <= 0x1p400));
+    o.plain = !__any(!(f2_L >= 0x1p-700) || !(f2_R >= 0x1p-700) || !(f2_L + f2_R + fabs(dJ) < 0x1p900) ||
+                     !(o.tau <= 0x1p400));
     if (__builtin_expect(o.plain, 1)) {
         f_L = root(f2_L);
         f_R = root(f2_R);
@@ -262,6 +266,8 @@ __device__ __forceinline__ Recon reconstruct(const Stencil& s, const double* iv,
         f_R = sqrt(f2_R);
         inv_L = f_L > 0.0 ? 1.0 / f_L : 0.0;
         inv_R = f_R > 0.0 ? 1.0 / f_R : 0.0;
+        J_L = dmax(s.J[0] + dJL * dL, kJeps);
+        J_R = dmax(s.J[1] - dJR * dR, kJeps);
     }
     o.nr_L = fr_L * inv_L; o.nz_L = fz_L * inv_L;
     o.nr_R = fr_R * inv_R; o.nz_R = fz_R * inv_R;
@@ -379,7 +385,7 @@ __device__ __forceinline__ FaceResult interface_flux(int dir, int hll, const Ste
     }
     FaceResult r;
     r.F = F;
-    if (u_over_c != 0.0) {   // the face velocity is one value for all bins: a uniform branch
+    if (u_over_c != 0.0 || !q.plain) {   // uniform: the face velocity is one value for all bins
         // GetAdvectionFlux: src/AdvectJandH.jl:276-282
         bool up = (u_over_c < 0.0);
         r.F.J = F.J + u_over_c * (up ? q.J_R : q.J_L);
