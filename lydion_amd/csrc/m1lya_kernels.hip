@@ -594,21 +594,25 @@ __device__ __forceinline__ void one_minus_phi(double P, double r, double& o, dou
     chi = small ? (sgn < 0 ? 1.0 : -1.0) - 0.5 * P : quot(1.0 - e, P, r);
 }
 
+// The high word of |x|: 0x07b00000 at 2^-900, 0x78300000 at 2^900, more for infinities and NaN.
+__device__ __forceinline__ unsigned magnitude(double x) { return (unsigned)__double2hiint(x) & 0x7fffffffu; }
+
 // AbsorptionUpdateJorH (src/ConstantsAndFunctions.jl:451-462) for J and the two components of H,
 // which share their divisor.
 __device__ __forceinline__ void absorb(double aJ, double dJdt, double aH, double ct, double dt, double& J, double& Hr,
                                        double& Hz)
 {
-    const double den = 1.0 + aH * ct * dt, rden = rcp_nr(den);
-    double jn = quot(J + dJdt * dt, 1.0 + aJ * ct * dt);
+    const double num = J + dJdt * dt, denJ = 1.0 + aJ * ct * dt, den = 1.0 + aH * ct * dt, rden = rcp_nr(den);
+    double jn = quot(num, denJ);
     double hrn = quot(Hr + 0.0 * dt, den, rden);
     double hzn = quot(Hz + 0.0 * dt, den, rden);
-    // numerators whose residual could underflow, and divisors out of range
-    if (__builtin_expect(!(fabs(Hr) > 0x1p-900) || !(fabs(Hz) > 0x1p-900) || !(fabs(den) < 0x1p500) ||
-                             !(fabs(aJ) * ct * dt < 0x1p500), 0)) {
+    // numerators whose residual could underflow or that are not finite, and divisors out of range
+    const unsigned mj = magnitude(num), mr = magnitude(Hr), mz = magnitude(Hz);
+    if (__builtin_expect(min(min(mj, mr), mz) < 0x07b00000u || max(max(mj, mr), mz) >= 0x78300000u ||
+                             !(fabs(den) + fabs(denJ) < 0x1p500), 0)) {
+        jn = num / denJ;
         hrn = (Hr + 0.0 * dt) / den;
         hzn = (Hz + 0.0 * dt) / den;
-        jn = (J + dJdt * dt) / (1.0 + aJ * ct * dt);
     }
     J = jn; Hr = hrn; Hz = hzn;
 }

@@ -62,3 +62,11 @@ def test_advection(lut, plants, hll):
     o.advect_lya(cloud.c_tilde * cloud.dt, bc_z_bot=cloud.bc_z_bot)
     M.advect_lya(cloud.c_tilde * cloud.dt, ctx, bc_z_bot=cloud.bc_z_bot)
     _same(ctx, o, STATE)
+
+
+@pytest.mark.parametrize("plants", PLANTS.values(), ids=PLANTS.keys())
+def test_emission_and_absorption(lut, plants):
+    cloud, ctx, o = _planted(lut, plants, 0.0, False)
+    o.emission_absorption(cloud.c_tilde, cloud.dt)
+    M.lya_emission_absorption_update(ctx, cloud.c_tilde, cloud.dt)
+    _same(ctx, o, STATE)
