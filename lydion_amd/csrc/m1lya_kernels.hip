@@ -454,8 +454,8 @@ __device__ __forceinline__ int gtsv_general(int n, double* dl, double* d, double
 // The solve is one serial chain per column, and one wavefront's worth of instructions whatever the
 // number of columns it solves: dependent FP64 operations issue back to back on CDNA4 (5 cycles,
 // 16 for the reciprocal estimate), so its time is the count of a row's instructions, forward and
-// back.  For tame systems (every sub-diagonal entry at least kTameMin and no entry above kTameMax
-// in magnitude, which row formation tests) a pivot, interchanged or not, is no smaller than the
+// back.  For tame systems (every sub-diagonal entry at least kTameMin and no entry or right-hand side
+// above kTameMax in magnitude, which row formation tests) a pivot, interchanged or not, is no smaller than the
 // entry below it, so that every division is one of quot's: reciprocal refinement and residual
 // correction, the same quotient.  The pivots' reciprocals stay in rp for the back substitution,
 // where a row is then four operations for its numerator and three for the quotient instead of a
@@ -808,10 +808,12 @@ __global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
                     if (STOREF) { a.Fkp[base + k] = Fkp; a.Fk[base + k] = Fk; a.Fkm[base + k] = Fkm; }
                     if (!SOLVE) return;
                     sD[(size_t)lc * S + row] = -(Fk + dw);
-                    sB[(size_t)lc * S + row] = -dw * Jo[w][q];
+                    const double rhs = -dw * Jo[w][q];
+                    sB[(size_t)lc * S + row] = rhs;
                     if (row >= 1) sDL[(size_t)lc * S + row - 1] = Fkm;
                     if (row <= n - 2) sDU[(size_t)lc * S + row] = Fkp;
-                    wild |= (row >= 1 && !(fabs(Fkm) >= kTameMin)) || !(fabs(Fkp) + fabs(Fk + dw) + fabs(Fkm) < kTameMax);
+                    wild |= (row >= 1 && !(fabs(Fkm) >= kTameMin)) ||
+                            !(fabs(Fkp) + fabs(Fk + dw) + fabs(Fkm) + fabs(rhs) < kTameMax);
                 };
                 if (FREQ) {
                     const double dnuD = a.dnuD ? a.dnuD[c] : 0.0;

@@ -70,3 +70,15 @@ def test_emission_and_absorption(lut, plants):
     o.emission_absorption(cloud.c_tilde, cloud.dt)
     M.lya_emission_absorption_update(ctx, cloud.c_tilde, cloud.dt)
     _same(ctx, o, STATE)
+
+
+FINITE_H = {k: v for k, v in PLANTS.items() if all(f == "J" or np.isfinite(x) for f, x in v)}
+
+
+@pytest.mark.parametrize("umax", [0.0, 150.0])
+@pytest.mark.parametrize("plants", FINITE_H.values(), ids=FINITE_H.keys())
+def test_frequency_update(lut, plants, umax):
+    cloud, ctx, o = _planted(lut, plants, umax, False)
+    o.frequency_update_all_cells(cloud.c_tilde * cloud.dt, update_ff=True)
+    M.frequency_update_j_lya_all_cells(cloud.c_tilde * cloud.dt, ctx)
+    _same(ctx, o, STATE)
