@@ -760,6 +760,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
             if (c >= ncells) continue;
             const size_t base = (size_t)c * nn;
             double Jcur[KPL], hv[KPL];
+            double sum = 0.0;   // not finite if an H (without emission, also a J) of the cell is not
 #pragma unroll
             for (int q = 0; q < KPL; ++q) { Jo[w][q] = 1.0; Hr[w][q] = 0.5; Hz[w][q] = 0.5; hv[q] = 1.0; }   // bins past N_ν
             load_bins<KPL>((FUSED ? a.J : a.J_old) + base, k0, nn, Jo[w]);
@@ -784,6 +785,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
                 }
                 sr = wave_sum_dpp(sr);
                 sz = wave_sum_dpp(sz);
+                sum = sr + sz;
                 if (!FUSED) {
                     if (lane == 0) {
                         a.drhou_r[c] += fpc_ict * sr;
@@ -797,6 +799,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
 #pragma unroll
                 for (int q = 0; q < KPL; ++q) Jcur[q] = 0.0;
                 load_bins<KPL>(a.J + base, k0, nn, Jcur);
+#pragma unroll
+                for (int q = 0; q < KPL; ++q) sum += fabs(Hr[w][q]) + fabs(Hz[w][q]) + fabs(Jcur[q]);
             }
             if (FREQ || SOLVE) {
                 // rows of FrequencyUpdateJLyα! (src/UpdateLyaJandH.jl:200-215) in gtsv form:
@@ -821,10 +825,11 @@ __global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
                     const double RECOIL_0 = kHoverKB / a.T[c];
                     const double durdr = a.dur_dr[c], durdz = a.dur_dz[c];
                     const double duzdr = a.duz_dr[c], duzdz = a.duz_dz[c], urr = a.ur_over_r[c];
-                    // With no velocity gradient D:∇u is +0 whatever D is (D finite; its rr, zz and
+                    // With no velocity gradient D:∇u is +0 whatever D is (D finite, as with H and J; its rr, zz and
                     // ϕϕ entries are >= 0): the cell's bins skip the closure, and a bin's exponents
                     // are the same in the three rows it enters
-                    const bool still = durdr == 0.0 && durdz == 0.0 && duzdr == 0.0 && duzdz == 0.0 && urr == 0.0;
+                    const bool still = durdr == 0.0 && durdz == 0.0 && duzdr == 0.0 && duzdz == 0.0 && urr == 0.0 &&
+                                       !__any(!__builtin_isfinite(sum));
                     auto vel = [&](double J, double hr, double hz) {
                         if (still) return 0.0;
                         return D_colon_grad_u(D_edd(hr, hz, J), durdr, durdz, duzdr, duzdz, urr) * kInvC;
@@ -1138,8 +1143,9 @@ __global__ __launch_bounds__(256) void k_bins(ColumnArgs a)
             if (k < 1 || k > nn - 2) continue;
             const size_t idx = base + k;
             double VEL = 0.0;
-            if (!still)
-                VEL = D_colon_grad_u(D_edd(a.Hr[idx], a.Hz[idx], a.J[idx]), durdr, durdz, duzdr, duzdz, urr) * kInvC;
+            const double hr = a.Hr[idx], hz = a.Hz[idx], J = a.J[idx];
+            if (!still || !__builtin_isfinite(fabs(hr) + fabs(hz) + fabs(J)))
+                VEL = D_colon_grad_u(D_edd(hr, hz, J), durdr, durdz, duzdr, duzdz, urr) * kInvC;
             freq_row_general(a, idx, k, VEL, PREFACT, RECOIL_0, a.Fkp[idx], a.Fk[idx], a.Fkm[idx]);
         }
     }

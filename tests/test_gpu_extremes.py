@@ -36,8 +36,8 @@ def lut():
     return L.VoigtLUT()
 
 
-def _planted(lut, plants, umax, hll):
-    cloud = randomize(small_cloud(n_r=14, n_z=11, n_nu=66, tau0=1e7, umax=umax, lut=lut), seed=31)
+def _planted(lut, plants, umax, hll, n_nu=66):
+    cloud = randomize(small_cloud(n_r=14, n_z=11, n_nu=n_nu, tau0=1e7, umax=umax, lut=lut), seed=31)
     cloud.lya.hll = hll
     for j, i in ((0, 0), (5, 6), (10, 13)):
         for k, v in plants:
@@ -72,13 +72,14 @@ def test_emission_and_absorption(lut, plants):
     _same(ctx, o, STATE)
 
 
-FINITE_H = {k: v for k, v in PLANTS.items() if all(f == "J" or np.isfinite(x) for f, x in v)}
-
-
+@pytest.mark.parametrize("n_nu", [66, 260])
 @pytest.mark.parametrize("umax", [0.0, 150.0])
-@pytest.mark.parametrize("plants", FINITE_H.values(), ids=FINITE_H.keys())
-def test_frequency_update(lut, plants, umax):
-    cloud, ctx, o = _planted(lut, plants, umax, False)
+@pytest.mark.parametrize("plants", PLANTS.values(), ids=PLANTS.keys())
+def test_frequency_factors_and_update(lut, plants, umax, n_nu):
+    cloud, ctx, o = _planted(lut, plants, umax, False, n_nu)
+    o.update_freq_factors()
+    M.update_freq_factors(ctx)
+    _same(ctx, o, ("Fkp", "Fk", "Fkm"))
     o.frequency_update_all_cells(cloud.c_tilde * cloud.dt, update_ff=True)
     M.frequency_update_j_lya_all_cells(cloud.c_tilde * cloud.dt, ctx)
     _same(ctx, o, STATE)
