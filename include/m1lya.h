@@ -457,7 +457,9 @@ int m1lya_reset_kernel_stats(m1lya_ctx *ctx);
 
 /* Runs n IEEE operations on the device for the bit-exactness self-test:
  * op 0: a/b, 1: sqrt(a), 2: the library's exp(a), 3: a plain copy out = a
- * (one kernel reading and writing n doubles; calibrates HBM byte counters). */
+ * (one kernel reading and writing n doubles; calibrates HBM byte counters), and the short forms
+ * that most of the FP64 step uses, 4: a/b, 5: 1/a, 6: sqrt(a), 7: exp(a), each for operands
+ * of its own range. */
 int m1lya_selftest_math(int op, const double *a, const double *b, double *out, size_t n);
 
 #ifdef __cplusplus

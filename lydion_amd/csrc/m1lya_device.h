@@ -46,9 +46,11 @@ __device__ __forceinline__ double dclamp(double x, double lo, double hi)
 // of the exponent range the scaling is by 1 and the fix-up changes nothing.  What remains is the
 // hardware estimate, two Newton steps (a reciprocal r within an ulp) and Markstein's correction
 // q = RN(n r), RN(q + (n - q d) r), whose residual an FMA forms exactly: the IEEE quotient, in
-// 5 instructions per divisor and 3 per numerator.  Operands: 2^-500 <= |d| <= 2^500, and n zero
-// or 2^-500 <= |n| <= 2^500; infinities and NaN give NaN.  (A numerator below 2^-969 may lose its
-// last bit, since the residual then underflows.)
+// 5 instructions per divisor and 3 per numerator.  Operands: 2^-1000 <= |d| <= 2^1000, and n zero
+// or 2^-960 <= |n| <= 2^1000 with a quotient between 2^-1000 and 2^1000; infinities and NaN give
+// NaN.  (A numerator below 2^-969 may lose its last bit, since the residual then underflows.)  The
+// smallest and largest divisors of the callers are 1e-300, the floor of τ and of S_R - S_L, and
+// 2^800, the blend's at a depth of 2^400.
 __device__ __forceinline__ double rcp_nr(double d)
 {
     double r = __builtin_amdgcn_rcp(d);

@@ -1329,6 +1329,10 @@ __global__ void k_selftest(int op, const double* a, const double* b, double* out
     if (op == 0) out[t] = a[t] / b[t];
     else if (op == 1) out[t] = sqrt(a[t]);
     else if (op == 2) out[t] = exp_det(a[t]);
+    else if (op == 4) out[t] = quot(a[t], b[t]);
+    else if (op == 5) out[t] = recip(a[t]);
+    else if (op == 6) out[t] = root(a[t]);
+    else if (op == 7) out[t] = exp_core(a[t]);
     else out[t] = a[t];
 }
 

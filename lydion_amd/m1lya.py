@@ -277,7 +277,8 @@ def run_until_steady(ctx: M1LyaContext, max_steps: int, tol: float, c_tilde: flo
 
 
 def selftest_math(op: int, a: np.ndarray, b: np.ndarray | None = None) -> np.ndarray:
-    """Runs a/b (op 0), sqrt(a) (op 1) or the library's exp (op 2) on the device."""
+    """Runs a/b (op 0), sqrt(a) (op 1) or the library's exp (op 2) on the device, or the short forms
+    of a/b (4), 1/a (5), sqrt(a) (6) and exp(a) (7)."""
     lib = _lib.load()
     a = _f64(a)
     b = _f64(b) if b is not None else None
