@@ -402,11 +402,17 @@ int  m1lya_batch_scalars(m1lya_batch *b, double *out);
 /* [n_clouds][2] active-bin ranges the next step uses (0-based, inclusive). */
 int  m1lya_batch_active_bins(m1lya_batch *b, int *out);
 /* Tile shape: cells per wavefront segment along r (1..64), wavefronts per block (1..8).
- * The state after a step does not depend on the tile shape. */
+ * The state after a step does not depend on the tile shape.  By default the segments follow
+ * from the batch's sizes, one length for the clouds of N_ν > 32 and one for the others, with 8
+ * wavefronts; the step scalars are then summed in the order of tiles of 16 by 8 whatever the
+ * lengths.  With tiles that the caller sets they are summed in the order of the tiles (their
+ * last bits may differ).  seg_len 0 goes back to the default.  get_tiles reports the lengths in
+ * use; of the default's two the one of the clouds of N_ν > 32, if there are any. */
 int  m1lya_batch_set_tiles(m1lya_batch *b, int seg_len, int waves_per_block);
 int  m1lya_batch_get_tiles(const m1lya_batch *b, int *seg_len, int *waves_per_block);
 /* Times each candidate tile shape over trial_steps steps, in two passes over the
- * candidates, and keeps the fastest; the state is restored afterwards.  Outputs may be NULL. */
+ * candidates, and keeps the fastest; the state is restored afterwards.  The outputs (which may
+ * be NULL) set the same tiles with m1lya_batch_set_tiles. */
 int  m1lya_batch_autotune(m1lya_batch *b, int trial_steps, int *seg_len, int *waves_per_block, double *best_ms);
 /* on != 0: steps replay a captured hipGraph (one per state-buffer parity). */
 int  m1lya_batch_set_graph(m1lya_batch *b, int on);

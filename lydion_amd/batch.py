@@ -180,6 +180,8 @@ class M1LyaBatch:
 
     # ---- tiles, autotuner, graph ----
     def set_tiles(self, seg_len: int, waves_per_block: int) -> None:
+        """Cells per wavefront segment and wavefronts per block; seg_len 0: tiles sized from the batch
+        (the default)."""
         self._check(self.lib.m1lya_batch_set_tiles(self.handle, int(seg_len), int(waves_per_block)))
 
     def tiles(self) -> tuple[int, int]:

@@ -1688,6 +1688,14 @@ int auto_segment(const m1lya_batch* b, bool pair)
     return best_seg;
 }
 
+// Segment lengths that follow from the batch's sizes: of the clouds out of pair mode and in it.
+void sized_segments(const m1lya_batch* b, int (&len)[2])
+{
+    bool any[2] = {false, false};
+    for (const Cloud& cl : b->cl) any[cl.pair != 0] = true;
+    for (int p = 0; p < 2; ++p) len[p] = any[p] ? auto_segment(b, p != 0) : kSegLen;
+}
+
 // Work tables.  Per cloud, row segments of one length, wpb of them (same i range, consecutive
 // rows) per block; blocks never mix clouds.  The blocks of clouds in pair mode come first.  With
 // segments of the caller's choice, or of the default length, a block is a partial row of its cloud;
@@ -1728,11 +1736,9 @@ void build_tiles(m1lya_batch* b)
     const int len_rows[2] = {kSegLen, kSegLen};
     int len[2] = {b->seg_len, b->seg_len};   // clouds out of / in pair mode
     if (b->auto_tiles) {
-        bool any[2] = {false, false};
-        for (const Cloud& cl : b->cl) any[cl.pair != 0] = true;
-        for (int p = 0; p < 2; ++p) len[p] = any[p] ? auto_segment(b, p != 0) : kSegLen;
+        sized_segments(b, len);
         b->wpb = kRowWaves;
-        b->seg_len = len[any[0] ? 0 : 1];
+        b->seg_len = std::any_of(b->cl.begin(), b->cl.end(), [](const Cloud& cl) { return !cl.pair; }) ? len[0] : len[1];
     }
     b->step_rows = !b->auto_tiles || (len[0] == kSegLen && len[1] == kSegLen);
     std::vector<Seg> segs, row_segs;
@@ -2576,10 +2582,10 @@ int m1lya_batch_set_tiles(m1lya_batch* b, int seg_len, int waves_per_block)
 {
     return bguard(b, [&] {
         if (!b) bfail(nullptr, M1LYA_ERR_ARG, "batch is NULL");
-        if (seg_len < 1 || seg_len > 64) bfail(b, M1LYA_ERR_ARG, "seg_len out of range [1, 64]");
+        if (seg_len < 0 || seg_len > 64) bfail(b, M1LYA_ERR_ARG, "seg_len out of range [0, 64]");
         if (waves_per_block < 1 || waves_per_block > kMaxWaves) bfail(b, M1LYA_ERR_ARG, "waves_per_block must be 1..8");
         bchk(b, hipStreamSynchronize(b->stream), "hipStreamSynchronize");
-        b->auto_tiles = false;
+        b->auto_tiles = seg_len == 0;
         b->seg_len = seg_len;
         b->wpb = waves_per_block;
         build_tiles(b);
@@ -2604,8 +2610,7 @@ int m1lya_batch_set_graph(m1lya_batch* b, int on)
     });
 }
 
-// Times every tile shape of the candidate set, and the one that the batch's sizes give, on the
-// live batch and keeps the fastest.  State, active-bin ranges and buffer parity are restored, so the call
+// Times every tile shape of the candidate set on the live batch and keeps the fastest.  State, active-bin ranges and buffer parity are restored, so the call
 // does not advance the simulation (the step scalars are those of the last trial).
 // Everything m1lya_batch_autotune changes, put back on every exit: the trial buffers and
 // events are released, profiling is restored, and unless the sweep finished the tile shape,
@@ -2695,10 +2700,17 @@ int m1lya_batch_autotune(m1lya_batch* b, int trial_steps, int* seg_len, int* wav
         // segment lengths: powers of two (16 gives 4 wavefronts per SIMD, the kernel's
         // occupancy, on 256 rows of 256 cells) and the lengths that give 3 or 6 wavefronts
         // per SIMD on 256-cell rows; 2, 4 or 8 wavefronts per block (taller blocks share
-        // more Z interfaces and halo rows, shorter ones fit more blocks per CU)
-        static const int seg_opts[] = {0, 6, 8, 11, 16, 22, 32, 43, 64};
+        // more Z interfaces and halo rows, shorter ones fit more blocks per CU); and the lengths
+        // that follow from the sizes.  All as a caller would set them, so that the outputs set the
+        // same tiles on another batch; their blocks form their partial rows themselves, which on
+        // small batches is faster than the sized tiles with k_rows (32x32x64 25 us per step, 31).
+        std::vector<int> seg_opts = {6, 8, 11, 16, 22, 32, 43, 64};
+        int len[2];
+        sized_segments(b, len);
+        for (int l : len)
+            if (std::find(seg_opts.begin(), seg_opts.end(), l) == seg_opts.end()) seg_opts.push_back(l);
         static const int wpb_opts[] = {2, 4, 8};
-        int best_s = b->auto_tiles ? 0 : b->seg_len, best_w = b->wpb;
+        int best_s = b->seg_len, best_w = b->wpb;
         double best = 1e300;
         bchk(b, hipEventCreate(&scope.e0), "hipEventCreate");
         bchk(b, hipEventCreate(&scope.e1), "hipEventCreate");
@@ -2707,9 +2719,7 @@ int m1lya_batch_autotune(m1lya_batch* b, int trial_steps, int* seg_len, int* wav
         for (int pass = 0; pass < 2; ++pass)
         for (int s : seg_opts)
             for (int w : wpb_opts) {
-                // segment length 0: the length that follows from the sizes, once
-                if (s == 0 && w != wpb_opts[0]) continue;
-                b->auto_tiles = s == 0;
+                b->auto_tiles = false;
                 b->seg_len = s;
                 b->wpb = w;
                 build_tiles(b);
@@ -2733,7 +2743,7 @@ int m1lya_batch_autotune(m1lya_batch* b, int trial_steps, int* seg_len, int* wav
                     best_w = w;
                 }
             }
-        b->auto_tiles = best_s == 0;
+        b->auto_tiles = false;
         b->seg_len = best_s;
         b->wpb = best_w;
         build_tiles(b);
