@@ -163,14 +163,16 @@ def run_fp64(cloud, steps, warmup):
 def run_fp32(clouds, steps, warmup, autotune):
     """Timed batched FP32 steps of a batch of clouds.  The timed region launches the
     kernels eagerly with HIP events around each k_step launch (the dominant kernel; no
-    host synchronisation).  An untimed pass of up to 20 steps with every launch bracketed
-    gives the small reduction kernels' share, and a last pass replays the captured hipGraph."""
+    host synchronisation); a batch of clouds of N_ν <= 32 and of wider ones is timed without
+    events, since with them each kind has a launch of its own.  An untimed pass of up to 20
+    steps with every launch bracketed gives the other kernels' share, and a last pass replays
+    the captured hipGraph."""
     from lydion_amd.batch import M1LyaBatch
     b = M1LyaBatch(clouds)
     tiles = b.autotune(trial_steps=3) if autotune else (*b.tiles(), None)
     b.run_steps(warmup, history=False)
     b.reset_kernel_stats()
-    b.set_profiling(2)
+    b.set_profiling(0 if len({c.lya.n_nu <= 32 for c in clouds}) > 1 else 2)
     b.synchronize()
     t0 = time.perf_counter()
     b.run_steps(steps, history=False)

@@ -139,7 +139,9 @@ void m1lya_destroy(m1lya_ctx *ctx);
 int  m1lya_last_error(const m1lya_ctx *ctx, char *buf, size_t len);
 int  m1lya_set_geometry(m1lya_ctx *ctx, const m1lya_geometry *geometry);
 int  m1lya_set_freq_grid(m1lya_ctx *ctx, const m1lya_freq_grid *grid);
-/* count must equal the field's element count. */
+/* count must equal the field's element count.  Large downloads into ordinary (pageable) memory,
+ * from 8 MiB on, run on up to 8 host threads with pinned buffers of 2 MiB each, which the
+ * context keeps until it is destroyed; a gradient's outputs come the same way. */
 int  m1lya_upload(m1lya_ctx *ctx, int field, const double *host, size_t count);
 int  m1lya_download(m1lya_ctx *ctx, int field, double *host, size_t count);
 int  m1lya_fill(m1lya_ctx *ctx, int field, double value);
@@ -371,6 +373,7 @@ int  m1lya_batch_set_freq_grid(m1lya_batch *b, int cloud, const m1lya_freq_grid 
 int  m1lya_batch_set_scale(m1lya_batch *b, int cloud, double J0);
 int  m1lya_batch_get_scale(const m1lya_batch *b, int cloud, double *J0);
 int  m1lya_batch_upload(m1lya_batch *b, int cloud, int field, const double *host, size_t count);
+/* Large fields come on several host threads, as with m1lya_download. */
 int  m1lya_batch_download(m1lya_batch *b, int cloud, int field, double *host, size_t count);
 /* c̃, Δt, Z_center and the boundary conditions of one cloud's steps. */
 /* The device-side coefficient refresh of one cloud, as m1lya_set_voigt_lut and
@@ -420,7 +423,8 @@ int  m1lya_batch_synchronize(m1lya_batch *b);
 /* on = 1: every launch of a step is bracketed by timing events (m1lya_batch_kernel_stats);
  * on = 2: only the step kernels k_step and k_step_pair (clouds of N_ν <= 32), the step's
  * dominant work (two events per launch instead of around every launch);
- * 0: none.  Graph replay is suspended while profiling. */
+ * 0: none.  Graph replay is suspended while profiling, and k_step and k_step_pair, which
+ * otherwise may share a launch, have one each: their times are not those of the untimed step. */
 int  m1lya_batch_set_profiling(m1lya_batch *b, int on);
 int  m1lya_batch_kernel_stats_count(m1lya_batch *b);
 int  m1lya_batch_kernel_stats(m1lya_batch *b, int index, char *name, size_t name_len,
