@@ -1119,9 +1119,9 @@ __device__ __forceinline__ void step_block(const Cloud* __restrict__ clouds, con
     }
 }
 
-// The step of the blocks [blk0, blk1) of the batch.  Two cells per wavefront at rest fit in 96 VGPRs,
-// so that five of the wavefronts of blocks of four (or fewer) share a SIMD: 32 clouds of 128x128x32
-// in tiles of 16x4, 523 us, 594 at 97 VGPRs and four.
+// The step of the blocks [blk0, blk1) of the batch.  Two cells per wavefront (no sheared gradients)
+// fit in 96 VGPRs, so that a SIMD holds five wavefronts where blocks have four or fewer: 32 clouds of
+// 128x128x32 in tiles of 16x4, 523 us, 594 at 97 VGPRs and four wavefronts.
 template <bool kShear, int NQ, bool kPair>
 __global__ __launch_bounds__(64 * kMaxWaves, NQ > 2 ? 2 : kPair && !kShear ? 5 : 4) void k_step(const Cloud* __restrict__ clouds, Arrays A,
                                                             const Seg* __restrict__ segs, int blk0, int blk1,

@@ -239,8 +239,9 @@ __device__ __forceinline__ void advect_cell_update(const AdvectArgs& a, int i, i
 // What bounds it: FP64 instruction issue (67 % of its cycles) and the wait for the block's
 // slowest wavefront at each cell's barrier.  256x256x128 cone cloud: 405 -> 345 us and 1.58e8 ->
 // 1.05e8 wave instructions (H/J formed once per cell, divisions and roots without range
-// handling, no closure for cells at rest), -> 325 us with one barrier per cell instead of two
-// and the window loaded a cell ahead.  Blocks of 4 rows: 344 us.
+// handling, no closure for cells at rest), -> 326 us with one barrier per cell instead of two
+// and the window loaded a cell ahead.  Blocks of 4 rows: 344 us.  The window holds H/J, so a cell's
+// own H is read again for its update: 759 MB per launch, 624 with H in the window too.
 // ------------------------------------------------------------------------
 template <int WPB>
 __global__ __launch_bounds__(64 * WPB, 4) void k_advect(AdvectArgs a, int seg_len)
@@ -665,10 +666,11 @@ __device__ __forceinline__ void store_bins(double* __restrict__ p, int k0, int n
 // took 256 and 284 bytes of scratch, and 360 to 512 from five bins on (one wavefront per SIMD).
 // 90x90x194: 140 us, 165 with all terms at once.
 // What bounds it: instruction issue in P1 and P3 (two wavefronts per SIMD, whose loads are not
-// all covered), and P2's one wavefront per block.  256x256x128 cone cloud: 592 -> 397 us (P1 and
-// P3 alone 410 -> 240 us: shared factors, divisions without range handling, one pass of per-cell
-// terms per column group); 77x90x194: 251 -> 179 us; 32x32x64: 33 -> 18 us (columns spread over
-// four times the blocks).  Loads three or four rows ahead in P2 measured no better than two.
+// all covered, and 70 to 115 KB of code for an instruction cache of 64), and P2's one wavefront per
+// block.  256x256x128 cone cloud: 592 -> 380 us (P1 and P3 alone 410 -> 240 us: shared factors,
+// divisions without range handling, one pass of per-cell terms per column group); 77x90x194: 253 ->
+// 149 us; 32x32x64: 33 -> 18 us (columns spread over four times the blocks); 45x61x320: 219 -> 158
+// us.  Loads three or four rows ahead in P2 measured no better than two.
 // LDS per block: 5 arrays x (N_ν-2) rows x W·NW columns (odd row stride, so that the
 // lane-per-column sweep is bank-conflict free).
 // ------------------------------------------------------------------------
@@ -883,6 +885,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
                         const double Bl_n = next_lane(Bl), oRl_n = next_lane(oRl);
 #pragma unroll
                         for (int q = 0; q < KPL; ++q) {
+                            if (kWide) __builtin_amdgcn_sched_barrier(0);   // a row at a time, for the registers
                             double A = A_e, oL = oL_e, B = B_e, oR = oR_e, Bp = Bl_n, oRp = oRl_n;
                             if (q + 1 < KPL) {
                                 right(S0, qR, A, oL, B, oR);
@@ -906,6 +909,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_column(ColumnArgs a)
                         const double S_n = next_lane(S0), qL_n = next_lane(qL);
 #pragma unroll
                         for (int q = 0; q < KPL; ++q) {
+                            if (kWide) __builtin_amdgcn_sched_barrier(0);   // a row at a time, for the registers
                             const int k = min(max(k0 + q, 1), nn - 2);
                             double Sp = S_n, qp = qL_n, qRp = qR;
                             if (q + 1 < KPL) bin(q + 1, Sp, qRp, qp);
@@ -1361,9 +1365,9 @@ void launch_active_final(hipStream_t s, const double* red, int nn, int kcmin, in
 void launch_advect(hipStream_t s, const AdvectArgs& a)
 {
     // Rows of 8 wavefronts marching over segments of up to 16 cells: 1.0625 r faces and 1.125 Z
-    // faces per cell, 32 KB of LDS per block.  The segment is the one of the least estimated time: a
+    // faces per cell, 63 KB of LDS per block.  The segment is the one of the least estimated time: a
     // block takes its cells plus the face before the first one (about 0.6 of a cell), two blocks on a
-    // CU (all that 121 VGPRs allow) take 1.65 times one block's time, and a CU gets its share of the
+    // CU (all that 125 VGPRs and the LDS allow) take 1.65 times one block's time, and a CU gets its share of the
     // blocks.  On the 32x32x64 cloud that is single cells, 13 us against 29 us for the four-cell
     // segments that a fixed lower bound gave; on 77x90x194 eight cells, 133 against 135 us for four;
     // on 128x192x64 four, 80 against 86 us for seven.
